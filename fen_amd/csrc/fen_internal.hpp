@@ -116,9 +116,8 @@ __device__ __forceinline__ void march_images(R *f, const Box &b, int ax, int i, 
 // so the stencil neighbours a workgroup needs are in its own XCD's L2.
 __device__ __forceinline__ int xcd_remap(int b, int nb)
 {
-    if (nb & 7) return b;
-    const int per = nb >> 3;
-    return (b & 7) * per + (b >> 3);
+    const int per = nb >> 3, more = nb & 7, x = b & 7;   // the first `more` XCDs get one workgroup more
+    return x * per + (x < more ? x : more) + (b >> 3);
 }
 
 // Kernels whose launches are timed by the profiler.

@@ -8,6 +8,8 @@
 // the checks compute in FP64 from the stored values and round once to R.
 #pragma once
 
+#include <cmath>
+
 #include "fen_internal.hpp"
 
 namespace fen {
@@ -55,6 +57,34 @@ template <class R> struct MomArgs {
     int rpow2;   // rhof is a power of two
     int nbx, nby, img;
 };
+
+// True when r is a power of two (its reciprocal is then exact).
+template <class T> static bool pow2_value(T r)
+{
+    int e = 0;
+    return r > T(0) && std::frexp(r, &e) == T(0.5);
+}
+
+template <class R> static MomArgs<R> momentum_args(fen_ctx *c, double dt, double A, double B)
+{
+    MomArgs<R> a{};
+    a.u = as<R>(c->d_u[0]); a.v = as<R>(c->d_u[1]); a.w = as<R>(c->d_u[2]); a.p = as<R>(c->d_p);
+    a.us = as<R>(c->d_us[0]); a.vs = as<R>(c->d_us[1]); a.ws = as<R>(c->d_us[2]);
+    a.dvo0 = as<R>(c->d_dvo[0]); a.dvo1 = as<R>(c->d_dvo[1]); a.dvo2 = as<R>(c->d_dvo[2]);
+    a.s0 = as<R>(c->d_S[0]); a.s1 = as<R>(c->d_S[1]); a.s2 = as<R>(c->d_S[2]);
+    a.b = c->box;
+    // coefficients are formed in FP64 and rounded once to R
+    a.id = (R)(1.0 / c->delta);
+    a.id2 = (R)(1.0 / (c->delta * c->delta));
+    a.mu = (R)c->viscosity;
+    a.rhof = (R)(0.5 * (c->density + c->density));
+    a.rpow2 = pow2_value(a.rhof) ? 1 : 0;
+    a.irhof = a.rpow2 ? R(1) / a.rhof : R(0);
+    a.dt = (R)dt; a.A = (R)A; a.B = (R)B;
+    a.g0 = (R)c->g[0]; a.g1 = (R)c->g[1]; a.g2 = (R)c->g[2];
+    a.img = c->img_vel;
+    return a;
+}
 
 // One cell of the momentum update.  U, V, W, P are accessors returning the
 // field value at offset (di, dj, dk) from cell (i, j, k); o0..o2 are the

@@ -21,13 +21,6 @@ namespace fen {
 
 constexpr int kTX = 64, kTY = 4, kThreads = kTX * kTY;
 
-// True when r is a power of two (its reciprocal is then exact).
-template <class T> static bool pow2_value(T r)
-{
-    int e = 0;
-    return r > T(0) && std::frexp(r, &e) == T(0.5);
-}
-
 // ---------------------------------------------------------------------------
 // Ghost fill: scalar%update_ghost_nodes (src/scalar.f90:223-396) evaluated
 // as a pure function of the interior.  The reference fills left, right,
@@ -237,24 +230,17 @@ __global__ __launch_bounds__(kThreads) void momentum_kernel_2d(MomArgs<R> a)
 // sweep of tile height, planes per workgroup, ring unrolling and prefetch
 // depth on MI355X at 256^3.
 // (tile height TY, planes per workgroup KB, ring unrolling UN, prefetch depth
-// PF, minimum waves per SIMD for the register allocation OCC; the fused
-// kernel's tiles are FTX = 128 wide: two waves per row, so every row of a
-// tile plane is a 1 KB (FP64) contiguous run -- 0.811 -> 0.804 ms FP64 and
-// 0.464 -> 0.456 ms FP32 per step against 64 x 8 tiles; 256 x 2 lost 10%.
-// 128-wide momentum and projection tiles gained 0.6% on the per-step path
-// of the Neumann solvers and are not used: MTXW = PTXW = 64)
+// PF, minimum waves per SIMD for the register allocation OCC.  128-wide
+// momentum and projection tiles gained 0.6% on the per-step path of the
+// Neumann solvers and are not used: MTXW = PTXW = 64)
 template <class R> struct Shape;
 template <> struct Shape<double> {
     static constexpr int MTY = 8, MKB = 32, MUN = 1, MPF = 1, MOCC = 1, MTXW = 64;   // momentum
     static constexpr int PTY = 4, PKB = 16, PUN = 1, PPF = 1, POCC = 1, PTXW = 64;   // projection
-    static constexpr int FTY = 4, FKB = 16, FOCC = 1, FTX = 128;          // projection + momentum
-    static constexpr bool FLONG = true;   // march as many planes as keep every CU busy
 };
 template <> struct Shape<float> {
     static constexpr int MTY = 4, MKB = 16, MUN = 2, MPF = 2, MOCC = 1, MTXW = 64;
     static constexpr int PTY = 4, PKB = 16, PUN = 1, PPF = 1, POCC = 4, PTXW = 64;
-    static constexpr int FTY = 4, FKB = 32, FOCC = 1, FTX = 128;
-    static constexpr bool FLONG = false;   // two workgroups per CU: longer marches measured slower
 };
 constexpr int MTX = 64;
 
@@ -271,14 +257,12 @@ static void grid_blocks(const Box &b, int ty, int kb, int *nbx, int *nby, int *n
     }
 }
 
-// Workgroups of the kernels that write one partial each (projection, fused
-// projection + momentum), either element type: the partial buffer's size.
+// Workgroups of the kernels that write one partial each (the projection),
+// either element type: the partial buffer's size.
 long stencil_blocks(const Box &b)
 {
-    const int shapes[4][3] = {{Shape<double>::PTY, Shape<double>::PKB, Shape<double>::PTXW},
-                              {Shape<float>::PTY, Shape<float>::PKB, Shape<float>::PTXW},
-                              {Shape<double>::FTY, Shape<double>::FKB, Shape<double>::FTX},
-                              {Shape<float>::FTY, Shape<float>::FKB, Shape<float>::FTX}};
+    const int shapes[2][3] = {{Shape<double>::PTY, Shape<double>::PKB, Shape<double>::PTXW},
+                              {Shape<float>::PTY, Shape<float>::PKB, Shape<float>::PTXW}};
     long most = 0;
     for (const auto &sh : shapes) {
         int nbx, nby, nbz;
@@ -286,27 +270,6 @@ long stencil_blocks(const Box &b)
         most = std::max(most, (long)nbx * nby * nbz);
     }
     return most;
-}
-
-template <class R> MomArgs<R> momentum_args(fen_ctx *c, double dt, double A, double B)
-{
-    MomArgs<R> a{};
-    a.u = as<R>(c->d_u[0]); a.v = as<R>(c->d_u[1]); a.w = as<R>(c->d_u[2]); a.p = as<R>(c->d_p);
-    a.us = as<R>(c->d_us[0]); a.vs = as<R>(c->d_us[1]); a.ws = as<R>(c->d_us[2]);
-    a.dvo0 = as<R>(c->d_dvo[0]); a.dvo1 = as<R>(c->d_dvo[1]); a.dvo2 = as<R>(c->d_dvo[2]);
-    a.s0 = as<R>(c->d_S[0]); a.s1 = as<R>(c->d_S[1]); a.s2 = as<R>(c->d_S[2]);
-    a.b = c->box;
-    // coefficients are formed in FP64 and rounded once to R
-    a.id = (R)(1.0 / c->delta);
-    a.id2 = (R)(1.0 / (c->delta * c->delta));
-    a.mu = (R)c->viscosity;
-    a.rhof = (R)(0.5 * (c->density + c->density));
-    a.rpow2 = pow2_value(a.rhof) ? 1 : 0;
-    a.irhof = a.rpow2 ? R(1) / a.rhof : R(0);
-    a.dt = (R)dt; a.A = (R)A; a.B = (R)B;
-    a.g0 = (R)c->g[0]; a.g1 = (R)c->g[1]; a.g2 = (R)c->g[2];
-    a.img = c->img_vel;
-    return a;
 }
 
 template <class R> void launch_momentum(fen_ctx *c, double dt, double A, double B)
@@ -518,133 +481,6 @@ template <class R> void launch_project(fen_ctx *c, double dt, double *checks_out
     prof_end(c, K_REDUCE, 24.0 * nblk);
 }
 
-// x and y periodic for every field, z faces no-slip walls (the ghost rules
-// the fused kernel evaluates itself): u, v, w Dirichlet, p and phi Neumann.
-bool fused_z_walls(const fen_ctx *c)
-{
-    if (c->box.dim != 3 || c->img_vel != 3 || c->img_p != 3 || c->img_phi != 3) return false;
-    for (int f : {FEN_FRONT, FEN_BACK}) {
-        if (c->bc_type[FEN_U][f] != 1 || c->bc_type[FEN_V][f] != 1 || c->bc_type[FEN_W][f] != 1) return false;
-        if (c->bc_type[FEN_P][f] != 2 || c->bc_type[FEN_PHI][f] != 2) return false;
-    }
-    return true;
-}
-
-// The general-wall form of the fused kernel (3-D FP64, no pending mean
-// shift; the Neumann-direction grids npn and nnn): every axis of every
-// state field is periodic on both faces, or Dirichlet/Neumann on both
-// (the tile formation evaluates the ghost fill's rule chain).  Grids the
-// two dedicated forms take are excluded.
-bool fused_general_walls(const fen_ctx *c)
-{
-    if (c->box.dim != 3 || c->precision != FEN_FP64) return false;
-    if (c->solver != FEN_SOLVER_NPN && c->solver != FEN_SOLVER_NNN) return false;
-    for (int ax = 0; ax < 3; ax++) {
-        const bool per = c->periodic[ax] != 0;
-        for (int f : {FEN_U, FEN_V, FEN_W, FEN_P, FEN_PHI})
-            for (int side = 0; side < 2; side++) {
-                const int t = c->bc_type[f][2 * ax + side];
-                if (per ? t != 0 : (t != 1 && t != 2)) return false;
-            }
-    }
-    return true;
-}
-
-// Step n's projection fused with step n+1's momentum (a grid periodic in
-// every direction, x, y periodic with z walls, or the general walls of
-// fused_general_walls).  Step n's checks are not formed: step n+1 ends
-// pending, so its own checks are what a reader asks for.
-// us_in/p_in: u*, v*, w* and p of step n;
-// us_out/p_out: u*, v*, w* of step n+1 and p after step n (distinct arrays);
-// save (FP64, periodic grid, no source), if given: u, v, w of step n with
-// their periodic images.
-template <class R>
-void launch_project_momentum(fen_ctx *c, double dt_p, double dt_m, double A, double B, void *const *us_in,
-                             const void *p_in, void *const *us_out, void *p_out, void *const *save)
-{
-    const bool periodic = c->img_vel == 7 && c->img_p == 7 && c->img_phi == 7 && !c->shift_active;
-    const bool zwalls = fused_z_walls(c);
-    const bool general = !periodic && !zwalls && std::is_same<R, double>::value && fused_general_walls(c) &&
-                         !c->shift_active;
-    if (c->box.dim != 3 || !(periodic || zwalls || general))
-        throw std::runtime_error("fused projection + momentum needs a periodic grid, x, y periodic with z walls, "
-                                 "or the npn/nnn walls");
-    PMArgs<R> a{};
-    if (general) {
-        a.wall = (c->periodic[0] ? 0 : 1) | (c->periodic[1] ? 0 : 2) | (c->periodic[2] ? 0 : 4);
-        // packed per field: face f's bc type in bits 2f..2f+1, location in bits 12..13
-        const int fid[4] = {FEN_U, FEN_V, FEN_W, FEN_P};
-        const int loc[4] = {1, 2, 3, 0};
-        for (int q = 0; q < 4; q++) {
-            a.gtype[q] = loc[q] << 12;
-            for (int f = 0; f < 6; f++) a.gtype[q] |= c->bc_type[fid[q]][f] << (2 * f);
-        }
-        a.gplane = reinterpret_cast<const R *const *>(c->d_plane_tab);
-        if (!c->d_wallbuf) FEN_HIP_CHECK(hipMalloc(&c->d_wallbuf, 4 * pm_wall_layout(c->box).per_field * sizeof(R)));
-        a.wbuf = as<R>(c->d_wallbuf);
-    }
-    if (zwalls) {
-        a.shift = c->shift_active ? c->d_shift : nullptr;
-        for (int d = 0; d < 3; d++) {
-            a.zlo[d] = as<R>(c->d_plane[FEN_U + d][FEN_FRONT]);
-            a.zhi[d] = as<R>(c->d_plane[FEN_U + d][FEN_BACK]);
-        }
-    }
-    a.m = momentum_args<R>(c, dt_m, A, B);
-    a.m.us = as<R>(us_out[0]); a.m.vs = as<R>(us_out[1]); a.m.ws = as<R>(us_out[2]);
-    a.us = as<R>(us_in[0]); a.vs = as<R>(us_in[1]); a.ws = as<R>(us_in[2]);
-    a.phi = as<R>(c->d_phi);
-    a.p_in = static_cast<const R *>(p_in);
-    a.p_out = as<R>(p_out);
-    a.pid = 1.0 / c->delta;
-    a.pdt = dt_p;
-    a.prhof = 0.5 * (c->density + c->density);
-    a.prpow2 = pow2_value(a.prhof) ? 1 : 0;
-    a.pirhof = a.prpow2 ? 1.0 / a.prhof : 0.0;
-    using SH = Shape<R>;
-    int nbz;
-    grid_blocks(c->box, SH::FTY, SH::FKB, &a.m.nbx, &a.m.nby, &nbz, SH::FTX);
-    // planes per workgroup: FKB, or with FLONG the longest march (each
-    // workgroup loads two planes before its first) that leaves no CU idle
-    a.kb = SH::FKB;
-    if (SH::FLONG) {
-        const long cols = (long)a.m.nbx * a.m.nby;
-        while (2 * a.kb <= c->box.nz && cols * ((c->box.nz + 2 * a.kb - 1) / (2 * a.kb)) >= c->num_cu) a.kb *= 2;
-    }
-    nbz = (c->box.nz + a.kb - 1) / a.kb;
-    const long nblk = (long)a.m.nbx * a.m.nby * nbz;
-    if (general) {
-        // the state at the wall positions, read by the march below
-        const long nw = pm_wall_layout(c->box).per_field;
-        hipLaunchKernelGGL(wall_state_kernel<R>, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, c->stream, a);
-    }
-    prof_begin(c, K_PROJ_MOM);
-    const dim3 grid((unsigned)nblk), block(SH::FTX * SH::FTY);
-#define FEN_PM(SRC, ZW) \
-    hipLaunchKernelGGL((project_momentum_kernel<R, SRC, ZW, SH::FTY, SH::FOCC, SH::FTX>), grid, block, 0, c->stream, a)
-    if (save) {
-        if constexpr (std::is_same<R, double>::value) {
-            if (!periodic || c->has_source) throw std::runtime_error("state saving needs a periodic grid and no source");
-            for (int d = 0; d < 3; d++) a.save[d] = as<R>(save[d]);
-            hipLaunchKernelGGL((project_momentum_kernel<R, 0, 0, SH::FTY, SH::FOCC, SH::FTX, 1>), grid, block, 0,
-                               c->stream, a);
-        } else {
-            throw std::runtime_error("state saving is FP64");
-        }
-    } else if (c->has_source) {
-        if (zwalls) FEN_PM(1, 1);
-        else if (general) FEN_PM(1, 2);
-        else FEN_PM(1, 0);
-    } else {
-        if (zwalls) FEN_PM(0, 1);
-        else if (general) FEN_PM(0, 2);
-        else FEN_PM(0, 0);
-    }
-#undef FEN_PM
-    // reads u*, v*, w*, p, phi, dv_o (+ S); writes p, u*, v*, w*, dv_o
-    prof_end(c, K_PROJ_MOM, (c->has_source ? 18.0 : 15.0) * sizeof(R) * c->n_int);
-}
-
 // ---------------------------------------------------------------------------
 // Stand-alone checks on the resident velocity (used before the first step
 // of a CFL-controlled run): same quantities as above, ghosts already filled.
@@ -716,10 +552,6 @@ template void launch_momentum<double>(fen_ctx *, double, double, double);
 template void launch_momentum<float>(fen_ctx *, double, double, double);
 template void launch_project<double>(fen_ctx *, double, double *, bool);
 template void launch_project<float>(fen_ctx *, double, double *, bool);
-template void launch_project_momentum<double>(fen_ctx *, double, double, double, double, void *const *, const void *,
-                                              void *const *, void *, void *const *);
-template void launch_project_momentum<float>(fen_ctx *, double, double, double, double, void *const *, const void *,
-                                             void *const *, void *, void *const *);
 template void launch_checks<double>(fen_ctx *, const double *const *, double *);
 template void launch_checks<float>(fen_ctx *, const float *const *, double *);
 

@@ -21,8 +21,10 @@
 
 namespace fen {
 
-template <int TY, int TX_ = 64> struct TileShape {
-    static constexpr int TX = TX_, LX = TX + 2, LY = TY + 2, N = LX * LY, NT = TX * TY;
+// NJ: rows (adjacent in j) computed by one thread.
+template <int TY, int TX_ = 64, int NJ = 1> struct TileShape {
+    static_assert(TY % NJ == 0, "whole rows per thread");
+    static constexpr int TX = TX_, LX = TX + 2, LY = TY + 2, N = LX * LY, NT = TX * TY / NJ;
     static constexpr int PER = (N + NT - 1) / NT;
 };
 
@@ -333,6 +335,21 @@ __global__ __launch_bounds__(TX * TY, OCC) void project_march_kernel(ProjArgs<R>
 // planes are indexed at the cell's own, unwrapped (i, j)), w = bc (and the
 // last interior w is overwritten with bc), p = the neighbouring interior
 // value; a pending mean shift of phi is subtracted as the projection does.
+//
+// What bounds it: HBM on large grids (256^3 FP64 2.013 GB in 420 us, 4.8
+// TB/s, 0.84 of what a copy reaches); on small ones the chain of one plane
+// (load, form, barrier, stencil: 2.4 us alone on a CU).  Both ask for more
+// work per plane and barrier, so a thread owns two rows: the tile's halo is
+// 1.27 instead of 1.52 of its cells, the rows share their neighbours, edge
+// products and the face between them, and what plane k needs of k - 1 (the
+// thread's own u, v, w and three fluxes) is carried in registers, so the ring
+// is read at planes k and k + 1 only and one barrier per plane suffices.
+// One row per thread and two barriers took 479 us at 256^3 (FP32 259, now
+// 235), 62 at 128^3 (now 49), 43 at 32^3 (now 7); 64 x 16 tiles with four rows
+// per thread 453; 64 x 8 with two, 470.
+// Loads and stores take a uniform base and a 32-bit offset per element: with
+// 64-bit pointers the compiler hoisted some 70 registers of addresses out of
+// the march (254 registers, one wave per SIMD; now 209).
 template <class R> struct PMArgs {
     MomArgs<R> m;                  // momentum of step n+1 (m.u, m.v, m.w, m.p unused)
     const R *__restrict__ us;      // u*, v*, w* of step n
@@ -450,9 +467,13 @@ __device__ __forceinline__ int pm_src(int g, int n, bool wall)
 // SAVE (periodic grids): also store u, v, w of step n and their periodic
 // images into a.save, for callers that keep every state (the adjoint's
 // recomputed segments).
-template <class R, int SRC, int TY, int ZW, int TX = 64, int SAVE = 0>
+// P2: rhof is a power of two (1/rhof exact), else every division is an IEEE
+// divide.  A template parameter: as a run-time test each of the 39 divisions
+// of the unrolled body kept its branch and its inlined divide, which split the
+// body into some 60 blocks.
+template <class R, int SRC, int TY, int ZW, int TX = 64, int SAVE = 0, int NJ = 2, int P2 = 1>
 struct ProjectMomentumMarch {
-    using S = TileShape<TY, TX>;
+    using S = TileShape<TY, TX, NJ>;
     static constexpr int NT = S::NT, NRAW = 8;
     struct Raw {
         R v[NRAW][S::PER];
@@ -507,6 +528,17 @@ struct ProjectMomentumMarch {
         return t;
     }
 
+    // base[element offset], the offset kept as 32-bit bytes and the base
+    // uniform: one address VGPR per element instead of a 64-bit pair per load.
+    __device__ __forceinline__ static R at_off(const R *base, unsigned bytes)
+    {
+        return *reinterpret_cast<const R *>(reinterpret_cast<const char *>(base) + bytes);
+    }
+    __device__ __forceinline__ static R *to_off(R *base, unsigned bytes)
+    {
+        return reinterpret_cast<R *>(reinterpret_cast<char *>(base) + bytes);
+    }
+
     __device__ __forceinline__ static void fetch(Raw &r, const PMArgs<R> &a, const TileIdx<S> &t,
                                                  const WallIdx &wi, int kk)
     {
@@ -515,7 +547,9 @@ struct ProjectMomentumMarch {
         const int kw = ZW == 1   ? (kk == 0 ? 1 : (kk == b.nz + 1 ? b.nz : kk))
                        : ZW == 2 ? pm_src(kk, b.nz, a.wall & 4)
                                  : (kk == 0 ? b.nz : (kk == b.nz + 1 ? 1 : kk));
-        const long kofs = (long)kw * b.gxy, sj = b.gx, sk = b.gxy;
+        const long kofs = (long)kw * b.gxy;
+        const R *bu = a.us + kofs, *bv = a.vs + kofs, *bw = a.ws + kofs, *bp = a.p_in + kofs;
+        const R *f0 = a.phi + kofs, *fy = f0 + b.gx, *fz = f0 + b.gxy;
         // ZW == 2: elements on a wall position load u, v, w, p of the face
         // buffer instead (a z wall plane: all of them)
         [[maybe_unused]] int pz = -1;
@@ -527,9 +561,10 @@ struct ProjectMomentumMarch {
         }
 #pragma unroll
         for (int q = 0; q < S::PER; q++) {
-            const long o = t.off[q] + kofs;
-            const R *su = a.us + o, *sv = a.vs + o, *sw = a.ws + o, *sp = a.p_in + o;
+            const unsigned o = (unsigned)t.off[q] * (unsigned)sizeof(R);
             if constexpr (ZW == 2) {
+                const R *su = to_off(const_cast<R *>(bu), o), *sv = to_off(const_cast<R *>(bv), o),
+                        *sw = to_off(const_cast<R *>(bw), o), *sp = to_off(const_cast<R *>(bp), o);
                 const bool wl = pz >= 0 || wi.ofs[q] >= 0;
                 const long ow = pz >= 0 ? L.zs + pz * L.zp + wi.zo[q] : wi.ofs[q] + (long)wi.str[q] * kk;
                 if (wl) {
@@ -537,15 +572,20 @@ struct ProjectMomentumMarch {
                     su = w0; sv = w0 + L.per_field; sw = w0 + 2 * L.per_field; sp = w0 + 3 * L.per_field;
                     r.wl |= 1 << q;
                 }
+                r.v[0][q] = *su;
+                r.v[1][q] = *sv;
+                r.v[2][q] = *sw;
+                r.v[3][q] = *sp;
+            } else {
+                r.v[0][q] = at_off(bu, o);
+                r.v[1][q] = at_off(bv, o);
+                r.v[2][q] = at_off(bw, o);
+                r.v[3][q] = at_off(bp, o);
             }
-            r.v[0][q] = *su;
-            r.v[1][q] = *sv;
-            r.v[2][q] = *sw;
-            r.v[3][q] = *sp;
-            r.v[4][q] = a.phi[o];
-            r.v[5][q] = a.phi[o + 1];
-            r.v[6][q] = a.phi[o + sj];
-            r.v[7][q] = a.phi[o + sk];
+            r.v[4][q] = at_off(f0, o);
+            r.v[5][q] = at_off(f0 + 1, o);
+            r.v[6][q] = at_off(fy, o);
+            r.v[7][q] = at_off(fz, o);
         }
     }
 
@@ -555,7 +595,7 @@ struct ProjectMomentumMarch {
     __device__ __forceinline__ static void commit(R *lds, SL slot, const Raw &r, const PMArgs<R> &a,
                                                   const PlaneIdx &pi, int kk, double sh)
     {
-        auto dr = [&](double x) { return over_rho(x, a.prhof, a.pirhof, a.prpow2); };
+        auto dr = [&](double x) { return over_rho(x, a.prhof, a.pirhof, P2); };
         const int nz = a.m.b.nz;
 #pragma unroll
         for (int q = 0; q < S::PER; q++) {
@@ -628,50 +668,165 @@ struct ProjectMomentumMarch {
         return wi;
     }
 
-    template <class SM, class SC, class SN>
-    __device__ __forceinline__ static void plane(const PMArgs<R> &a, R *lds, Raw &r, const TileIdx<S> &t,
-                                                 const PlaneIdx &pi, double sh, int i, int j, int k, int kend,
-                                                 bool active, int c, R (&o)[3], bool xedge, SM sm, SC sc, SN sn,
-                                                 const WallIdx &wi)
+    // What the march carries from plane k - 1 to plane k in registers: the
+    // thread's own u, v, w at k - 1 and the three fluxes through its cells'
+    // k - 1/2 faces (the k + 1/2 fluxes of the plane before, bit for bit).
+    struct Carry {
+        R um[NJ], vm[NJ], wm[NJ];
+        R fu[NJ], fv[NJ], fw[NJ];
+    };
+
+    // The carry into plane k from slots sm (plane k - 1) and sc (plane k).
+    __device__ __forceinline__ static void start(const R *lds, int sm, int sc, int c, Carry &x)
+    {
+        const R c025 = R(0.25);
+        auto at = [&](int f, int slot, int di, int dj) { return lds[(f * 3 + slot) * S::N + c + dj * S::LX + di]; };
+#pragma unroll
+        for (int r = 0; r < NJ; r++) {
+            const R um = at(0, sm, 0, r), vm = at(1, sm, 0, r), wm = at(2, sm, 0, r), wc = at(2, sc, 0, r);
+            x.um[r] = um; x.vm[r] = vm; x.wm[r] = wm;
+            x.fu[r] = ((at(0, sc, 0, r) + um) * (at(2, sm, 1, r) + wm)) * c025;
+            x.fv[r] = ((at(1, sc, 0, r) + vm) * (at(2, sm, 0, r + 1) + wm)) * c025;
+            x.fw[r] = ((wm + wc) * (wm + wc)) * c025;
+        }
+    }
+
+    // march_images() from a uniform base: v to every periodic image (axes
+    // `ax`) of cell (i, j, k), whose row starts at `row` (uniform) and whose
+    // in-plane byte offset is gb; xb is the offset of its x image.  Only
+    // uniform values are hoisted out of the march (64-bit image addresses
+    // per lane would be, and would live through it).
+    __device__ __forceinline__ static void images(R *row, const Box &b, int ax, int j, int k, unsigned gb, unsigned xb,
+                                                  bool xi, R v)
+    {
+        if ((ax & 1) && xi) *to_off(row, xb) = v;
+        const bool yj = (ax & 2) && (j == 1 || j == b.ny);
+        const bool zk = (ax & 4) && (k == 1 || k == b.nz);
+        if (yj || zk) {
+            const long dy = (j == 1 ? b.ny : -b.ny) * b.gx, dz = (k == 1 ? b.nz : -b.nz) * b.gxy;
+            auto put = [&](R *to) {
+                *to_off(to, gb) = v;
+                if ((ax & 1) && xi) *to_off(to, xb) = v;
+            };
+            if (yj) put(row + dy);
+            if (zk) put(row + dz);
+            if (yj && zk) put(row + dy + dz);
+        }
+    }
+
+    // Momentum of the thread's NJ cells at plane k (slots sc: k, sn: k + 1).
+    // momentum_cell's expressions; each flux two of the cells or two of the
+    // equations share (u v on the z edges: u's y flux and v's x flux; u w; v
+    // w; a face between the thread's rows) is formed once.
+    __device__ __forceinline__ static void momentum(const PMArgs<R> &a, const R *lds, int sc, int sn, int c, int i,
+                                                    int j, int k, bool active, bool xedge, Carry &x,
+                                                    const R (&o)[3][NJ])
     {
         const MomArgs<R> &m = a.m;
-        commit(lds, sn, r, a, pi, k + 1, sh);   // state at plane k+1
-        __syncthreads();
-        if (k + 2 <= kend + 1) {
-            fetch(r, a, t, wi, k + 2);
-        }
-        R on[3] = {R(0), R(0), R(0)};
-        const long q = active ? m.b.q(i, j, k) : 0;
-        const long qs = (long)m.b.nx * m.b.ny;
-        if (active && k + 1 <= kend) {
-            on[0] = load_stream(&m.dvo0[q + qs]);
-            on[1] = load_stream(&m.dvo1[q + qs]);
-            on[2] = load_stream(&m.dvo2[q + qs]);
-        }
-        if (active) {
-            // p of step n; its checks are not formed here: the step ends
-            // pending, and a read of the scalars runs the checks-only pass
-            store_stream(&a.p_out[m.b.g(i, j, k)], lds[(3 * 3 + (int)sc) * S::N + c]);
-            if constexpr (SAVE) {
+        const R id = m.id, id2 = m.id2, c0 = R(0.0), c025 = R(0.25), c2 = R(2.0);
+        const R A = m.A, B = m.B, dt = m.dt;
+        auto at = [&](int f, int slot, int di, int dj) { return lds[(f * 3 + slot) * S::N + c + dj * S::LX + di]; };
+        auto dr = [&](R v) { return over_rho(v, m.rhof, m.irhof, P2); };
+        // in-plane byte offsets of cell (i, j); planes and rows move the uniform base
+        const unsigned gb = (unsigned)((i + (int)m.b.gx * j) * (int)sizeof(R));
+        const unsigned qb = (unsigned)(((i - 1) + m.b.nx * (j - 1)) * (int)sizeof(R));
+        const bool xi = xedge && (i == 1 || i == m.b.nx);
+        const unsigned xb = i == 1 ? gb + (unsigned)(m.b.nx * (int)sizeof(R)) : gb - (unsigned)(m.b.nx * (int)sizeof(R));
+        const long gk = (long)k * m.b.gxy, qk = (long)(k - 1) * m.b.nx * m.b.ny;
+        R U[NJ + 2], V[NJ + 2], W[NJ + 2], V1[NJ + 1], Ul[NJ + 1], P[NJ + 1];   // rows -1 .. NJ at [row + 1]
 #pragma unroll
-                for (int f = 0; f < 3; f++) {
-                    const R st = lds[(f * 3 + (int)sc) * S::N + c];
-                    a.save[f][m.b.g(i, j, k)] = st;
-                    march_images(a.save[f], m.b, 7, i, j, k, st, xedge);
+        for (int r = -1; r <= NJ; r++) {
+            U[r + 1] = at(0, sc, 0, r);
+            V[r + 1] = at(1, sc, 0, r);
+            W[r + 1] = at(2, sc, 0, r);
+        }
+#pragma unroll
+        for (int r = 0; r <= NJ; r++) {
+            V1[r] = at(1, sc, 1, r - 1);   // v at i + 1, rows -1 .. NJ - 1
+            Ul[r] = at(0, sc, -1, r);      // u at i - 1, rows 0 .. NJ
+            P[r] = at(3, sc, 0, r);
+        }
+        R exy[NJ + 1], fyy[NJ + 1];   // u v on the edge and v v through the face above rows -1 .. NJ - 1
+#pragma unroll
+        for (int r = 0; r <= NJ; r++) {
+            const R vv = V[r + 1] + V[r];
+            exy[r] = ((U[r + 1] + U[r]) * (V1[r] + V[r])) * c025;
+            fyy[r] = c025 * (vv * vv);
+        }
+        R vwlo = ((W[1] + W[0]) * (V[0] + at(1, sn, 0, -1))) * c025;   // v w on the edge below row 0
+#pragma unroll
+        for (int r = 0; r < NJ; r++) {
+            const R u0 = U[r + 1], v0 = V[r + 1], w0 = W[r + 1];
+            const R ur = at(0, sc, 1, r), ul = Ul[r], un = at(0, sn, 0, r), vn = at(1, sn, 0, r), wn = at(2, sn, 0, r);
+            const R wr = at(2, sc, 1, r), wl = at(2, sc, -1, r);
+            const R uwkp = ((un + u0) * (wr + w0)) * c025;
+            const R vwkp = ((vn + v0) * (W[r + 2] + w0)) * c025;
+            const R wwkp = ((w0 + wn) * (w0 + wn)) * c025;
+            const long g = gk + r * m.b.gx, q = qk + (long)r * m.b.nx;   // + the cell's in-plane offset
+            const bool live = active && j + r <= m.b.ny;
+            auto put = [&](R *us, R *dvo, R val, R dv) {
+                if (live) {
+                    *to_off(us + g, gb) = val;
+                    images(us + g, m.b, m.img, j + r, k, gb, xb, xi, val);
+                    store_stream(to_off(dvo + q, qb), dv);
+                }
+            };
+            // ---- x momentum
+            {
+                const R uuip = c025 * ((ur + u0) * (ur + u0)), uuim = c025 * ((ul + u0) * (ul + u0));
+                R s = (c0 - (uuip - uuim) * id) - (exy[r + 1] - exy[r]) * id;
+                s = s - (uwkp - x.fu[r]) * id;
+                R l = (((ur - c2 * u0) + ul) + ((U[r + 2] - c2 * u0) + U[r])) * id2;
+                l = l + ((un - c2 * u0) + x.um[r]) * id2;
+                s = s + dr(m.mu * l);
+                if constexpr (SRC) s = s + dr(live ? at_off(m.s0 + q, qb) : c0);
+                else s = s + c0;
+                const R gp = (at(3, sc, 1, r) - P[r]) * id;
+                const R rhs = ((-dr(gp) + A * s) + B * o[0][r]) + m.g0;
+                put(m.us, m.dvo0, u0 + dt * rhs, s);
+            }
+            // ---- y momentum
+            {
+                const R vl = at(1, sc, -1, r);
+                const R vuim = ((v0 + vl) * (Ul[r + 1] + ul)) * c025;
+                R s = (c0 - (exy[r + 1] - vuim) * id) - (fyy[r + 1] - fyy[r]) * id;
+                s = s - (vwkp - x.fv[r]) * id;
+                R l = (((V1[r + 1] - c2 * v0) + vl) + ((V[r + 2] - c2 * v0) + V[r])) * id2;
+                l = l + ((vn - c2 * v0) + x.vm[r]) * id2;
+                s = s + dr(m.mu * l);
+                if constexpr (SRC) s = s + dr(live ? at_off(m.s1 + q, qb) : c0);
+                else s = s + c0;
+                const R gp = (P[r + 1] - P[r]) * id;
+                const R rhs = ((-dr(gp) + A * s) + B * o[1][r]) + m.g1;
+                put(m.vs, m.dvo1, v0 + dt * rhs, s);
+            }
+            // ---- z momentum
+            {
+                const R wuim = ((w0 + wl) * (ul + at(0, sn, -1, r))) * c025;
+                R s = ((c0 - (uwkp - wuim) * id) - (vwkp - vwlo) * id) - (wwkp - x.fw[r]) * id;
+                const R l = ((((wr - c2 * w0) + wl) + ((W[r + 2] - c2 * w0) + W[r])) + ((wn - c2 * w0) + x.wm[r])) * id2;
+                s = s + dr(m.mu * l);
+                if constexpr (SRC) s = s + dr(live ? at_off(m.s2 + q, qb) : c0);
+                else s = s + c0;
+                const R gp = (at(3, sn, 0, r) - P[r]) * id;
+                const R rhs = ((-dr(gp) + A * s) + B * o[2][r]) + m.g2;
+                put(m.ws, m.dvo2, w0 + dt * rhs, s);
+            }
+            if (live) store_stream(to_off(a.p_out + g, gb), P[r]);
+            if constexpr (SAVE) {
+                if (live) {
+                    const R st[3] = {u0, v0, w0};
+#pragma unroll
+                    for (int f = 0; f < 3; f++) {
+                        *to_off(a.save[f] + g, gb) = st[f];
+                        images(a.save[f] + g, m.b, 7, j + r, k, gb, xb, xi, st[f]);
+                    }
                 }
             }
-            // momentum of step n+1
-            auto at = [&](int f) {
-                return [=](int di, int dj, int dk) {
-                    const int slotv = dk < 0 ? (int)sm : (dk > 0 ? (int)sn : (int)sc);
-                    return lds[(f * 3 + slotv) * S::N + c + dj * S::LX + di];
-                };
-            };
-            auto img = [&](R *f, R v) { march_images(f, m.b, m.img, i, j, k, v, xedge); };
-            momentum_cell<1, SRC>(m, i, j, k, at(0), at(1), at(2), at(3), o[0], o[1], o[2], img);
+            vwlo = vwkp;
+            x.um[r] = u0; x.vm[r] = v0; x.wm[r] = w0;
+            x.fu[r] = uwkp; x.fv[r] = vwkp; x.fw[r] = wwkp;
         }
-        o[0] = on[0]; o[1] = on[1]; o[2] = on[2];
-        __syncthreads();
     }
 
     __device__ __forceinline__ static void run(const PMArgs<R> &a, R *lds)
@@ -685,38 +840,68 @@ struct ProjectMomentumMarch {
         const bool xedge = bx == 0 || bx == m.nbx - 1;
         const int i0 = bx * S::TX + 1, j0 = by * TY + 1, k0 = bz * a.kb + 1;
         const int kend = min(k0 + a.kb - 1, b.nz);
-        const int i = i0 + tx, j = j0 + ty;
+        const int i = i0 + tx, j = j0 + NJ * ty;
         const bool active = i <= b.nx && j <= b.ny;
-        const int c = (ty + 1) * S::LX + tx + 1;
+        const int c = (NJ * ty + 1) * S::LX + tx + 1;
         const TileIdx<S> t = index(b, i0, j0, a.wall);
         const PlaneIdx pi = plane_index(b, i0, j0);
         const double sh = (ZW == 1 && a.shift) ? a.shift[0] : 0.0;
+        const long qs = (long)b.nx * b.ny;
         Raw r;
         const WallIdx wi = wall_index(a, i0, j0);
         fetch(r, a, t, wi, k0 - 1);
-        commit(lds, IC<0>{}, r, a, pi, k0 - 1, sh);
+        commit(lds, 0, r, a, pi, k0 - 1, sh);
         fetch(r, a, t, wi, k0);
-        commit(lds, IC<1>{}, r, a, pi, k0, sh);
+        commit(lds, 1, r, a, pi, k0, sh);
         fetch(r, a, t, wi, k0 + 1);
-        R o[3] = {R(0), R(0), R(0)};
-        if (active) {
-            const long q = b.q(i, j, k0);
-            o[0] = load_stream(&m.dvo0[q]); o[1] = load_stream(&m.dvo1[q]); o[2] = load_stream(&m.dvo2[q]);
-        }
+        // dv_o of the thread's cells at plane k (a cell past the grid reads the plane's first)
+        unsigned ob[NJ];
+#pragma unroll
+        for (int y = 0; y < NJ; y++)
+            ob[y] = active && j + y <= b.ny ? (unsigned)(((i - 1) + b.nx * (j + y - 1)) * (int)sizeof(R)) : 0u;
+        auto old = [&](R (&o)[3][NJ], int k) {
+            const long qk = (long)(k - 1) * qs;
+#pragma unroll
+            for (int y = 0; y < NJ; y++) {
+                o[0][y] = load_stream(to_off(m.dvo0 + qk, ob[y]));
+                o[1][y] = load_stream(to_off(m.dvo1 + qk, ob[y]));
+                o[2][y] = load_stream(to_off(m.dvo2 + qk, ob[y]));
+            }
+        };
+        R o[3][NJ];
+        old(o, k0);
+        Carry x;
+        __syncthreads();
+        start(lds, 0, 1, c, x);
         int sm = 0, sc = 1, sn = 2;
+        // One barrier per plane: plane k reads slots k and k + 1 (what it needs
+        // of k - 1 is carried), so the next plane's commit, into the slot of
+        // k - 1, may run beside it; the barrier of plane k stands between that
+        // commit and every read of slot k - 1.
         for (int k = k0; k <= kend; k++) {
-            plane(a, lds, r, t, pi, sh, i, j, k, kend, active, c, o, xedge, sm, sc, sn, wi);
+            commit(lds, sn, r, a, pi, k + 1, sh);   // state at plane k+1
+            __syncthreads();
+            if (k < kend) fetch(r, a, t, wi, k + 2);
+            R on[3][NJ] = {};
+            if (k < kend) old(on, k + 1);
+            // p of step n; its checks are not formed here: the step ends
+            // pending, and a read of the scalars runs the checks-only pass
+            momentum(a, lds, sc, sn, c, i, j, k, active, xedge, x, o);
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+#pragma unroll
+                for (int y = 0; y < NJ; y++) o[f][y] = on[f][y];
             const int tmp = sm;
             sm = sc; sc = sn; sn = tmp;
         }
     }
 };
 
-template <class R, int SRC, int ZW, int TY, int OCC = 1, int TX = 64, int SAVE = 0>
-__global__ __launch_bounds__(TX * TY, OCC) void project_momentum_kernel(PMArgs<R> a)
+template <class R, int SRC, int ZW, int TY, int OCC, int TX, int SAVE, int NJ, int P2>
+__global__ __launch_bounds__(TX *TY / NJ, OCC) void project_momentum_kernel(PMArgs<R> a)
 {
-    __shared__ R lds[ring_size<TileShape<TY, TX>, 4>()];
-    ProjectMomentumMarch<R, SRC, TY, ZW, TX, SAVE>::run(a, lds);
+    __shared__ R lds[ring_size<TileShape<TY, TX, NJ>, 4>()];
+    ProjectMomentumMarch<R, SRC, TY, ZW, TX, SAVE, NJ, P2>::run(a, lds);
 }
 
 // The general-wall form's face buffer: u, v, w, p of step n at every wall
