@@ -765,15 +765,14 @@ int fen_create(fen_ctx **out, int dim, int nx, int ny, int nz, double lx, double
         const size_t nspec = (size_t)c->hx * ny * nz;
         c->d_spec = dev_alloc_bytes(nspec * 2 * es);
         const size_t hy = (size_t)ny / 2 + 1;
-        if (c->solver == FEN_SOLVER_PPN) {
-            c->d_c1 = dev_alloc<double>(nspec);
-            if (precision != FEN_FP64) c->d_dd = dev_alloc<double2>(nspec);
-        }
-        if (c->solver == FEN_SOLVER_PN) c->d_c1 = dev_alloc<double>((size_t)c->hx * ny);
-        if (c->solver == FEN_SOLVER_NN || c->solver == FEN_SOLVER_NNN) c->d_c1 = dev_alloc<double>(c->n_int);
-        if (c->solver == FEN_SOLVER_NPN) {
-            c->d_spec2 = dev_alloc<double2>((size_t)nx * nz * hy);
-            c->d_c1 = dev_alloc<double>((size_t)nx * nz * hy);
+        if (c->solver == FEN_SOLVER_NPN) c->d_spec2 = dev_alloc<double2>((size_t)nx * nz * hy);
+        if (c->solver != FEN_SOLVER_PPP && c->solver != FEN_SOLVER_PP) {   // a tridiagonal direction
+            if (fen::thomas_chunks(c)) c->d_c1 = dev_alloc<double>(fen::thomas_chunk_c1_count(c));
+            else if (c->solver == FEN_SOLVER_PPN || c->solver == FEN_SOLVER_PN) c->d_c1 = dev_alloc<double>(nspec);
+            else if (c->solver == FEN_SOLVER_NPN) c->d_c1 = dev_alloc<double>((size_t)nx * nz * hy);
+            else c->d_c1 = dev_alloc<double>(c->n_int);
+            if (c->solver == FEN_SOLVER_PPN && precision != FEN_FP64 && !fen::thomas_chunks(c))
+                c->d_dd = dev_alloc<double2>(nspec);
         }
         // DCT directions use the pi-based wavenumbers (src/poisson.f90:265,794,881,899)
         c->d_mwx = dev_copy(modified_wavenumbers(nx, c->delta, pb[0] ? 2.0 : 1.0));
@@ -793,6 +792,10 @@ int fen_create(fen_ctx **out, int dim, int nx, int ny, int nz, double lx, double
             a[0] = 0.0;
             cc[n - 1] = 0.0;
             c->d_ta = dev_copy(a); c->d_tb = dev_copy(bb); c->d_tc = dev_copy(cc);
+            c->tri_a = 1.0 / d2;
+            c->tri_b0 = bb[0];
+            c->tri_bi = -(2.0 / d2);
+            c->tri_bn = bb[n - 1];
         }
         if (!pb[0]) c->d_mkx = dev_copy(dct_twiddles(nx));
         if (c->solver == FEN_SOLVER_NNN) c->d_mky = dev_copy(dct_twiddles(ny));

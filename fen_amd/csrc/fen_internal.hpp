@@ -205,8 +205,10 @@ struct fen_ctx {
     int hx = 0;                  // nx/2 + 1
     int num_cu = 256;            // compute units of the device (queried at create)
     void *d_spec = nullptr;      // complex R, [kx][k][j] (npn, nnn: real, [k][kx][j])
-    double *d_c1 = nullptr;      // Thomas c1, computed at create (layout of the sweep's columns)
-    double2 *d_dd = nullptr;     // FP64 Thomas right-hand side (ppn, FP32 form), [kx][k][j]
+    double *d_c1 = nullptr;      // Thomas c1, computed at create: chunk starts (3-D), every row (2-D); columns
+                                 // longer than the chunk kernel takes: every row, in the columns' layout
+    double2 *d_dd = nullptr;     // FP64 Thomas right-hand side (ppn, FP32 form, such columns), [kx][k][j]
+    double tri_a = 0, tri_b0 = 0, tri_bi = 0, tri_bn = 0;   // off-diagonal; first, inner and last diagonal
     double2 *d_spec2 = nullptr;  // npn: y half spectrum of the real x-DCT lines, [k][kx][jy]
     double2 *d_mkx = nullptr, *d_mky = nullptr;   // (cos, sin)(pi k/(2n)), k < n: DCTs along x, y
     double *d_mwx = nullptr, *d_mwy = nullptr, *d_mwz = nullptr;
@@ -314,6 +316,11 @@ void launch_dct_y(fen_ctx *c, int inverse, double post);
 void launch_rfft_y(fen_ctx *c, int inverse, double post);
 void launch_thomas_neumann(fen_ctx *c);
 void launch_thomas_c1(fen_ctx *c);
+// Tridiagonal columns in registers (tridiag_kernels.hip).
+bool thomas_chunks(const fen_ctx *c);
+size_t thomas_chunk_c1_count(fen_ctx *c);
+void launch_thomas_chunk_c1(fen_ctx *c);
+void launch_thomas_chunks(fen_ctx *c);
 template <class R> void launch_apply_shift(fen_ctx *c, R *f, size_t n);
 void launch_advection_only(fen_ctx *c, double *rx, double *ry, double *rz);   // FP64 contexts
 

@@ -479,7 +479,9 @@ __global__ __launch_bounds__(kNB) void irfft_rows_kernel(RfftArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Batched Thomas sweeps over strided columns.  Column t = o*ni + q starts at
+// Batched Thomas sweeps over strided columns, one thread per column, for
+// columns longer than thomas_chunk_kernel takes (tridiag_kernels.hip).
+// Column t = o*ni + q starts at
 // o*os + q and has stride s and length n; its diagonal shift is mwx[o]
 // (+ mwy[q] in 3-D).  E is double (real spectra) or double2 (complex).
 // ASSOC2D: the 2-D solvers' form (src/poisson.f90:346-384): divisions, c1
@@ -620,64 +622,6 @@ template <int ASSOC2D> __global__ __launch_bounds__(kNB) void thomas_c1_kernel(T
             c1[k * s] = c1p;
         }
     }
-}
-
-// 2-D solvers (ASSOC2D form, contiguous columns): a few hundred columns of up
-// to 1024 cells, so one thread per column leaves the sweeps bound by memory
-// latency, and the dependent chain of each step bounds any layout.  One wave
-// per column stages the column, its stored c1 (thomas_c1_kernel) and the
-// coefficients in LDS.  With c1 known the pivot (b_k + mx) - a_k c1_{k-1} is
-// off the chain, which keeps one multiply, one subtract and one division per
-// step; the real and imaginary parts of a complex column are independent
-// chains, run by lanes 0 and 1.  Each lane reads its operands one step ahead
-// of the step's store.  Same arithmetic as thomas_general_kernel<E, 1>.
-// Dynamic LDS: E x[n], then double c1[n], A[n], B[n].
-template <class E> __global__ __launch_bounds__(64) void thomas_column_kernel(ThomasGArgs a)
-{
-    extern __shared__ double smem[];
-    constexpr int NC = sizeof(E) / sizeof(double);   // components per element
-    const int n = a.n;
-    const long o = blockIdx.x;
-    const E *xg = static_cast<const E *>(a.x) + o * a.os;
-    const double *c1g = a.c1 + o * a.os;
-    double *x = smem;                 // element k, component l at x[NC * k + l]
-    double *c1 = smem + (long)n * NC;
-    double *A = c1 + n, *B = A + n;
-    for (int k = threadIdx.x; k < n; k += 64) {
-        reinterpret_cast<E *>(x)[k] = xg[k];
-        c1[k] = c1g[k];
-        A[k] = a.ta[k];
-        B[k] = a.tb[k];
-    }
-    __syncthreads();
-    const int l = threadIdx.x;
-    if (l < NC) {
-        const double mx = a.mwx[o];
-        double d = x[l] / (B[0] + mx);
-        x[l] = d;
-        // operands of row k held one row ahead
-        double Ak = A[1], Bk = B[1], cp = c1[0], xk = x[NC + l];
-        for (int k = 1; k < n - 1; k++) {
-            const double An = A[k + 1], Bn = B[k + 1], cn = c1[k], xn = x[NC * (k + 1) + l];
-            d = (xk - d * Ak) / ((Bk + mx) - Ak * cp);
-            x[NC * k + l] = d;
-            Ak = An; Bk = Bn; cp = cn; xk = xn;
-        }
-        const double frac = (Bk + mx) - Ak * cp;   // row n-1 (n >= 2)
-        d = frac != 0.0 ? (xk - d * Ak) / frac : 0.0;
-        x[NC * (n - 1) + l] = d;
-        double xr = d, dk = x[NC * (n - 2) + l], ck = c1[n - 2];
-        for (int k = n - 2; k >= 0; k--) {
-            const int kp = k > 0 ? k - 1 : 0;
-            const double dn = x[NC * kp + l], cnx = c1[kp];
-            xr = dk - xr * ck;
-            x[NC * k + l] = xr;
-            dk = dn; ck = cnx;
-        }
-    }
-    __syncthreads();
-    E *xo = static_cast<E *>(a.x) + o * a.os;
-    for (int k = threadIdx.x; k < n; k += 64) xo[k] = reinterpret_cast<const E *>(x)[k];
 }
 
 }  // namespace
@@ -891,6 +835,10 @@ static ThomasGArgs thomas_layout(fen_ctx *c, bool *complex_out, bool *assoc2d_ou
 // c1 of every column, once per context (after the coefficients are uploaded).
 void launch_thomas_c1(fen_ctx *c)
 {
+    if (thomas_chunks(c)) {
+        launch_thomas_chunk_c1(c);
+        return;
+    }
     bool complex_e = false, assoc2d = false;
     const ThomasGArgs a = thomas_layout(c, &complex_e, &assoc2d);
     const dim3 grid((unsigned)((a.ncol + kNB - 1) / kNB));
@@ -901,19 +849,16 @@ void launch_thomas_c1(fen_ctx *c)
 // Thomas sweeps of the pn, nn, npn and nnn solvers.
 void launch_thomas_neumann(fen_ctx *c)
 {
+    if (c->solver == FEN_SOLVER_PPN) throw std::runtime_error("ppn sweeps use launch_thomas");
+    if (thomas_chunks(c)) {
+        launch_thomas_chunks(c);
+        return;
+    }
     bool complex_e = false, assoc2d = false;
-    if (c->solver == FEN_SOLVER_PPN) throw std::runtime_error("ppn sweeps use thomas_kernel");
     ThomasGArgs a = thomas_layout(c, &complex_e, &assoc2d);
     const dim3 grid((unsigned)((a.ncol + kNB - 1) / kNB));
     prof_begin(c, K_THOMAS);
-    const size_t lds = (size_t)a.n * ((complex_e ? sizeof(double2) : sizeof(double)) + 3 * sizeof(double));
-    if (assoc2d && a.s == 1 && a.os == a.n && lds <= 65536) {
-        // contiguous columns that fit in LDS: one wave each
-        if (complex_e)
-            hipLaunchKernelGGL(thomas_column_kernel<double2>, dim3((unsigned)a.ncol), dim3(64), lds, c->stream, a);
-        else
-            hipLaunchKernelGGL(thomas_column_kernel<double>, dim3((unsigned)a.ncol), dim3(64), lds, c->stream, a);
-    } else if (complex_e) {
+    if (complex_e) {
         // real and imaginary parts on adjacent threads
         const dim3 g2((unsigned)((2 * a.ncol + kNB - 1) / kNB));
         if (assoc2d) hipLaunchKernelGGL((thomas_general_kernel<double, 1, 1>), g2, dim3(kNB), 0, c->stream, a);
@@ -921,9 +866,9 @@ void launch_thomas_neumann(fen_ctx *c)
     }
     else if (assoc2d) hipLaunchKernelGGL((thomas_general_kernel<double, 1>), grid, dim3(kNB), 0, c->stream, a);
     else hipLaunchKernelGGL((thomas_general_kernel<double, 0>), grid, dim3(kNB), 0, c->stream, a);
-    // columns read and written in each sweep, c1 read in the back substitution (LDS kernel: once each)
+    // columns read and written in each sweep, c1 read in the back substitution
     const double eb = complex_e ? 16.0 : 8.0, cells = (double)a.ncol * a.n;
-    prof_end(c, K_THOMAS, (assoc2d && a.s == 1 && lds <= 65536 ? 2.0 * eb : 4.0 * eb + 8.0) * cells);
+    prof_end(c, K_THOMAS, (4.0 * eb + 8.0) * cells);
 }
 
 }  // namespace fen

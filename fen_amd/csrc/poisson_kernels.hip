@@ -346,8 +346,8 @@ __global__ __launch_bounds__(kBlock) void z_solve_pair_kernel(ZArgs<float> a)
 }
 
 // ---------------------------------------------------------------------------
-// K4 (ppn): Thomas sweep along z for every (kx, j) column
-// (src/poisson.f90:1094-1135); one thread per column, adjacent threads own
+// K4 (ppn), columns longer than thomas_chunk_kernel takes: Thomas sweep along
+// z for every (kx, j) column (src/poisson.f90:1094-1135); one thread per column, adjacent threads own
 // adjacent j so every k-row access is coalesced.  The sweep is FP64 for
 // either element type: c1 lives in an FP64 array of the spectrum's layout,
 // computed once per context (launch_thomas_c1: it does not depend on the
@@ -635,6 +635,10 @@ template <class R> void launch_z_solve(fen_ctx *c, double inv_n)
 
 template <class R> void launch_thomas(fen_ctx *c)
 {
+    if (thomas_chunks(c)) {
+        launch_thomas_chunks(c);
+        return;
+    }
     ThomasArgs<R> a{};
     a.spec = as<CplxT<R>>(c->d_spec);
     a.c1 = c->d_c1;

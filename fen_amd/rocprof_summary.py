@@ -33,8 +33,8 @@ _PATTERNS = [
     (r"y_kernel<(?:double|float), \d+, 1, 0>", "y_inv"),
     (r"y_kernel<(?:double|float), \d+, -?1, 1>", "y_solve"),
     (r"z_solve_kernel|z_solve_pair_kernel", "z_solve"),
-    (r"thomas_c1_kernel", "thomas_c1"),
-    (r"thomas_kernel|thomas_general_kernel|thomas_column_kernel", "thomas"),
+    (r"thomas_c1_kernel|thomas_starts_kernel", "thomas_c1"),
+    (r"thomas_kernel|thomas_general_kernel|thomas_column_kernel|thomas_chunk_kernel", "thomas"),
     (r"vof_reconstruct_kernel", "vof_reconstruct"),
     (r"vof_sweep_kernel", "vof_sweep"),
     (r"vof_finish_kernel", "vof_finish"),
