@@ -17,7 +17,6 @@ namespace fen {
 constexpr int kBlock = 256;
 
 template <int N> constexpr int threads_per_line() { return N / 8; }
-template <int N> constexpr int lines_per_block() { return kBlock / (N / 8); }
 
 // ---------------------------------------------------------------------------
 // K2: phi = (div(u*) * rho) / dt on TJ consecutive (j,k) rows, x r2c of row
@@ -210,11 +209,11 @@ template <class C> __device__ __forceinline__ C scale_div(C X, double s1, double
     return C{(R)(x / s2), (R)(y / s2)};
 }
 
-template <class R, int N, int SIGN, int MODE>
-__global__ __launch_bounds__(kBlock) void y_kernel(YArgs<R> a)
+template <class R, int N, int SIGN, int MODE, int NT = kBlock>
+__global__ __launch_bounds__(NT) void y_kernel(YArgs<R> a)
 {
     using C = typename Cplx<R>::type;
-    constexpr int T = threads_per_line<N>(), L = lines_per_block<N>(), LL = lds_line<N>();
+    constexpr int T = threads_per_line<N>(), L = NT / T, LL = lds_line<N>();
     __shared__ C buf[L * LL];
     __shared__ C tw[N];
     load_twiddles<N>(tw, a.tw);   // first read after the first stage's barrier
@@ -510,16 +509,46 @@ template <class R> static double spec_bytes(const fen_ctx *c)
 
 template <class R> using CplxT = typename Cplx<R>::type;
 
-// The x passes (div_r2c, c2r) at N = 512 run 512-thread workgroups: 16 rows
-// per workgroup, so each access to a kx plane of the spectrum covers 256
-// contiguous bytes instead of 128.
-static int x_pass_threads(const fen_ctx *c) { return c->nx == 512 ? 512 : kBlock; }
+// Threads per workgroup of the line transforms (N/8 threads per line, `lines`
+// lines).  x passes at N = 512 run 512 threads: 16 rows per workgroup, so each
+// access to a kx plane of the spectrum covers 256 contiguous bytes instead of
+// 128.  Where 256-thread workgroups would leave most of the chip idle (fewer
+// than one for every other CU) one wave each takes their place: the transform's barriers
+// then cost nothing and the lines spread over four times as many CUs.
+// (32^3: div_r2c 7.5 -> 5.7 us, z 5.2 -> 4.2, y 3.5 -> 3.0; a step 35.1 ->
+// 30.9; 128^2: y solve 6.5 -> 5.5, a step 40.5 -> 38.1.)
+static int line_threads(const fen_ctx *c, int n, long lines, bool x_pass)
+{
+    if (n <= 512 && lines * (n / 8) < (long)kBlock * (c->num_cu / 2)) return 64;
+    return x_pass && n == 512 ? 512 : kBlock;
+}
+static int x_pass_threads(const fen_ctx *c) { return line_threads(c, c->nx, ((long)c->ny * c->nz + 1) / 2, true); }
 
 template <class R, int D3, int N, int DIRECT>
-static void launch_div_r2c_n(const fen_ctx *c, dim3 grid, const DivR2CArgs<R> &a)
+static void launch_div_r2c_n(const fen_ctx *c, dim3 grid, int nt, const DivR2CArgs<R> &a)
 {
-    if constexpr (N == 512) hipLaunchKernelGGL((div_r2c_kernel<R, D3, N, DIRECT, 512>), grid, dim3(512), 0, c->stream, a);
-    else hipLaunchKernelGGL((div_r2c_kernel<R, D3, N, DIRECT>), grid, dim3(kBlock), 0, c->stream, a);
+    if constexpr (N <= 512) {
+        if (nt == 64) {
+            hipLaunchKernelGGL((div_r2c_kernel<R, D3, N, DIRECT, 64>), grid, dim3(64), 0, c->stream, a);
+            return;
+        }
+    }
+    constexpr int NT = N == 512 ? 512 : kBlock;
+    hipLaunchKernelGGL((div_r2c_kernel<R, D3, N, DIRECT, NT>), grid, dim3(NT), 0, c->stream, a);
+}
+
+template <class R, int N, int SIGN, int MODE>
+static void launch_y_n(const fen_ctx *c, const YArgs<R> &a)
+{
+    const int nt = line_threads(c, N, a.nlines, false), L = nt / (N / 8);
+    const dim3 grid((unsigned)((a.nlines + L - 1) / L));
+    if constexpr (N <= 512) {
+        if (nt == 64) {
+            hipLaunchKernelGGL((y_kernel<R, N, SIGN, MODE, 64>), grid, dim3(64), 0, c->stream, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((y_kernel<R, N, SIGN, MODE>), grid, dim3(kBlock), 0, c->stream, a);
 }
 
 // vel == nullptr: direct mode, the RHS is already in `direct_src` (phi array).
@@ -540,14 +569,14 @@ void launch_div_r2c_impl(fen_ctx *c, const R *const *vel, const R *direct_src, l
     a.nrows = (long)c->ny * c->nz;
     a.kxs = (long)c->ny * c->nz;
     a.ny_shift = ilog2(c->ny);
-    const int tj = 2 * (x_pass_threads(c) / (c->nx / 8));
+    const int nt = x_pass_threads(c), tj = 2 * (nt / (c->nx / 8));
     const dim3 grid((unsigned)((a.nrows + tj - 1) / tj));
     const double bytes = (vel ? (c->dim == 3 ? 3.0 : 2.0) : 1.0) * sizeof(R) * c->n_int + spec_bytes<R>(c);
     prof_begin(c, K_DIV_R2C);
 #define L_DIV(NN)                                                                                        \
-    if (a.direct) launch_div_r2c_n<R, 0, NN, 1>(c, grid, a);                                             \
-    else if (c->dim == 3) launch_div_r2c_n<R, 1, NN, 0>(c, grid, a);                                     \
-    else launch_div_r2c_n<R, 0, NN, 0>(c, grid, a);
+    if (a.direct) launch_div_r2c_n<R, 0, NN, 1>(c, grid, nt, a);                                             \
+    else if (c->dim == 3) launch_div_r2c_n<R, 1, NN, 0>(c, grid, nt, a);                                     \
+    else launch_div_r2c_n<R, 0, NN, 0>(c, grid, nt, a);
     FEN_DISPATCH_N(c->nx, L_DIV)
 #undef L_DIV
     prof_end(c, K_DIV_R2C, bytes);
@@ -561,13 +590,11 @@ template <class R> void launch_y_fft(fen_ctx *c, int sign, double post)
     a.nlines = (long)c->hx * c->nz;
     a.post = post;
     a.nz = c->nz;
-    const int L = kBlock / (c->ny / 8);
-    const dim3 grid((unsigned)((a.nlines + L - 1) / L));
     const int kid = sign < 0 ? K_Y_FWD : K_Y_INV;
     prof_begin(c, kid);
 #define L_Y(NN)                                                                                  \
-    if (sign < 0) hipLaunchKernelGGL((y_kernel<R, NN, -1, 0>), grid, dim3(kBlock), 0, c->stream, a); \
-    else hipLaunchKernelGGL((y_kernel<R, NN, 1, 0>), grid, dim3(kBlock), 0, c->stream, a);
+    if (sign < 0) launch_y_n<R, NN, -1, 0>(c, a);                                                \
+    else launch_y_n<R, NN, 1, 0>(c, a);
     FEN_DISPATCH_N(c->ny, L_Y)
 #undef L_Y
     prof_end(c, kid, 2.0 * spec_bytes<R>(c));
@@ -584,13 +611,17 @@ template <class R> void launch_y_solve_2d(fen_ctx *c, double inv_n)
     a.mwx = c->d_mwx;
     a.mwy = c->d_mwy;
     a.nz = c->nz;
-    const int L = kBlock / (c->ny / 8);
-    const dim3 grid((unsigned)((a.nlines + L - 1) / L));
     prof_begin(c, K_Y_SOLVE);
-#define L_YS(NN) hipLaunchKernelGGL((y_kernel<R, NN, -1, 1>), grid, dim3(kBlock), 0, c->stream, a);
+#define L_YS(NN) launch_y_n<R, NN, -1, 1>(c, a);
     FEN_DISPATCH_N(c->ny, L_YS)
 #undef L_YS
     prof_end(c, K_Y_SOLVE, 2.0 * spec_bytes<R>(c));
+}
+
+template <class R, int N> static void launch_z_small(const fen_ctx *c, dim3 grid, const ZArgs<R> &a)
+{
+    if constexpr (N <= 512) hipLaunchKernelGGL((z_solve_kernel<R, N, 64>), grid, dim3(64), 0, c->stream, a);
+    else throw std::logic_error("z lines of at most 512 take one wave");
 }
 
 template <class R> void launch_z_solve(fen_ctx *c, double inv_n)
@@ -609,14 +640,16 @@ template <class R> void launch_z_solve(fen_ctx *c, double inv_n)
     // so every k row of a workgroup is a 128-byte run instead of 64 bytes
     // (measured at 256^3: 61 -> 52 us).  FP64 keeps 256 threads: 512 would
     // need 74 KB of LDS per workgroup and leave 2 per CU (87 -> 100 us).
-    const int nt = (sizeof(R) == sizeof(float) && c->ny % (512 / (c->nz / 8)) == 0) ? 512 : kBlock;
+    // Small grids take one wave per workgroup (line_threads).
+    const bool small = line_threads(c, c->nz, (long)c->ny * c->hx, false) == 64;
+    const int nt = small ? 64 : (sizeof(R) == sizeof(float) && c->ny % (512 / (c->nz / 8)) == 0) ? 512 : kBlock;
     const int L = nt / (c->nz / 8);
     const dim3 grid((unsigned)((c->ny + L - 1) / L), (unsigned)c->hx);
     prof_begin(c, K_Z_SOLVE);
     if constexpr (sizeof(R) == sizeof(float)) {
         // two lines per thread: 2 * (kBlock / (nz / 8)) lines per workgroup
         const int lp = 2 * (kBlock / (c->nz / 8));
-        if (c->ny % lp == 0) {
+        if (!small && c->ny % lp == 0) {
             const dim3 gp((unsigned)(c->ny / lp), (unsigned)c->hx);
 #define L_ZP(NN) hipLaunchKernelGGL((z_solve_pair_kernel<NN>), gp, dim3(kBlock), 0, c->stream, a);
             FEN_DISPATCH_N(c->nz, L_ZP)
@@ -626,7 +659,8 @@ template <class R> void launch_z_solve(fen_ctx *c, double inv_n)
         }
     }
 #define L_Z(NN)                                                                                       \
-    if (nt == 512) hipLaunchKernelGGL((z_solve_kernel<R, NN, 512>), grid, dim3(512), 0, c->stream, a); \
+    if (nt == 64) launch_z_small<R, NN>(c, grid, a);                                                  \
+    else if (nt == 512) hipLaunchKernelGGL((z_solve_kernel<R, NN, 512>), grid, dim3(512), 0, c->stream, a); \
     else hipLaunchKernelGGL((z_solve_kernel<R, NN, kBlock>), grid, dim3(kBlock), 0, c->stream, a);
     FEN_DISPATCH_N(c->nz, L_Z)
 #undef L_Z
@@ -665,8 +699,14 @@ template <class R> void launch_thomas(fen_ctx *c)
 // Workgroups of the x c2r (each writes one block sum when the mean is taken).
 template <class R, int N> static void launch_c2r_n(const fen_ctx *c, long nblk, const C2RArgs<R> &a)
 {
-    if constexpr (N == 512) hipLaunchKernelGGL((c2r_kernel<R, N, 512>), dim3((unsigned)nblk), dim3(512), 0, c->stream, a);
-    else hipLaunchKernelGGL((c2r_kernel<R, N>), dim3((unsigned)nblk), dim3(kBlock), 0, c->stream, a);
+    if constexpr (N <= 512) {
+        if (x_pass_threads(c) == 64) {
+            hipLaunchKernelGGL((c2r_kernel<R, N, 64>), dim3((unsigned)nblk), dim3(64), 0, c->stream, a);
+            return;
+        }
+    }
+    constexpr int NT = N == 512 ? 512 : kBlock;
+    hipLaunchKernelGGL((c2r_kernel<R, N, NT>), dim3((unsigned)nblk), dim3(NT), 0, c->stream, a);
 }
 
 long c2r_blocks(const fen_ctx *c)
