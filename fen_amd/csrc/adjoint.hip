@@ -289,7 +289,7 @@ void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, dou
     launch_y_fft<double>(c, -1, 1.0);
     launch_z_solve<double>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
     launch_y_fft<double>(c, +1, 1.0);
-    launch_c2r<double>(c, r, 0, sx, sy, false, 0);
+    launch_c2r<double>(c, r, 0, sx, sy, false, AxisCopies{});
     AdjProjArgs pa{};
     pa.ub = ub[0]; pa.vb = ub[1]; pa.wb = ub[2];
     pa.psi = r;

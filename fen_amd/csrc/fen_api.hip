@@ -77,18 +77,6 @@ void prof_end(fen_ctx *c, int k, double bytes)
 
 namespace {
 
-const char *kKernelNames[fen::K_COUNT] = {
-    "momentum", "ghost", "div_r2c", "y_fwd", "z_solve", "thomas", "y_inv", "y_solve", "c2r", "project",
-    "checks", "reduce", "project_momentum"};
-
-int fail(fen_ctx *c, int code, const std::string &msg)
-{
-    if (c) c->err = msg;
-    return code;
-}
-
-bool pow2(int n) { return n >= 8 && n <= 1024 && (n & (n - 1)) == 0; }
-
 int field_slot(int field)   // index into bc_type / d_plane
 {
     return field >= FEN_P && field <= FEN_W ? field : -1;
@@ -103,6 +91,41 @@ char field_loc(int field)
     default: return 'c';
     }
 }
+
+}  // namespace
+
+namespace fen {
+template <class R> GhostDesc<R> make_desc(fen_ctx *c, int field, void *arr)
+{
+    GhostDesc<R> d{};
+    d.f = as<R>(arr);
+    const int s = field_slot(field);
+    for (int f = 0; f < 6; f++) {
+        d.type[f] = c->bc_type[s][f];
+        d.plane[f] = as<R>(c->d_plane[s][f]);
+    }
+    d.loc = field_loc(field);
+    d.groups = 7;
+    return d;
+}
+
+template GhostDesc<double> make_desc<double>(fen_ctx *, int, void *);
+template GhostDesc<float> make_desc<float>(fen_ctx *, int, void *);
+}  // namespace fen
+
+namespace {
+
+const char *kKernelNames[fen::K_COUNT] = {
+    "momentum", "ghost", "div_r2c", "y_fwd", "z_solve", "thomas", "y_inv", "y_solve", "c2r", "project",
+    "checks", "reduce", "project_momentum"};
+
+int fail(fen_ctx *c, int code, const std::string &msg)
+{
+    if (c) c->err = msg;
+    return code;
+}
+
+bool pow2(int n) { return n >= 8 && n <= 1024 && (n & (n - 1)) == 0; }
 
 // BC mapping of allocate_navier_stokes_fields (src/navier_stokes.f90:779-1017).
 int map_bc(int field, int face, int pc, bool *ok)
@@ -246,22 +269,24 @@ size_t plane_count(const fen_ctx *c, int face)
     return gx * gy;
 }
 
-template <class R> GhostDesc<R> make_desc(fen_ctx *c, int field, void *arr)
-{
-    GhostDesc<R> d{};
-    d.f = as<R>(arr);
-    const int s = field_slot(field);
-    for (int f = 0; f < 6; f++) {
-        d.type[f] = c->bc_type[s][f];
-        d.plane[f] = as<R>(c->d_plane[s][f]);
-    }
-    d.loc = field_loc(field);
-    d.groups = 7;
-    return d;
-}
+using fen::make_desc;
 
-// Ghost groups left after a producer that wrote the images along `img` axes.
-int remaining_groups(const fen_ctx *c, int img) { return ~img & (c->dim == 3 ? 7 : 3); }
+// Ghost groups left after a producer that wrote the images along `img` axes
+// (the 2-D producers of u*, v*, u, v and p fill all of theirs).
+int remaining_groups(const fen_ctx *c, int img) { return c->dim == 3 ? ~img & 7 : 0; }
+
+// The ghosts of phi as copies of its interior, per axis, when every one is
+// (faces periodic or Neumann, alike on both sides of an axis); else false.
+bool phi_copies(const fen_ctx *c, fen::AxisCopies *out)
+{
+    int *ax[3] = {&out->x, &out->y, &out->z};
+    for (int d = 0; d < c->dim; d++) {
+        const int lo = c->bc_type[FEN_PHI][2 * d], hi = c->bc_type[FEN_PHI][2 * d + 1];
+        if (lo != hi || lo == 1) return false;
+        *ax[d] = lo == 0 ? fen::COPY_PERIODIC : fen::COPY_MIRROR;
+    }
+    return out->x == (c->periodic[0] ? fen::COPY_PERIODIC : fen::COPY_MIRROR);
+}
 
 void refresh_images(fen_ctx *c)
 {
@@ -296,7 +321,7 @@ void free_all(fen_ctx *c)
     for (int d = 0; d < 3; d++) { f(c->d_u[d]); f(c->d_us[d]); f(c->d_dvo[d]); f(c->d_S[d]); }
     f(c->d_p); f(c->d_p2); f(c->d_phi); f(c->d_spec); f(c->d_c1); f(c->d_dd);
     f(c->d_mwx); f(c->d_mwy); f(c->d_mwz); f(c->d_ta); f(c->d_tb); f(c->d_tc);
-    f(c->d_twx); f(c->d_twy); f(c->d_twz); f(c->d_spec2); f(c->d_mkx); f(c->d_mky); f(c->d_part); f(c->d_scal);
+    f(c->d_twx); f(c->d_twy); f(c->d_twz); f(c->d_spec2); f(c->d_mkx); f(c->d_mky); f(c->d_part); f(c->d_chk); f(c->d_scal);
     for (int s = 0; s < 5; s++) for (int p = 0; p < 6; p++) f(c->d_plane[s][p]);
     f(c->d_plane_tab);
     f(c->d_wallbuf);
@@ -388,19 +413,20 @@ void solve_to_x_spectrum(fen_ctx *c, const R *const *vel, const R *direct, long 
 }
 
 // x backward transform of the spectrum into the interior of phi; sums the
-// interior for the mean when `mean`; writes the periodic images in `img`.
-template <class R> void x_backward(fen_ctx *c, R *phi, int gl, long sx, long sy, bool mean, int img,
-                                   double *part = nullptr, size_t n_part = 0, double *shift = nullptr)
+// interior for the mean when `mean`; writes the ghosts `copies` names.
+template <class R> void x_backward(fen_ctx *c, R *phi, int gl, long sx, long sy, bool mean, fen::AxisCopies copies,
+                                   double *part = nullptr, size_t n_part = 0, double *shift = nullptr,
+                                   bool defer = false)
 {
     if constexpr (std::is_same_v<R, double>) {
         if (x_cosine(c)) {
             // nn divides by 2nx after the DCT-III (src/poisson.f90:594)
             fen::launch_dct3_x(c, phi, gl, sx, sy, c->solver == FEN_SOLVER_NN ? 1.0 / (2.0 * (double)c->nx) : 1.0,
-                               img != 0);
+                               copies);
             return;
         }
     }
-    fen::launch_c2r<R>(c, phi, gl, sx, sy, mean, img, part, n_part, shift);
+    fen::launch_c2r<R>(c, phi, gl, sx, sy, mean, copies, part, n_part, shift, defer);
 }
 
 // K2..K6 of a step: the Poisson solve on u*, v*, w* (`us`) up to phi with
@@ -414,29 +440,31 @@ template <class R> void solve_phi(fen_ctx *c, double dt, void *const *us)
     const bool mean = removes_mean(c);
     bool dirichlet = false;
     for (int f = 0; f < 6; f++) dirichlet = dirichlet || c->bc_type[FEN_PHI][f] == 1;
-    // images written by the c2r only when no shift has to be applied first;
-    // the DCT-III writes every ghost when they are all copies, else none
-    const int img_phi = x_cosine(c) ? (fen::dct3_writes_ghosts(c) ? 7 : 0)
-                                    : ((mean && dirichlet) ? 0 : c->img_phi);
-    x_backward<R>(c, as<R>(c->d_phi), 1, c->box.gx, c->box.gxy, mean, img_phi);
+    // the x backward transform writes phi's ghosts when they are all copies
+    // (which commute with the mean's shift); otherwise the ghost kernel does
+    AxisCopies copies;
+    const bool filled = phi_copies(c, &copies);
+    if (!filled) copies = AxisCopies{};
+    x_backward<R>(c, as<R>(c->d_phi), 1, c->box.gx, c->box.gxy, mean, copies, nullptr, 0, nullptr,
+                  c->dim == 2 && !dirichlet);
     c->shift_active = mean;
     if (mean && dirichlet) {   // the shift does not commute with 2*bc - f: apply it first
         launch_apply_shift<R>(c, as<R>(c->d_phi), c->n_ghost);
         c->shift_active = false;
     }
-    if (const int rest = remaining_groups(c, img_phi)) {
+    if (!filled) {
         GhostDesc<R> g = make_desc<R>(c, FEN_PHI, c->d_phi);
-        g.groups = rest;
         launch_ghost_desc<R>(c, &g, 1);
     }
 }
 
 // K7..K8 of a step: projection, pressure update, checks and ghosts of u, p.
-template <class R> void finish_step(fen_ctx *c, double dt)
+// p_old (two-phase): receives p before the update.
+template <class R> void finish_step(fen_ctx *c, double dt, R *p_old = nullptr)
 {
     using namespace fen;
     const bool d3 = c->dim == 3;
-    launch_project<R>(c, dt, c->d_scal);
+    launch_project<R>(c, dt, true, p_old);
     if (const int rest = remaining_groups(c, c->img_vel & c->img_p)) {
         GhostDesc<R> g[4] = {make_desc<R>(c, FEN_U, c->d_u[0]), make_desc<R>(c, FEN_V, c->d_u[1]),
                              d3 ? make_desc<R>(c, FEN_W, c->d_u[2]) : make_desc<R>(c, FEN_P, c->d_p),
@@ -482,16 +510,9 @@ void advance_mf(fen_ctx *c, double dt)
     // :85 and p_hat (:88-92), with ghosts; the constant-CFL form extrapolates with dt_o
     mf_update_fields(c, true, c->constant_cfl ? dt : 0.0);
     mf_momentum(c, dt);            // predicted_velocity_field with MF (:140-213)
-    if (const int rest = remaining_groups(c, c->img_vel)) {
-        GhostDesc<double> g[2] = {make_desc<double>(c, FEN_U, c->d_us[0]), make_desc<double>(c, FEN_V, c->d_us[1])};
-        for (auto &d : g) d.groups = rest;
-        launch_ghost_desc<double>(c, g, 2);
-    }
     solve_phi<double>(c, dt, c->d_us);
     // update_pressure with MF: p_o = p before p = p + phi (:553-559)
-    FEN_HIP_CHECK(hipMemcpyAsync(c->mf->p_o, c->d_p, c->n_ghost * sizeof(double), hipMemcpyDeviceToDevice,
-                                 c->stream));
-    finish_step<double>(c, dt);
+    finish_step<double>(c, dt, c->mf->p_o);
 }
 
 // Whether a step may end with its projection pending, to be fused into the
@@ -561,7 +582,7 @@ void flush_pending(fen_ctx *c)
 void pending_checks(fen_ctx *c)
 {
     if (!c->pending || c->pending_checked) return;
-    with_type(c, [&](auto tag) { fen::launch_project<decltype(tag)>(c, c->pend_dt, c->d_scal, false); });
+    with_type(c, [&](auto tag) { fen::launch_project<decltype(tag)>(c, c->pend_dt, false); });
     c->pending_checked = true;
 }
 }  // namespace
@@ -651,6 +672,8 @@ void advance_graph(fen_ctx *c, double dt)
         (void)hipGraphDestroy(g);
         FEN_HIP_CHECK(e);
         c->graph_dt = dt;
+        c->graph_shift_parts = c->shift_parts;
+        c->graph_chk_blocks = c->chk_blocks;
         c->graph_dt_o = c->dt_o;
         c->graph_version = c->config_version;
     } else {
@@ -660,6 +683,8 @@ void advance_graph(fen_ctx *c, double dt)
         bool dirichlet = false;
         for (int f = 0; f < 6; f++) dirichlet = dirichlet || c->bc_type[FEN_PHI][f] == 1;
         c->shift_active = mean && !dirichlet;
+        c->shift_parts = c->graph_shift_parts;
+        c->chk_blocks = c->graph_chk_blocks;
         c->checks_valid = true;
     }
     FEN_HIP_CHECK(hipGraphLaunch(c->step_graph, c->stream));
@@ -809,9 +834,10 @@ int fen_create(fen_ctx **out, int dim, int nx, int ny, int nz, double lx, double
             fen::launch_thomas_c1(c);
             FEN_HIP_CHECK(hipGetLastError());
         }
-        c->n_part = std::max<size_t>(std::max<size_t>(3 * 1024, (size_t)ny * nz / 2 + 1),
-                                     3 * (size_t)fen::stencil_blocks(c->box));
+        c->n_part = (size_t)ny * nz / 2 + 1;
         c->d_part = dev_alloc<double>(c->n_part);
+        c->n_chk = std::max<size_t>(3 * 1024, 3 * (size_t)fen::stencil_blocks(c->box));
+        c->d_chk = dev_alloc<double>(c->n_chk);
         c->d_scal = dev_alloc<double>(8);
         c->d_shift = c->d_scal + 3;
         FEN_HIP_CHECK(hipHostMalloc((void **)&c->h_scal, 8 * sizeof(double)));
@@ -968,6 +994,7 @@ int fen_get_scalars(fen_ctx *c, double *maxdiv, double *maxcfl, double *dt_o, do
             if (maxcfl) *maxcfl = 0.0;
         } else if (maxdiv || maxcfl) {
             pending_checks(c);
+            fen::reduce_checks(c);
             FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal, c->d_scal, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
             sync(c);
             if (maxdiv) *maxdiv = c->h_scal[0];
@@ -1029,6 +1056,7 @@ int fen_download(fen_ctx *c, int field, double *host, size_t count)
         }
         copy_out(c, host, src, n);
         if (field == FEN_PHI && c->shift_active) {
+            fen::reduce_shift(c);
             FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal + 3, c->d_shift, sizeof(double), hipMemcpyDeviceToHost, c->stream));
             sync(c);
             const double s = c->h_scal[3];
@@ -1122,9 +1150,10 @@ int fen_ns_step(fen_ctx *c, int step, double *dt, double *maxdiv, double *maxcfl
                 with_type(c, [&](auto tag) {
                     using R = decltype(tag);
                     const R *vn[3] = {as<R>(c->d_u[0]), as<R>(c->d_u[1]), as<R>(c->d_u[2])};
-                    fen::launch_checks<R>(c, vn, c->d_scal);
+                    fen::launch_checks<R>(c, vn);
                 });
             }
+            fen::reduce_checks(c);
             FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal, c->d_scal, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
             sync(c);
             c->dt_o = *dt;
@@ -1219,7 +1248,7 @@ int fen_poisson_solve(fen_ctx *c, double *f, int gl)
         with_type(c, [&](auto tag) {
             using R = decltype(tag);
             solve_to_x_spectrum<R>(c, nullptr, as<R>(buf), sx, sy, gl, 1.0, 1.0);
-            x_backward<R>(c, as<R>(buf), gl, sx, sy, mean, 0);
+            x_backward<R>(c, as<R>(buf), gl, sx, sy, mean, fen::AxisCopies{});
         });
         copy_out(c, f, buf, n);
         if (mean) {
@@ -1254,7 +1283,7 @@ int fen_poisson_solve_noalloc(fen_ctx *c, double *f, int gl)
         double *buf = as<double>(c->d_us[0]);   // context memory between steps
         FEN_HIP_CHECK(hipMemcpyAsync(buf, f, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
         solve_to_x_spectrum<double>(c, nullptr, buf, sx, sy, gl, 1.0, 1.0);
-        x_backward<double>(c, buf, gl, sx, sy, mean, 0, part, kNoAllocParts, shift);
+        x_backward<double>(c, buf, gl, sx, sy, mean, fen::AxisCopies{}, part, kNoAllocParts, shift);
         FEN_HIP_CHECK(hipMemcpyAsync(f, buf, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         double s = 0.0;
         if (mean) FEN_HIP_CHECK(hipMemcpyAsync(&s, shift, sizeof(double), hipMemcpyDeviceToHost, c->stream));

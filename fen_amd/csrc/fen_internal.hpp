@@ -111,6 +111,63 @@ __device__ __forceinline__ void march_images(R *f, const Box &b, int ax, int i, 
     }
 }
 
+// Stores v at 2-D interior cell (i, j) of a ghosted field, or the Dirichlet
+// value that the ghost fill overwrites a high normal face with (f(N) = bc),
+// and every ghost that the x -> y fill takes from this cell (the rules of
+// src/scalar.f90:254-388): the producer of a field leaves it filled and no
+// ghost launch follows (each took 4 us, most of a 2-D kernel's time).  The
+// descriptor's members are read at fixed indexes only.
+template <class R>
+__device__ __forceinline__ void put_ghosted(const GhostDesc<R> &d, const Box &b, R *f, int i, int j, R v)
+{
+    const R two = R(2.0);
+    // S1(gi, j) = s: the y rules of column gi
+    auto column = [&](int gi, R s) {
+        const long pi = gi + (long)(b.nx + 2);   // index into a bottom/top plane at k = 1
+        f[b.g(gi, j, 1)] = (j == b.ny && d.type[3] == 1 && d.loc == 'y') ? d.plane[3][pi] : s;
+        if (j == (d.type[2] == 0 ? b.ny : 1)) {
+            R t = s;
+            if (d.type[2] == 1) t = d.loc == 'y' ? d.plane[2][pi] : two * d.plane[2][pi] - s;
+            f[b.g(gi, 0, 1)] = t;
+        }
+        if (j == (d.type[3] == 0 ? 1 : b.ny)) {
+            R t = s;
+            if (d.type[3] == 1) t = d.loc == 'y' ? d.plane[3][pi] : two * d.plane[3][pi] - s;
+            f[b.g(gi, b.ny + 1, 1)] = t;
+        }
+    };
+    const long pj = j + (long)(b.ny + 2);   // index into a left/right plane at k = 1
+    column(i, (i == b.nx && d.type[1] == 1 && d.loc == 'x') ? d.plane[1][pj] : v);
+    if (i == (d.type[0] == 0 ? b.nx : 1)) {
+        R t = v;
+        if (d.type[0] == 1) t = d.loc == 'x' ? d.plane[0][pj] : two * d.plane[0][pj] - v;
+        column(0, t);
+    }
+    if (i == (d.type[1] == 0 ? 1 : b.nx)) {
+        R t = v;
+        if (d.type[1] == 1) t = d.loc == 'x' ? d.plane[1][pj] : two * d.plane[1][pj] - v;
+        column(b.nx + 1, t);
+    }
+}
+
+// How a kernel that writes whole rows of a field fills the ghosts along one
+// axis when they are copies of interior cells: periodic images, the mirror of
+// Neumann faces, or not at all.
+enum { COPY_NONE = 0, COPY_PERIODIC = 1, COPY_MIRROR = 2 };
+
+// The ghosted indices that hold row index J (interior 1..n) of such an axis:
+// J itself, and the ghost rows 0 and n + 1 that copy it.  Returns how many.
+__device__ __forceinline__ int copy_rows(int J, int n, int mode, int (&d)[3])
+{
+    int m = 0;
+    d[m++] = J;
+    if (mode != COPY_NONE) {
+        if (J == (mode == COPY_PERIODIC ? n : 1)) d[m++] = 0;
+        if (J == (mode == COPY_PERIODIC ? 1 : n)) d[m++] = n + 1;
+    }
+    return m;
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X; this
 // renumbering gives every XCD one contiguous range of the grid (a k-slab),
 // so the stencil neighbours a workgroup needs are in its own XCD's L2.
@@ -217,11 +274,15 @@ struct fen_ctx {
     double phi_shift = 0.0;      // mean/N removed lazily (pp, ppn)
     double *d_shift = nullptr;   // device copy of the subtracted mean
     bool shift_active = false;
+    long shift_parts = 0;        // > 0: that many block sums in d_part, not yet reduced to d_shift (reduce_shift)
 
     int img_vel = 0, img_p = 0, img_phi = 0;   // image_axes of (u,v,w), p, phi
 
     // reductions
-    double *d_part = nullptr;    // per-block partials
+    double *d_part = nullptr;    // per-block sums of the mean
+    double *d_chk = nullptr;     // per-block maxima of the checks
+    long chk_blocks = 0;         // > 0: that many entries of d_chk not yet reduced to d_scal (reduce_checks)
+    size_t n_chk = 0;
     double *d_noalloc = nullptr; // device address of the allocation-free entry point's scratch (this device)
     size_t n_part = 0;
     double *d_scal = nullptr;    // [0] maxdiv [1] max|u|+|v|+|w| [2] nonfinite flag [3] mean shift
@@ -253,6 +314,7 @@ struct fen_ctx {
     bool fused_run = true;                  // FEN_FUSED_RUN=0 at create turns fen_ns_run's fusion off
     hipGraphExec_t step_graph = nullptr;
     double graph_dt = 0.0, graph_dt_o = 0.0;
+    long graph_shift_parts = 0, graph_chk_blocks = 0;   // shift_parts and chk_blocks a replay leaves
     int graph_version = -1;
     int config_version = 0;
 
@@ -286,11 +348,26 @@ template <class R> void launch_thomas(fen_ctx *c);
 long c2r_blocks(const fen_ctx *c);
 // part/n_part/shift: where the block sums and the mean go (default: the
 // context's d_part, n_part, d_shift).
-template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long sy, bool want_sum, int img,
-                                   double *part = nullptr, size_t n_part = 0, double *shift = nullptr);
+// copies: how the ghosts of phi (gl_out == 1) along x, y, z are filled (COPY_*).
+// defer: leave the block sums unreduced (shift_parts) when there are at most
+// kDeferParts of them, for a 2-D projection that adds them itself.
+constexpr int kDeferParts = 256;
+struct AxisCopies {
+    int x = COPY_NONE, y = COPY_NONE, z = COPY_NONE;
+    __host__ __device__ bool any() const { return x || y || z; }
+};
+template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long sy, bool want_sum, AxisCopies copies,
+                                   double *part = nullptr, size_t n_part = 0, double *shift = nullptr,
+                                   bool defer = false);
+// The pending mean of phi from its block sums, if a 2-D step left it unreduced.
+void reduce_shift(fen_ctx *c);
+// The last checks' maxima into d_scal, if they are still per block.
+void reduce_checks(fen_ctx *c);
 // store == false: the checks of the projection only (max div, max |u|+|v|+|w|
 // of the projected velocity), nothing written but the reduction (3-D).
-template <class R> void launch_project(fen_ctx *c, double dt, double *checks_out, bool store = true);
+// The checks stay in d_chk until reduce_checks.  In 2-D the projection also
+// fills the ghosts of u, v and p, and `p_old` (two-phase) receives p before it.
+template <class R> void launch_project(fen_ctx *c, double dt, bool store = true, R *p_old = nullptr);
 bool fused_z_walls(const fen_ctx *c);
 void mf_advect_vof(fen_ctx *c, double dt);
 // p_hat = 2 p - p_o, or with `dt` > 0 (constant CFL) p_o + (dt + dt_o)(p - p_o)/dt_o.
@@ -303,15 +380,13 @@ bool fused_general_walls(const fen_ctx *c);
 template <class R>
 void launch_project_momentum(fen_ctx *c, double dt_p, double dt_m, double A, double B, void *const *us_in,
                              const void *p_in, void *const *us_out, void *p_out, void *const *save = nullptr);
-template <class R> void launch_checks(fen_ctx *c, const R *const *vel, double *out2);
+template <class R> void launch_checks(fen_ctx *c, const R *const *vel);
+template <class R> GhostDesc<R> make_desc(fen_ctx *c, int field, void *arr);   // fen_api.hip
 long stencil_blocks(const Box &b);   // workgroups of the momentum / projection grids
 // Neumann-direction solver passes (neumann_kernels.hip, FP64).
 void launch_dct2_x(fen_ctx *c, const double *const *vel, const double *direct, long sx, long sy, int gl, double rho,
                    double dt, double post);
-// Whether every ghost of phi is a copy of an interior value (x Neumann;
-// y, z periodic or Neumann), so that the x DCT-III can write them.
-bool dct3_writes_ghosts(const fen_ctx *c);
-void launch_dct3_x(fen_ctx *c, double *phi, int gl, long sx, long sy, double post, bool img = false);
+void launch_dct3_x(fen_ctx *c, double *phi, int gl, long sx, long sy, double post, AxisCopies copies);
 void launch_dct_y(fen_ctx *c, int inverse, double post);
 void launch_rfft_y(fen_ctx *c, int inverse, double post);
 void launch_thomas_neumann(fen_ctx *c);

@@ -209,11 +209,11 @@ __global__ __launch_bounds__(256) void mf_fields_kernel(long n, const double *vo
 }
 
 struct MFMomArgs {
+    GhostDesc<double> gu, gv;   // u* and v*, left with their ghosts filled
     Box b;
     double id, dt, A, B, g0, g1, sigma, irhomin;
     const double *u, *v, *p, *p_hat, *rho, *mu, *vof, *curv, *s0, *s1;
     double *us, *vs, *dvo0, *dvo1;
-    int img;
 };
 
 // predicted_velocity_field with MF (src/navier_stokes.f90:140-213): advection
@@ -285,8 +285,7 @@ template <int SRC> __global__ __launch_bounds__(kBX *kBY) void mf_momentum_kerne
         double rhs = ((-(gp / rfx) + a.A * rx) + a.B * a.dvo0[q]) + a.g0;
         rhs = ((rhs + gp / rfx) - a.irhomin * gp) - (1.0 / rfx - a.irhomin) * gh;
         const double val = u0 + a.dt * rhs;
-        a.us[g] = val;
-        write_images(a.us, a.b, a.img, i, j, 1, val);
+        put_ghosted(a.gu, a.b, a.us, i, j, val);
         a.dvo0[q] = rx;
     }
     {
@@ -294,8 +293,7 @@ template <int SRC> __global__ __launch_bounds__(kBX *kBY) void mf_momentum_kerne
         double rhs = ((-(gp / rfy) + a.A * ry) + a.B * a.dvo1[q]) + a.g1;
         rhs = ((rhs + gp / rfy) - a.irhomin * gp) - (1.0 / rfy - a.irhomin) * gh;
         const double val = v0 + a.dt * rhs;
-        a.vs[g] = val;
-        write_images(a.vs, a.b, a.img, i, j, 1, val);
+        put_ghosted(a.gv, a.b, a.vs, i, j, val);
         a.dvo1[q] = ry;
     }
 }
@@ -412,7 +410,8 @@ void mf_momentum(fen_ctx *c, double dt)
     a.s0 = as<double>(c->d_S[0]); a.s1 = as<double>(c->d_S[1]);
     a.us = as<double>(c->d_us[0]); a.vs = as<double>(c->d_us[1]);
     a.dvo0 = as<double>(c->d_dvo[0]); a.dvo1 = as<double>(c->d_dvo[1]);
-    a.img = c->img_vel;
+    a.gu = make_desc<double>(c, FEN_U, a.us);
+    a.gv = make_desc<double>(c, FEN_V, a.vs);
     prof_begin(c, K_MOMENTUM);
     if (c->has_source) hipLaunchKernelGGL(mf_momentum_kernel<1>, cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, a);
     else hipLaunchKernelGGL(mf_momentum_kernel<0>, cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, a);

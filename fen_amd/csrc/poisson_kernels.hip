@@ -107,8 +107,8 @@ template <class R> struct C2RArgs {
     int ny, gl, want_sum;
     int ny_shift;   // log2(ny)
     double *part;
-    Box b;     // ghosted box of `out` when img != 0
-    int img;   // periodic image axes to write (phi in the time step)
+    int nz;
+    AxisCopies copies;   // ghosts to write (phi in the time step)
 };
 
 template <class R, int N, int NT = kBlock>
@@ -163,15 +163,26 @@ __global__ __launch_bounds__(NT) void c2r_kernel(C2RArgs<R> a)
         const long r = row0 + 2 * l + h;
         if (r >= a.nrows) continue;
         const int j = (int)(r & (a.ny - 1)), k = (int)(r >> a.ny_shift);
-        R *orow = a.out + a.gl + a.sx * (j + a.gl) + a.sy * (k + a.gl);
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int i = t + q * (N / 8);
-            const R val = h ? v[q].y : v[q].x;
-            orow[i] = val;
-            if (a.img) write_images(a.out, a.b, a.img, i + 1, j + 1, k + 1, val);
-            acc += (double)val;
+        // the row and the ghost rows that copy it, each with its x ghosts
+        int jd[3], kd[3], nj = 1, nk = 1;
+        jd[0] = j + a.gl;
+        kd[0] = k + a.gl;
+        if (a.copies.any()) {
+            nj = copy_rows(j + 1, a.ny, a.copies.y, jd);
+            nk = copy_rows(k + 1, a.nz, a.copies.z, kd);
         }
+        for (int dk = 0; dk < nk; dk++)
+            for (int dj = 0; dj < nj; dj++) {
+                R *orow = a.out + a.gl + a.sx * jd[dj] + a.sy * kd[dk];
+#pragma unroll
+                for (int q = 0; q < 8; q++) orow[t + q * (N / 8)] = h ? v[q].y : v[q].x;
+                if (a.copies.x) {   // periodic: x(0) = x(n), x(n + 1) = x(1)
+                    if (t == 0) orow[N] = h ? v[0].y : v[0].x;
+                    if (t == T - 1) orow[-1] = h ? v[7].y : v[7].x;
+                }
+            }
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc += (double)(h ? v[q].y : v[q].x);
     }
     if (a.want_sum) {   // fft_regs has finished every read of buf: reuse it
         double *red = reinterpret_cast<double *>(buf);
@@ -715,9 +726,19 @@ long c2r_blocks(const fen_ctx *c)
     return ((long)c->ny * c->nz + tj - 1) / tj;
 }
 
-template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long sy, bool want_sum, int img,
-                                   double *part, size_t n_part, double *shift)
+static void launch_mean_shift(fen_ctx *c, const double *part, long nblk, double *shift)
 {
+    const double count = (double)(float)((long)c->nx * c->ny * c->nz);
+    prof_begin(c, K_REDUCE);
+    hipLaunchKernelGGL(mean_shift_kernel, dim3(1), dim3(kShiftThreads), 0, c->stream, part, nblk, count, shift);
+    prof_end(c, K_REDUCE, 8.0 * nblk);
+}
+
+template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long sy, bool want_sum,
+                                   AxisCopies copies, double *part, size_t n_part, double *shift, bool defer)
+{
+    if (copies.any() && gl_out != 1) throw std::runtime_error("c2r ghost writes need gl == 1");
+    if (copies.x == COPY_MIRROR) throw std::runtime_error("the c2r's x axis is periodic");
     if (!part) {
         part = c->d_part;
         n_part = c->n_part;
@@ -736,8 +757,8 @@ template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long
     a.ny_shift = ilog2(c->ny);
     a.want_sum = want_sum ? 1 : 0;
     a.part = part;
-    a.b = c->box;
-    a.img = img;
+    a.nz = c->nz;
+    a.copies = copies;
     const long nblk = c2r_blocks(c);
     if (want_sum && (size_t)nblk > n_part) throw std::runtime_error("partial-sum buffer too small");
     prof_begin(c, K_C2R);
@@ -746,16 +767,21 @@ template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long
 #undef L_C
     prof_end(c, K_C2R, spec_bytes<R>(c) + sizeof(R) * c->n_int);
     if (want_sum) {
-        const double count = (double)(float)((long)c->nx * c->ny * c->nz);
-        prof_begin(c, K_REDUCE);
-        hipLaunchKernelGGL(mean_shift_kernel, dim3(1), dim3(kShiftThreads), 0, c->stream, (const double *)part, nblk,
-                           count, shift);
-        prof_end(c, K_REDUCE, 8.0 * nblk);
+        if (defer && nblk <= kDeferParts) c->shift_parts = nblk;
+        else launch_mean_shift(c, part, nblk, shift);
     }
+}
+
+void reduce_shift(fen_ctx *c)
+{
+    if (!c->shift_active || c->shift_parts <= 0) return;
+    launch_mean_shift(c, c->d_part, c->shift_parts, c->d_shift);
+    c->shift_parts = 0;
 }
 
 template <class R> void launch_apply_shift(fen_ctx *c, R *f, size_t n)
 {
+    reduce_shift(c);
     hipLaunchKernelGGL(apply_shift_kernel<R>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, f, (long)n,
                        (const double *)c->d_shift);
     prof_end(c, K_REDUCE, 2.0 * sizeof(R) * n);
@@ -768,7 +794,8 @@ template <class R> void launch_apply_shift(fen_ctx *c, R *f, size_t n)
     template void launch_y_solve_2d<R>(fen_ctx *, double);                                                     \
     template void launch_z_solve<R>(fen_ctx *, double);                                                        \
     template void launch_thomas<R>(fen_ctx *);                                                                 \
-    template void launch_c2r<R>(fen_ctx *, R *, int, long, long, bool, int, double *, size_t, double *);       \
+    template void launch_c2r<R>(fen_ctx *, R *, int, long, long, bool, AxisCopies, double *, size_t, double *, \
+                                bool);                                                                         \
     template void launch_apply_shift<R>(fen_ctx *, R *, size_t);
 FEN_INSTANTIATE(double)
 FEN_INSTANTIATE(float)

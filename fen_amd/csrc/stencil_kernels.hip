@@ -210,9 +210,12 @@ template <class R> void launch_ghost_desc(fen_ctx *c, const GhostDesc<R> *descs,
 }
 
 // 2-D: one cell per thread, neighbours straight from memory (the whole
-// 128^2 problem fits in cache).
+// 128^2 problem fits in cache); u* and v* are left with their ghosts filled.
+template <class R> struct Ghosts2D {
+    GhostDesc<R> d[3];
+};
 template <class R, int SRC>
-__global__ __launch_bounds__(kThreads) void momentum_kernel_2d(MomArgs<R> a)
+__global__ __launch_bounds__(kThreads) void momentum_kernel_2d(MomArgs<R> a, Ghosts2D<R> gh)
 {
     const int i = blockIdx.x * kTX + (threadIdx.x % kTX) + 1;
     const int j = blockIdx.y * kTY + (threadIdx.x / kTX) + 1;
@@ -222,8 +225,11 @@ __global__ __launch_bounds__(kThreads) void momentum_kernel_2d(MomArgs<R> a)
         return [=](int di, int dj, int dk) { return f[g + di + sj * dj]; };
     };
     const long q = a.b.q(i, j, 1);
-    auto img = [&](R *f, R v) { write_images(f, a.b, a.img, i, j, 1, v); };
-    momentum_cell<0, SRC>(a, i, j, 1, at(a.u), at(a.v), at(a.w), at(a.p), a.dvo0[q], a.dvo1[q], R(0), img);
+    R val[2] = {R(0), R(0)};
+    auto keep = [&](R *f, R v) { (f == a.us ? val[0] : val[1]) = v; };
+    momentum_cell<0, SRC>(a, i, j, 1, at(a.u), at(a.v), at(a.w), at(a.p), a.dvo0[q], a.dvo1[q], R(0), keep);
+    put_ghosted(gh.d[0], a.b, a.us, i, j, val[0]);
+    put_ghosted(gh.d[1], a.b, a.vs, i, j, val[1]);
 }
 
 // 3-D launch shapes (see stencil_march.hpp), chosen per element type by a
@@ -291,8 +297,11 @@ template <class R> void launch_momentum(fen_ctx *c, double dt, double A, double 
                                grid, dim3(SH::MTXW * SH::MTY), 0, c->stream, a);
     } else {
         const dim3 grid((unsigned)a.nbx, (unsigned)a.nby);
-        if (c->has_source) hipLaunchKernelGGL((momentum_kernel_2d<R, 1>), grid, dim3(kThreads), 0, c->stream, a);
-        else hipLaunchKernelGGL((momentum_kernel_2d<R, 0>), grid, dim3(kThreads), 0, c->stream, a);
+        Ghosts2D<R> gh{};
+        gh.d[0] = make_desc<R>(c, FEN_U, a.us);
+        gh.d[1] = make_desc<R>(c, FEN_V, a.vs);
+        if (c->has_source) hipLaunchKernelGGL((momentum_kernel_2d<R, 1>), grid, dim3(kThreads), 0, c->stream, a, gh);
+        else hipLaunchKernelGGL((momentum_kernel_2d<R, 0>), grid, dim3(kThreads), 0, c->stream, a, gh);
     }
     prof_end(c, K_MOMENTUM, words * sizeof(R) * c->n_int);
 }
@@ -357,23 +366,63 @@ void launch_advection_only(fen_ctx *c, double *rx, double *ry, double *rz)
                            1.0 / c->delta);
 }
 
-template <class R, int SHIFT>
-__global__ __launch_bounds__(kThreads) void project_kernel_2d(ProjArgs<R> a)
+// The mean of phi from its block sums (n <= kThreads), by mean_shift_kernel's
+// own tree, for every thread of the block.
+__device__ __forceinline__ double block_mean(const double *part, int n, double count)
+{
+    __shared__ double red[kThreads];
+    red[threadIdx.x] = (int)threadIdx.x < n ? part[threadIdx.x] : 0.0;
+    __syncthreads();
+    for (int s = kThreads / 2; s >= 64; s >>= 1) {
+        if ((int)threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + s];
+        __syncthreads();
+    }
+    if (threadIdx.x < 64) {
+        double x = red[threadIdx.x];
+        for (int s = 32; s > 0; s >>= 1) x = x + __shfl_down(x, s);
+        if (threadIdx.x == 0) red[0] = x;
+    }
+    __syncthreads();
+    return red[0] / count;
+}
+
+// The projection, pressure update and checks of a 2-D step, u, v and p left
+// with their ghosts filled.  nparts > 0: the mean of phi is still in its block
+// sums and every workgroup adds them (a launch of its own took 4 us).  p_old:
+// receives p before the update (two-phase).  ST == 0: the checks only.
+template <class R> struct Project2D {
+    Ghosts2D<R> gh;   // u, v, p
+    const double *part;
+    double count;
+    int nparts;
+    R *p_old;
+};
+template <class R, int SHIFT, int ST>
+__global__ __launch_bounds__(kThreads) void project_kernel_2d(ProjArgs<R> a, Project2D<R> x)
 {
     const int i = blockIdx.x * kTX + (threadIdx.x % kTX) + 1;
     const int j = blockIdx.y * kTY + (threadIdx.x / kTX) + 1;
     const Box &b = a.b;
     double md = -HUGE_VAL, mv = 0.0, bad = 0.0;
+    double s = 0.0;
+    if constexpr (SHIFT) s = x.nparts > 0 ? block_mean(x.part, x.nparts, x.count) : a.shift[0];
     if (i <= b.nx && j <= b.ny) {
         const long g = b.g(i, j, 1), sj = b.gx;
-        const double s = SHIFT ? a.shift[0] : 0.0;
         auto F = [&](int di, int dj, int dk) -> double {
             if constexpr (SHIFT) return (double)a.phi[g + di + sj * dj] - s;
             else return (double)a.phi[g + di + sj * dj];
         };
-        auto img = [&](R *f, R v) { write_images(f, a.b, a.img, i, j, 1, v); };
-        project_cell<0>(a, i, j, 1, F, a.us[g], a.vs[g], 0.0, a.p[g], a.us[g - 1], a.vs[g - sj], 0.0, md, mv, bad,
-                        img);
+        R val[3] = {R(0), R(0), R(0)};
+        auto keep = [&](R *f, R v) { (f == a.u ? val[0] : (f == a.v ? val[1] : val[2])) = v; };
+        const R p0 = ST ? a.p[g] : R(0);
+        project_cell<0, R, decltype(F), decltype(keep), ST>(a, i, j, 1, F, a.us[g], a.vs[g], 0.0, p0, a.us[g - 1],
+                                                            a.vs[g - sj], 0.0, md, mv, bad, keep);
+        if constexpr (ST) {
+            if (x.p_old) x.p_old[g] = p0;
+            put_ghosted(x.gh.d[0], b, a.u, i, j, val[0]);
+            put_ghosted(x.gh.d[1], b, a.v, i, j, val[1]);
+            put_ghosted(x.gh.d[2], b, a.p, i, j, val[2]);
+        }
     }
     block_max3<kThreads>(md, mv, bad, a.part, (long)blockIdx.y * gridDim.x + blockIdx.x);
 }
@@ -418,14 +467,24 @@ __global__ __launch_bounds__(kFinalThreads) void checks_final_kernel(const doubl
     if (threadIdx.x == 0) { out[0] = sd[0]; out[1] = sv[0]; out[2] = sf[0]; }
 }
 
-template <class R> void launch_project(fen_ctx *c, double dt, double *checks_out, bool store)
+void reduce_checks(fen_ctx *c)
 {
-    if (!store && c->box.dim != 3) throw std::runtime_error("checks-only projection is 3-D");
+    if (c->chk_blocks <= 0) return;
+    prof_begin(c, K_REDUCE);
+    hipLaunchKernelGGL(checks_final_kernel, dim3(1), dim3(kFinalThreads), 0, c->stream, (const double *)c->d_chk,
+                       c->chk_blocks, c->d_scal);
+    prof_end(c, K_REDUCE, 24.0 * c->chk_blocks);
+    c->chk_blocks = 0;
+}
+
+template <class R> void launch_project(fen_ctx *c, double dt, bool store, R *p_old)
+{
+    if (p_old && c->box.dim != 2) throw std::runtime_error("the pressure before the step is kept in 2-D only");
     ProjArgs<R> a{};
     a.us = as<R>(c->d_us[0]); a.vs = as<R>(c->d_us[1]); a.ws = as<R>(c->d_us[2]); a.phi = as<R>(c->d_phi);
     a.u = as<R>(c->d_u[0]); a.v = as<R>(c->d_u[1]); a.w = as<R>(c->d_u[2]); a.p = as<R>(c->d_p);
     a.shift = c->d_shift;
-    a.part = c->d_part;
+    a.part = c->d_chk;
     const int lo[3] = {FEN_LEFT, FEN_BOTTOM, FEN_FRONT}, hi[3] = {FEN_RIGHT, FEN_TOP, FEN_BACK};
     for (int d = 0; d < 3; d++) {
         const int slot = FEN_U + d;
@@ -450,7 +509,7 @@ template <class R> void launch_project(fen_ctx *c, double dt, double *checks_out
     using SH = Shape<R>;
     grid_blocks(c->box, SH::PTY, SH::PKB, &a.nbx, &a.nby, &nbz, SH::PTXW);
     const long nblk = (long)a.nbx * a.nby * nbz;
-    if ((size_t)(3 * nblk) > c->n_part) throw std::runtime_error("partial buffer too small");
+    if ((size_t)(3 * nblk) > c->n_chk) throw std::runtime_error("partial buffer too small");
     const bool sh = c->shift_active;
     const int d3 = c->box.dim == 3;
     const int kid = store ? K_PROJECT : K_CHECKS;
@@ -470,15 +529,28 @@ template <class R> void launch_project(fen_ctx *c, double dt, double *checks_out
 #undef FEN_PJ
     } else {
         const dim3 grid((unsigned)a.nbx, (unsigned)a.nby);
-        if (sh) hipLaunchKernelGGL((project_kernel_2d<R, 1>), grid, dim3(kThreads), 0, c->stream, a);
-        else hipLaunchKernelGGL((project_kernel_2d<R, 0>), grid, dim3(kThreads), 0, c->stream, a);
+        Project2D<R> x{};
+        x.gh.d[0] = make_desc<R>(c, FEN_U, a.u);
+        x.gh.d[1] = make_desc<R>(c, FEN_V, a.v);
+        x.gh.d[2] = make_desc<R>(c, FEN_P, a.p);
+        x.part = c->d_part;
+        x.nparts = (int)c->shift_parts;
+        x.count = (double)(float)((long)c->nx * c->ny * c->nz);
+        x.p_old = p_old;
+#define FEN_PJ2(SH_, ST_) \
+    hipLaunchKernelGGL((project_kernel_2d<R, SH_, ST_>), grid, dim3(kThreads), 0, c->stream, a, x)
+        if (store) {
+            if (sh) FEN_PJ2(1, 1);
+            else FEN_PJ2(0, 1);
+        } else {
+            if (sh) FEN_PJ2(1, 0);
+            else FEN_PJ2(0, 0);
+        }
+#undef FEN_PJ2
     }
     // the checks alone read u*, v*, w* and phi
     prof_end(c, kid, (store ? (d3 ? 9.0 : 7.0) : 4.0) * sizeof(R) * c->n_int);
-    prof_begin(c, K_REDUCE);
-    hipLaunchKernelGGL(checks_final_kernel, dim3(1), dim3(kFinalThreads), 0, c->stream, (const double *)c->d_part,
-                       nblk, checks_out);
-    prof_end(c, K_REDUCE, 24.0 * nblk);
+    c->chk_blocks = nblk;
 }
 
 // ---------------------------------------------------------------------------
@@ -525,34 +597,31 @@ __global__ __launch_bounds__(256) void checks_kernel(const R *u, const R *v, con
     }
 }
 
-template <class R> void launch_checks(fen_ctx *c, const R *const *vel, double *out)
+template <class R> void launch_checks(fen_ctx *c, const R *const *vel)
 {
     const Box &b = c->box;
     const double id = 1.0 / c->delta;
     long nblk = ((long)c->n_int + 255) / 256;
     if (nblk > kCheckBlocks) nblk = kCheckBlocks;
-    if ((size_t)(3 * nblk) > c->n_part) throw std::runtime_error("partial buffer too small");
+    if ((size_t)(3 * nblk) > c->n_chk) throw std::runtime_error("partial buffer too small");
     prof_begin(c, K_CHECKS);
     if (b.dim == 3)
         hipLaunchKernelGGL((checks_kernel<R, 1>), dim3((unsigned)nblk), dim3(256), 0, c->stream, vel[0], vel[1],
-                           vel[2], b, id, c->d_part);
+                           vel[2], b, id, c->d_chk);
     else
         hipLaunchKernelGGL((checks_kernel<R, 0>), dim3((unsigned)nblk), dim3(256), 0, c->stream, vel[0], vel[1],
-                           vel[2], b, id, c->d_part);
+                           vel[2], b, id, c->d_chk);
     prof_end(c, K_CHECKS, (b.dim == 3 ? 3.0 : 2.0) * sizeof(R) * c->n_int);
-    prof_begin(c, K_REDUCE);
-    hipLaunchKernelGGL(checks_final_kernel, dim3(1), dim3(kFinalThreads), 0, c->stream, (const double *)c->d_part,
-                       nblk, out);
-    prof_end(c, K_REDUCE, 24.0 * nblk);
+    c->chk_blocks = nblk;
 }
 
 template void launch_ghost_desc<double>(fen_ctx *, const GhostDesc<double> *, int);
 template void launch_ghost_desc<float>(fen_ctx *, const GhostDesc<float> *, int);
 template void launch_momentum<double>(fen_ctx *, double, double, double);
 template void launch_momentum<float>(fen_ctx *, double, double, double);
-template void launch_project<double>(fen_ctx *, double, double *, bool);
-template void launch_project<float>(fen_ctx *, double, double *, bool);
-template void launch_checks<double>(fen_ctx *, const double *const *, double *);
-template void launch_checks<float>(fen_ctx *, const float *const *, double *);
+template void launch_project<double>(fen_ctx *, double, bool, double *);
+template void launch_project<float>(fen_ctx *, double, bool, float *);
+template void launch_checks<double>(fen_ctx *, const double *const *);
+template void launch_checks<float>(fen_ctx *, const float *const *);
 
 }  // namespace fen
