@@ -8,8 +8,8 @@
 //   K6 x c2r or DCT-III -> phi (+ mean, pp/ppn/pn)   ghost(phi)
 //   K7 projection + p update           ghost(u, p)
 //   K8 checks
-// On the 3-D grids the fused kernel supports (periodic, or periodic in x, y
-// with walls at z) a step ends after K6 with K7-K8 pending; the next step
+// On the grids the fused kernels support (deferrable) a step ends after K6 with
+// K7-K8 pending; the next step
 // runs them fused with its K1 (step_pending), and anything that reads or
 // changes the state first completes them (flush_pending).
 #include <algorithm>
@@ -518,10 +518,12 @@ void advance_mf(fen_ctx *c, double dt)
 // Whether a step may end with its projection pending, to be fused into the
 // next step's momentum (launch_project_momentum): 3-D, every field periodic
 // in every direction (ppp), x, y periodic with no-slip walls at z (ppn), or
-// npn/nnn in FP64 with the standard wall rules.
+// npn/nnn in FP64 with the standard wall rules; 2-D with walls of the same
+// kind on both faces (launch_step_2d).
 bool deferrable(const fen_ctx *c)
 {
-    if (!c->fused_run || c->dim != 3 || c->mf) return false;
+    if (!c->fused_run || c->mf) return false;
+    if (c->dim == 2) return fen::fused_2d(c);
     if (c->solver == FEN_SOLVER_PPP) return c->img_vel == 7 && c->img_p == 7 && c->img_phi == 7;
     if (c->solver == FEN_SOLVER_PPN) return fen::fused_z_walls(c);
     return fen::fused_general_walls(c);   // npn, nnn (FP64)
@@ -547,7 +549,8 @@ template <class R> void step_pending(fen_ctx *c, double dt, void *const *save = 
         c->last_dt = dt;
         c->step_count++;
         void *out[3] = {c->d_u[0], c->d_u[1], c->d_u[2]};
-        launch_project_momentum<R>(c, c->pend_dt, dt, A, B, c->d_us, c->d_p, out, c->d_p2, save);
+        if (c->dim == 2) launch_step_2d<R>(c, c->pend_dt, dt, A, B, c->d_us, c->d_p, out, c->d_p2);
+        else launch_project_momentum<R>(c, c->pend_dt, dt, A, B, c->d_us, c->d_p, out, c->d_p2, save);
         for (int d = 0; d < 3; d++) std::swap(c->d_u[d], c->d_us[d]);
         std::swap(c->d_p, c->d_p2);
         c->config_version++;   // a captured step graph holds the old array roles

@@ -380,6 +380,11 @@ bool fused_general_walls(const fen_ctx *c);
 template <class R>
 void launch_project_momentum(fen_ctx *c, double dt_p, double dt_m, double A, double B, void *const *us_in,
                              const void *p_in, void *const *us_out, void *p_out, void *const *save = nullptr);
+// The 2-D counterpart.
+bool fused_2d(const fen_ctx *c);
+template <class R>
+void launch_step_2d(fen_ctx *c, double dt_p, double dt_m, double A, double B, void *const *us_in, const void *p_in,
+                    void *const *us_out, void *p_out);
 template <class R> void launch_checks(fen_ctx *c, const R *const *vel);
 template <class R> GhostDesc<R> make_desc(fen_ctx *c, int field, void *arr);   // fen_api.hip
 long stencil_blocks(const Box &b);   // workgroups of the momentum / projection grids

@@ -281,25 +281,35 @@ __device__ __forceinline__ void project_cell(const ProjArgs<R> &a, int i, int j,
     if (vel > mv) mv = vel;
 }
 
-// Block-wide max of (maxdiv, maxvel, nonfinite flag) -> part[3*bid..].
+// Block-wide max of (maxdiv, maxvel, nonfinite flag) -> part[3*bid..]: each
+// wave by cross-lane reads, the waves through LDS with one barrier (a tree of
+// eight barriers over 256 threads took a fifth of a 2-D projection).
 template <int NT>
 __device__ __forceinline__ void block_max3(double md, double mv, double bad, double *part, long bid)
 {
-    __shared__ double sd[NT], sv[NT], sf[NT];
-    sd[threadIdx.x] = md; sv[threadIdx.x] = mv; sf[threadIdx.x] = bad;
-    __syncthreads();
-    for (int st = NT / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) {
-            if (sd[threadIdx.x + st] > sd[threadIdx.x]) sd[threadIdx.x] = sd[threadIdx.x + st];
-            if (sv[threadIdx.x + st] > sv[threadIdx.x]) sv[threadIdx.x] = sv[threadIdx.x + st];
-            if (sf[threadIdx.x + st] > sf[threadIdx.x]) sf[threadIdx.x] = sf[threadIdx.x + st];
-        }
-        __syncthreads();
+    constexpr int NW = NT / 64;
+    __shared__ double sd[NW], sv[NW], sf[NW];
+    for (int st = 32; st > 0; st >>= 1) {
+        const double d = __shfl_down(md, st), v = __shfl_down(mv, st), f = __shfl_down(bad, st);
+        if (d > md) md = d;
+        if (v > mv) mv = v;
+        if (f > bad) bad = f;
     }
+    if ((threadIdx.x & 63) == 0) {
+        sd[threadIdx.x >> 6] = md;
+        sv[threadIdx.x >> 6] = mv;
+        sf[threadIdx.x >> 6] = bad;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        part[3 * bid + 0] = sd[0];
-        part[3 * bid + 1] = sv[0];
-        part[3 * bid + 2] = sf[0];
+        for (int w = 1; w < NW; w++) {
+            if (sd[w] > md) md = sd[w];
+            if (sv[w] > mv) mv = sv[w];
+            if (sf[w] > bad) bad = sf[w];
+        }
+        part[3 * bid + 0] = md;
+        part[3 * bid + 1] = mv;
+        part[3 * bid + 2] = bad;
     }
 }
 

@@ -209,6 +209,17 @@ template <class R> void launch_ghost_desc(fen_ctx *c, const GhostDesc<R> *descs,
     prof_end(c, K_GHOST, 2.0 * sizeof(R) * cells);
 }
 
+// The mean of phi from its block sums (n <= 256), by mean_shift_kernel's own
+// tree, in every wave by itself: no barrier.
+__device__ __forceinline__ double wave_mean(const double *part, int n, double count)
+{
+    const int l = threadIdx.x & 63;
+    auto at = [&](int q) { return q < n ? part[q] : 0.0; };
+    double x = (at(l) + at(l + 128)) + (at(l + 64) + at(l + 192));
+    for (int s = 32; s > 0; s >>= 1) x = x + __shfl_down(x, s);
+    return __shfl(x, 0) / count;
+}
+
 // 2-D: one cell per thread, neighbours straight from memory (the whole
 // 128^2 problem fits in cache); u* and v* are left with their ghosts filled.
 template <class R> struct Ghosts2D {
@@ -366,26 +377,6 @@ void launch_advection_only(fen_ctx *c, double *rx, double *ry, double *rz)
                            1.0 / c->delta);
 }
 
-// The mean of phi from its block sums (n <= kThreads), by mean_shift_kernel's
-// own tree, for every thread of the block.
-__device__ __forceinline__ double block_mean(const double *part, int n, double count)
-{
-    __shared__ double red[kThreads];
-    red[threadIdx.x] = (int)threadIdx.x < n ? part[threadIdx.x] : 0.0;
-    __syncthreads();
-    for (int s = kThreads / 2; s >= 64; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x < 64) {
-        double x = red[threadIdx.x];
-        for (int s = 32; s > 0; s >>= 1) x = x + __shfl_down(x, s);
-        if (threadIdx.x == 0) red[0] = x;
-    }
-    __syncthreads();
-    return red[0] / count;
-}
-
 // The projection, pressure update and checks of a 2-D step, u, v and p left
 // with their ghosts filled.  nparts > 0: the mean of phi is still in its block
 // sums and every workgroup adds them (a launch of its own took 4 us).  p_old:
@@ -405,7 +396,7 @@ __global__ __launch_bounds__(kThreads) void project_kernel_2d(ProjArgs<R> a, Pro
     const Box &b = a.b;
     double md = -HUGE_VAL, mv = 0.0, bad = 0.0;
     double s = 0.0;
-    if constexpr (SHIFT) s = x.nparts > 0 ? block_mean(x.part, x.nparts, x.count) : a.shift[0];
+    if constexpr (SHIFT) s = x.nparts > 0 ? wave_mean(x.part, x.nparts, x.count) : a.shift[0];
     if (i <= b.nx && j <= b.ny) {
         const long g = b.g(i, j, 1), sj = b.gx;
         auto F = [&](int di, int dj, int dk) -> double {
@@ -465,6 +456,151 @@ __global__ __launch_bounds__(kFinalThreads) void checks_final_kernel(const doubl
         __syncthreads();
     }
     if (threadIdx.x == 0) { out[0] = sd[0]; out[1] = sv[0]; out[2] = sf[0]; }
+}
+
+// Step n's projection and pressure update fused with step n+1's momentum in
+// 2-D: the state of step n is formed in LDS for a 64 x 4 tile and its halo (the
+// projection of the interior cell the ghost fill reads, then the fill's rule
+// chain on a wall position), p of step n is stored and the tile advanced to u*,
+// v* of step n+1, left with their ghosts filled.  Latency bounds it, as every
+// 2-D kernel: the projection (6.9 us at 128^2) and momentum (4.1) apart, one
+// launch of 5.5 together.
+template <class R> struct Step2D {
+    MomArgs<R> m;                            // momentum of step n+1 (m.u, m.v, m.p unused)
+    Ghosts2D<R> gh;                          // its u*, v*
+    const R *us, *vs, *phi, *p_in;           // step n
+    R *p_out;
+    const double *shift, *part;              // pending mean of phi, or its block sums (nparts > 0)
+    double count;
+    int nparts;
+    double id, dt, rhof, irhof;
+    int rpow2;
+    int wall, gtype[3];                      // PMArgs::wall, gtype of u, v, p
+    const R *const *gplane;                  // PMArgs::gplane (u, v, w, p)
+};
+template <class R, int SRC, int SHIFT>
+__global__ __launch_bounds__(kThreads) void step_kernel_2d(Step2D<R> a)
+{
+    constexpr int LX = kTX + 2, N = LX * (kTY + 2), PER = (N + kThreads - 1) / kThreads;
+    __shared__ R lds[3][N];
+    const Box &b = a.m.b;
+    const int i0 = blockIdx.x * kTX + 1, j0 = blockIdx.y * kTY + 1;
+    // every load is issued before the mean is known
+    R raw[PER][6];
+    int gi[PER], gj[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int e = threadIdx.x + q * kThreads, ee = e < N ? e : 0;
+        gi[q] = min(i0 - 1 + ee % LX, b.nx + 1);
+        gj[q] = min(j0 - 1 + ee / LX, b.ny + 1);
+        const long o = b.g(pm_src(gi[q], b.nx, a.wall & 1), pm_src(gj[q], b.ny, a.wall & 2), 1);
+        raw[q][0] = a.us[o];
+        raw[q][1] = a.vs[o];
+        raw[q][2] = a.p_in[o];
+        raw[q][3] = a.phi[o];
+        raw[q][4] = a.phi[o + 1];
+        raw[q][5] = a.phi[o + b.gx];
+    }
+    double s = 0.0;
+    if constexpr (SHIFT) s = a.nparts > 0 ? wave_mean(a.part, a.nparts, a.count) : a.shift[0];
+    auto dr = [&](double x) { return over_rho(x, a.rhof, a.irhof, a.rpow2); };
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int e = threadIdx.x + q * kThreads;
+        double f0 = (double)raw[q][3], fx = (double)raw[q][4], fy = (double)raw[q][5];
+        if constexpr (SHIFT) {
+            f0 = f0 - s; fx = fx - s; fy = fy - s;
+        }
+        R st[3] = {(R)((double)raw[q][0] - dr((fx - f0) * a.id * a.dt)), (R)((double)raw[q][1] - dr((fy - f0) * a.id * a.dt)),
+                   (R)((double)raw[q][2] + f0)};
+        if (((a.wall & 1) && pm_wall_pos(gi[q], b.nx) >= 0) || ((a.wall & 2) && pm_wall_pos(gj[q], b.ny) >= 0)) {
+            const int jy = pm_src(gj[q], b.ny, a.wall & 2);
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+                st[f] = pm_ghost_chain(a.gtype[f], a.gplane + 6 * (f == 2 ? 3 : f), b, a.wall & 3, gi[q], gj[q], 1, jy, 1, st[f]);
+        }
+        if (e < N)
+#pragma unroll
+            for (int f = 0; f < 3; f++) lds[f][e] = st[f];
+    }
+    __syncthreads();
+    const int tx = threadIdx.x % kTX, ty = threadIdx.x / kTX, i = i0 + tx, j = j0 + ty;
+    if (i > b.nx || j > b.ny) return;
+    const int c = (ty + 1) * LX + tx + 1;
+    auto at = [&](int f) {
+        return [=](int di, int dj, int dk) { return lds[f][c + dj * LX + di]; };
+    };
+    const long q = b.q(i, j, 1);
+    a.p_out[b.g(i, j, 1)] = lds[2][c];
+    R val[2] = {R(0), R(0)};
+    auto keep = [&](R *f, R v) { (f == a.m.us ? val[0] : val[1]) = v; };
+    momentum_cell<0, SRC>(a.m, i, j, 1, at(0), at(1), at(0), at(2), a.m.dvo0[q], a.m.dvo1[q], R(0), keep);
+    put_ghosted(a.gh.d[0], b, a.m.us, i, j, val[0]);
+    put_ghosted(a.gh.d[1], b, a.m.vs, i, j, val[1]);
+}
+
+// Whether a 2-D step may end with its projection pending: every axis of u, v,
+// p and phi periodic on both faces, or walled on both (Dirichlet or Neumann);
+// phi's walls Neumann (its ghosts are then filled by the solve).
+bool fused_2d(const fen_ctx *c)
+{
+    if (c->box.dim != 2) return false;
+    for (int ax = 0; ax < 2; ax++)
+        for (int f : {FEN_U, FEN_V, FEN_P, FEN_PHI})
+            for (int side = 0; side < 2; side++) {
+                const int t = c->bc_type[f][2 * ax + side];
+                if (c->periodic[ax] ? t != 0 : (f == FEN_PHI ? t != 2 : t != 1 && t != 2)) return false;
+            }
+    return true;
+}
+
+// us_in, p_in: u*, v* and p of step n; us_out, p_out: u*, v* of step n+1 and p
+// after step n (distinct arrays).
+template <class R>
+void launch_step_2d(fen_ctx *c, double dt_p, double dt_m, double A, double B, void *const *us_in, const void *p_in,
+                    void *const *us_out, void *p_out)
+{
+    if (!fused_2d(c)) throw std::runtime_error("fused 2-D step needs periodic or walled axes");
+    Step2D<R> a{};
+    a.m = momentum_args<R>(c, dt_m, A, B);
+    a.m.us = as<R>(us_out[0]);
+    a.m.vs = as<R>(us_out[1]);
+    a.gh.d[0] = make_desc<R>(c, FEN_U, a.m.us);
+    a.gh.d[1] = make_desc<R>(c, FEN_V, a.m.vs);
+    a.us = as<R>(us_in[0]);
+    a.vs = as<R>(us_in[1]);
+    a.phi = as<R>(c->d_phi);
+    a.p_in = static_cast<const R *>(p_in);
+    a.p_out = as<R>(p_out);
+    a.shift = c->d_shift;
+    a.part = c->d_part;
+    a.nparts = (int)c->shift_parts;
+    a.count = (double)(float)((long)c->nx * c->ny * c->nz);
+    a.id = 1.0 / c->delta;
+    a.dt = dt_p;
+    a.rhof = 0.5 * (c->density + c->density);
+    a.rpow2 = pow2_value(a.rhof) ? 1 : 0;
+    a.irhof = a.rpow2 ? 1.0 / a.rhof : 0.0;
+    a.wall = (c->periodic[0] ? 0 : 1) | (c->periodic[1] ? 0 : 2);
+    const int fid[3] = {FEN_U, FEN_V, FEN_P}, loc[3] = {1, 2, 0};
+    for (int q = 0; q < 3; q++) {
+        a.gtype[q] = loc[q] << 12;
+        for (int f = 0; f < 4; f++) a.gtype[q] |= c->bc_type[fid[q]][f] << (2 * f);
+    }
+    a.gplane = reinterpret_cast<const R *const *>(c->d_plane_tab);
+    const dim3 grid((unsigned)((c->nx + kTX - 1) / kTX), (unsigned)((c->ny + kTY - 1) / kTY));
+    prof_begin(c, K_PROJ_MOM);
+#define FEN_S2(SRC, SH) hipLaunchKernelGGL((step_kernel_2d<R, SRC, SH>), grid, dim3(kThreads), 0, c->stream, a)
+    if (c->has_source) {
+        if (c->shift_active) FEN_S2(1, 1);
+        else FEN_S2(1, 0);
+    } else {
+        if (c->shift_active) FEN_S2(0, 1);
+        else FEN_S2(0, 0);
+    }
+#undef FEN_S2
+    // reads u*, v*, p, phi, dv_o (+ S); writes p, u*, v*, dv_o
+    prof_end(c, K_PROJ_MOM, (c->has_source ? 13.0 : 11.0) * sizeof(R) * c->n_int);
 }
 
 void reduce_checks(fen_ctx *c)
@@ -621,6 +757,10 @@ template void launch_momentum<double>(fen_ctx *, double, double, double);
 template void launch_momentum<float>(fen_ctx *, double, double, double);
 template void launch_project<double>(fen_ctx *, double, bool, double *);
 template void launch_project<float>(fen_ctx *, double, bool, float *);
+template void launch_step_2d<double>(fen_ctx *, double, double, double, double, void *const *, const void *, void *const *,
+                                     void *);
+template void launch_step_2d<float>(fen_ctx *, double, double, double, double, void *const *, const void *, void *const *,
+                                    void *);
 template void launch_checks<double>(fen_ctx *, const double *const *);
 template void launch_checks<float>(fen_ctx *, const float *const *);
 

@@ -10,7 +10,8 @@ import numpy as np
 import pytest
 
 from fen_amd import Solver
-from fen_amd._lib import BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, BOTTOM, LEFT, P, PHI, RIGHT, TOP, U, V, VOF
+from fen_amd._lib import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, BOTTOM, DVO_X, DVO_Y, FP32_REFINE, LEFT, P, PHI,
+                          RIGHT, S_X, S_Y, TOP, U, V, VOF)
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -107,3 +108,44 @@ def test_two_phase_steps_match_oracle(n, faces):
         g.navier_stokes_solver(step, dt, want_checks=False)
         o.step(step, dt)
     _compare(g, o, (U, V, VOF))
+
+
+@pytest.mark.parametrize("precision,source", [(0, False), (0, True), (FP32_REFINE, True)])
+@pytest.mark.parametrize("n,faces,types", [c for c in CASES if In not in c[1]] + [((64, 256), [Pe] * 4, {}), ((512, 16), [Wa] * 4, {})])
+def test_fused_steps_equal_single_steps(n, faces, types, precision, source, monkeypatch):
+    """The projection fused with the next step's momentum, bit for bit."""
+    if precision and Wa in faces:
+        pytest.skip("the FP32 form is periodic in 2-D")
+    print("fused 2-D", n, faces, types, precision, source, flush=True)
+    rng = np.random.default_rng(5)
+    init = {f: np.asfortranarray(0.1 * rng.standard_normal((n[0] + 2, n[1] + 2, 3))) for f in (U, V, P)}
+    planes = {(f, face): 0.05 * rng.standard_normal((n[1] + 2 if face < 2 else n[0] + 2, 3))
+              for f in (U, V) for face in (LEFT, RIGHT, BOTTOM, TOP)}
+    force = {f: np.asfortranarray(rng.standard_normal((n[0], n[1], 1))) for f in (S_X, S_Y)} if source else {}
+    res = {}
+    for fused in ("1", "0"):
+        monkeypatch.setenv("FEN_FUSED_RUN", fused)
+        g = Solver(2, (n[0], n[1], 1), (1.0, n[1] / n[0], 1.0), bc=faces + [Pe, Pe], precision=precision)
+        g.set_params(density=1.3, viscosity=0.02, g=(0.3, 0.0, 0.0), cfl=0.2)
+        for (f, face), t in types.items():
+            g.set_bc_type(f, face, t)
+        for (f, face), a in planes.items():
+            g.set_bc_plane(f, face, a)
+        for f, a in {**init, **force}.items():
+            g.upload(f, a)
+            if f in init:
+                g.update_ghost_nodes(f)
+        g.set_dt_o(0.02 / n[0])
+        out = []
+        for step in range(1, 6):
+            g.navier_stokes_solver(step, 0.02 / n[0], want_checks=False)
+            if step in (2, 3):
+                sc = g.scalars()      # the checks of a pending step
+                out += [sc["maxdiv"], sc["maxcfl"]]
+            if step == 3:
+                out += [g.download(f)[:, :, 1] for f in (U, V)]
+        out += [g.download(f)[:, :, 1] for f in (U, V, P, PHI)] + [g.download(f) for f in (DVO_X, DVO_Y)]
+        res[fused] = out
+        g.close()
+    for k, (a, b) in enumerate(zip(res["1"], res["0"])):
+        assert np.array_equal(np.asarray(a), np.asarray(b)), k
