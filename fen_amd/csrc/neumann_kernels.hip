@@ -26,7 +26,7 @@ namespace {
 constexpr int kNB = 256;
 
 template <int N> constexpr int nb_tpl() { return N / 8; }           // threads per complex line
-template <int N> constexpr int nb_lines() { return kNB / (N / 8); } // complex lines per block
+template <int N, int NT = kNB> constexpr int nb_lines() { return NT / (N / 8); } // complex lines per block
 
 // Position of x_i in Makhoul's reordered sequence v.
 __device__ __forceinline__ int mk_pos(int i, int n) { return (i & 1) ? n - 1 - (i >> 1) : (i >> 1); }
@@ -54,12 +54,12 @@ struct DctArgs {
 // 2L rows from their packed spectra in LDS (row 2l in Re, 2l + 1 in Im of
 // line l), times post.  Adjacent threads write adjacent addresses: rows
 // (x pass, orr = 1) or k (y pass, ok = 1).
-template <int N>
+template <int N, int NT = kNB>
 __device__ __forceinline__ void dct2_out(const DctArgs &a, const double2 *buf, const double2 *mks, long row0)
 {
-    constexpr int L = nb_lines<N>(), TJ = 2 * L, LL = lds_line<N>();
+    constexpr int L = nb_lines<N, NT>(), TJ = 2 * L, LL = lds_line<N>();
     const bool k_fast = a.ok == 1;
-    if constexpr (kNB % TJ == 0) {
+    if constexpr (NT % TJ == 0) {
         if (!k_fast) {
             // x pass: a thread keeps one row and walks k
             const int row = threadIdx.x % TJ;
@@ -68,7 +68,10 @@ __device__ __forceinline__ void dct2_out(const DctArgs &a, const double2 *buf, c
             const long zo = a.okz ? (long)((int)r / a.b.ny) * a.okz : 0;   // rows < 2^31: 32-bit division
             double *o = a.out + r * a.orr + zo;
             const double2 *line = buf + (row >> 1) * LL;
-            for (int k = threadIdx.x / TJ; k < N; k += kNB / TJ) {
+            // four steps' table entries are loaded together (one by one each
+            // step waited for its own)
+#pragma unroll 4
+            for (int k = threadIdx.x / TJ; k < N; k += NT / TJ) {
                 const double2 zk = line[lds_pad(k)], zn = line[lds_pad((N - k) & (N - 1))];
                 const double c = mks[k].x, s = mks[k].y;
                 double y;
@@ -79,7 +82,7 @@ __device__ __forceinline__ void dct2_out(const DctArgs &a, const double2 *buf, c
             return;
         }
     }
-    for (int e = threadIdx.x; e < TJ * N; e += kNB) {
+    for (int e = threadIdx.x; e < TJ * N; e += NT) {
         const int row = k_fast ? e / N : e % TJ, k = k_fast ? e % N : e / TJ;
         const long r = row0 + row;
         if (r >= a.nrows) continue;
@@ -165,11 +168,12 @@ __global__ __launch_bounds__(kNB) void dct2_rows_kernel(DctArgs a)
 //   T-j, and thread 0 takes its own from chunk r+1 (lane 0 loads a fifth
 //   pair, q = N, for x_{N-1}).  Needs 16-byte aligned fields and even gx.
 // MKL: the (cos, sin) table of the last step in LDS (it costs the x pass an
-// LDS-bound workgroup per CU, so only the y pass takes it).
-template <int N, int SRC, int MKL>
-__global__ __launch_bounds__(kNB) void dct2_pairs_kernel(DctArgs a)
+// LDS-bound workgroup per CU, so only the y pass and one-wave workgroups take
+// it).
+template <int N, int SRC, int MKL, int NT = kNB>
+__global__ __launch_bounds__(NT) void dct2_pairs_kernel(DctArgs a)
 {
-    constexpr int T = nb_tpl<N>(), L = nb_lines<N>(), TJ = 2 * L, LL = lds_line<N>();
+    constexpr int T = nb_tpl<N>(), L = nb_lines<N, NT>(), TJ = 2 * L, LL = lds_line<N>();
     static_assert(T <= 64 && (SRC == 0 || SRC == 2), "one wave per line; x pass or y pass");
     __shared__ double2 buf[L * LL];
     __shared__ double2 tw[N];
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(kNB) void dct2_pairs_kernel(DctArgs a)
 #pragma unroll
     for (int q = 0; q < 8; q++) line[lds_pad(j + q * T)] = v[q];
     __syncthreads();
-    dct2_out<N>(a, buf, mks, row0);
+    dct2_out<N, NT>(a, buf, mks, row0);
 }
 
 // ---------------------------------------------------------------------------
@@ -263,10 +267,10 @@ struct Dct3Args {
     double post;
 };
 
-template <int N, int DST>
-__global__ __launch_bounds__(kNB) void dct3_rows_kernel(Dct3Args a)
+template <int N, int DST, int NT = kNB>
+__global__ __launch_bounds__(NT) void dct3_rows_kernel(Dct3Args a)
 {
-    constexpr int T = nb_tpl<N>(), L = nb_lines<N>(), LL = lds_line<N>();
+    constexpr int T = nb_tpl<N>(), L = nb_lines<N, NT>(), LL = lds_line<N>();
     __shared__ double2 buf[L * LL];
     __shared__ double2 tw[N];
     load_twiddles<N>(tw, a.tw);
@@ -297,12 +301,12 @@ __global__ __launch_bounds__(kNB) void dct3_rows_kernel(Dct3Args a)
     } else {
         // x pass: rows are the contiguous direction (ir = 1): staged through
         // LDS with adjacent threads on adjacent rows; all loads issue first
-        constexpr int PER = L * N / kNB;
-        static_assert(PER * kNB == L * N, "staging");
+        constexpr int PER = L * N / NT;
+        static_assert(PER * NT == L * N, "staging");
         double a1[PER], b1[PER], a2[PER], b2[PER];   // x_k and x_{N-k} of both rows
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            const int e = threadIdx.x + m * kNB;
+            const int e = threadIdx.x + m * NT;
             const int ls = e % L, k = e / L;
             const long r = row0 + 2 * ls;
             a1[m] = 0.0; b1[m] = 0.0; a2[m] = 0.0; b2[m] = 0.0;
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(kNB) void dct3_rows_kernel(Dct3Args a)
         }
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            const int e = threadIdx.x + m * kNB;
+            const int e = threadIdx.x + m * NT;
             const int ls = e % L, k = e / L;
             buf[ls * LL + lds_pad(k)] = packed(a1[m], b1[m], a2[m], b2[m], k);
         }
@@ -628,13 +632,45 @@ template <int ASSOC2D> __global__ __launch_bounds__(kNB) void thomas_c1_kernel(T
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <int N, int SRC, int MKL> static void launch_dct2_pairs(unsigned grid, hipStream_t s, const DctArgs &a)
+static unsigned row_blocks(long nrows, int N, int nt = kNB)
 {
-    if constexpr (N <= 512) hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, MKL>), dim3(grid), dim3(kNB), 0, s, a);
-    else throw std::logic_error("dct2_pairs_kernel takes N <= 512");
+    const int rows = 2 * (nt / (N / 8));
+    return (unsigned)((nrows + rows - 1) / rows);
 }
 
-static unsigned row_blocks(long nrows, int N) { return (unsigned)((nrows + 2 * (kNB / (N / 8)) - 1) / (2 * (kNB / (N / 8)))); }
+// Grids whose rows would fill fewer than half the CUs with 256-thread
+// workgroups take one wave per workgroup (256 x 200 nn: x DCT-II 11.6 -> 9.9
+// us, DCT-III 6.8 -> 6.0).
+static bool one_wave(const fen_ctx *c, long nrows, int N)
+{
+    return N <= 512 && (long)row_blocks(nrows, N) < c->num_cu / 2;
+}
+
+template <int N, int SRC, int MKL> static void launch_dct2_pairs(const fen_ctx *c, const DctArgs &a)
+{
+    if constexpr (N <= 512) {
+        if (one_wave(c, a.nrows, N))
+            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, 1, 64>), dim3(row_blocks(a.nrows, N, 64)), dim3(64), 0,
+                               c->stream, a);
+        else
+            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, MKL>), dim3(row_blocks(a.nrows, N)), dim3(kNB), 0, c->stream,
+                               a);
+    } else {
+        throw std::logic_error("dct2_pairs_kernel takes N <= 512");
+    }
+}
+
+template <int N, int DST> static void launch_dct3_n(const fen_ctx *c, const Dct3Args &a)
+{
+    if constexpr (N <= 512) {
+        if (one_wave(c, a.nrows, N)) {
+            hipLaunchKernelGGL((dct3_rows_kernel<N, DST, 64>), dim3(row_blocks(a.nrows, N, 64)), dim3(64), 0, c->stream,
+                               a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((dct3_rows_kernel<N, DST>), dim3(row_blocks(a.nrows, N)), dim3(kNB), 0, c->stream, a);
+}
 
 // x DCT-II of the rows of div(u*)*rho/dt (vel != nullptr) or of phi (direct)
 // into the real spectrum A[kx*nrows + r], times post.
@@ -664,7 +700,7 @@ void launch_dct2_x(fen_ctx *c, const double *const *vel, const double *direct, l
     const bool pairs = vel && c->nx <= 512 && c->box.gx % 2 == 0 && aligned16(a.u) && aligned16(a.v) &&
                        (!a.d3 || aligned16(a.w));
 #define L_D2(NN)                                                                              \
-    if (pairs) launch_dct2_pairs<NN, 0, 0>(grid, c->stream, a);                               \
+    if (pairs) launch_dct2_pairs<NN, 0, 0>(c, a);                                             \
     else if (vel) hipLaunchKernelGGL((dct2_rows_kernel<NN, 0>), dim3(grid), dim3(kNB), 0, c->stream, a); \
     else hipLaunchKernelGGL((dct2_rows_kernel<NN, 1>), dim3(grid), dim3(kNB), 0, c->stream, a);
     FEN_NB_DISPATCH(c->nx, L_D2)
@@ -694,9 +730,8 @@ void launch_dct3_x(fen_ctx *c, double *phi, int gl, long sx, long sy, double pos
         throw std::runtime_error("DCT-III ghost writes need gl == 1 and Neumann x faces");
     a.copies = copies;
     a.post = post;
-    const unsigned grid = row_blocks(a.nrows, c->nx);
     prof_begin(c, K_C2R);
-#define L_D3(NN) hipLaunchKernelGGL((dct3_rows_kernel<NN, 0>), dim3(grid), dim3(kNB), 0, c->stream, a);
+#define L_D3(NN) launch_dct3_n<NN, 0>(c, a);
     FEN_NB_DISPATCH(c->nx, L_D3)
 #undef L_D3
     prof_end(c, K_C2R, 16.0 * c->n_int);
@@ -721,7 +756,7 @@ void launch_dct_y(fen_ctx *c, int inverse, double post)
         a.orr = c->ny;
         // the register-loading form for N <= 512, with the DCT's (cos, sin) table in LDS
 #define L_DY(NN)                                                                              \
-    if (c->ny <= 512) launch_dct2_pairs<NN, 2, 1>(grid, c->stream, a);                        \
+    if (c->ny <= 512) launch_dct2_pairs<NN, 2, 1>(c, a);                                      \
     else hipLaunchKernelGGL((dct2_rows_kernel<NN, 2>), dim3(grid), dim3(kNB), 0, c->stream, a);
         FEN_NB_DISPATCH(c->ny, L_DY)
 #undef L_DY
@@ -735,7 +770,7 @@ void launch_dct_y(fen_ctx *c, int inverse, double post)
         a.ik = 1;
         a.ir = c->ny;
         a.post = post;
-#define L_DY3(NN) hipLaunchKernelGGL((dct3_rows_kernel<NN, 1>), dim3(grid), dim3(kNB), 0, c->stream, a);
+#define L_DY3(NN) launch_dct3_n<NN, 1>(c, a);
         FEN_NB_DISPATCH(c->ny, L_DY3)
 #undef L_DY3
     }
