@@ -1193,37 +1193,24 @@ int fen_ns_run(fen_ctx *c, int step0, int nsteps, double *dt)
 
 namespace {
 
-// The whole-array semantics of the reference's solvers that the device
-// solve leaves to the host: the x backward transform writes the interior
-// only, so with ghosts (gl = 1) ppn/npn/nnn leave them 0 (phi%f = 0 first,
-// src/poisson.f90:1151, 1297, 1436) and nn divides them by 2nx with the rest
-// (:594); the mean s is subtracted over the whole array (pp :503, ppn
-// :1171) or the interior (pn :408).
-void poisson_host_fixups(const fen_ctx *c, double *f, size_t n, int gl, bool mean, double s)
+// launch_solve_end for the FP32 form, whose mean is subtracted in FP64 from
+// the FP32 solution: on the host array, row by row (pp, ppn and ppp only).
+void solve_end_fp32(const fen_ctx *c, double *f, int gl, bool mean, double s)
 {
-    const size_t gx = c->nx + 2, gy = c->ny + 2;
-    auto interior = [&](size_t q) {
-        const size_t i = q % gx, j = (q / gx) % gy, k = q / (gx * gy);
-        return i >= 1 && i <= (size_t)c->nx && j >= 1 && j <= (size_t)c->ny && k >= 1 && k <= (size_t)c->nz;
-    };
-    const int sv = c->solver;
-    if (gl && (sv == FEN_SOLVER_PPN || sv == FEN_SOLVER_NPN || sv == FEN_SOLVER_NNN)) {
-        for (size_t q = 0; q < n; q++)
-            if (!interior(q)) f[q] = 0.0;
-    }
-    if (gl && sv == FEN_SOLVER_NN) {
-        const double s2 = (double)(float)(2 * c->nx);
-        for (size_t q = 0; q < n; q++)
-            if (!interior(q)) f[q] = f[q] / s2;
-    }
-    if (mean) {
-        if (sv == FEN_SOLVER_PN) {
-            for (size_t q = 0; q < n; q++)
-                if (!gl || interior(q)) f[q] = f[q] - s;
-        } else {
-            for (size_t q = 0; q < n; q++) f[q] = f[q] - s;
+    const bool zero = gl && c->solver == FEN_SOLVER_PPN;
+    const size_t gx = (size_t)c->nx + 2 * gl, gy = (size_t)c->ny + 2 * gl, gz = (size_t)c->nz + 2 * gl;
+    if (!zero && !mean) return;
+    for (size_t k = 0; k < gz; k++)
+        for (size_t j = 0; j < gy; j++) {
+            double *row = f + (k * gy + j) * gx;
+            if (zero) {
+                const bool edge = k == 0 || k == gz - 1 || j == 0 || j == gy - 1;
+                if (edge) std::fill(row, row + gx, 0.0);
+                else row[0] = row[gx - 1] = 0.0;
+            }
+            if (mean)
+                for (size_t i = 0; i < gx; i++) row[i] = row[i] - s;
         }
-    }
 }
 
 }  // namespace
@@ -1253,12 +1240,15 @@ int fen_poisson_solve(fen_ctx *c, double *f, int gl)
             solve_to_x_spectrum<R>(c, nullptr, as<R>(buf), sx, sy, gl, 1.0, 1.0);
             x_backward<R>(c, as<R>(buf), gl, sx, sy, mean, fen::AxisCopies{});
         });
-        copy_out(c, f, buf, n);
-        if (mean) {
-            FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal + 3, c->d_shift, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            sync(c);
+        if (c->precision == FEN_FP64) {
+            fen::launch_solve_end(c, as<double>(buf), n, gl, mean ? c->d_shift : nullptr);
+            copy_out(c, f, buf, n);
+        } else {
+            if (mean)
+                FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal + 3, c->d_shift, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+            copy_out(c, f, buf, n);
+            solve_end_fp32(c, f, gl, mean, mean ? c->h_scal[3] : 0.0);
         }
-        poisson_host_fixups(c, f, n, gl, mean, mean ? c->h_scal[3] : 0.0);
     });
     return FEN_OK;
 }
@@ -1287,11 +1277,9 @@ int fen_poisson_solve_noalloc(fen_ctx *c, double *f, int gl)
         FEN_HIP_CHECK(hipMemcpyAsync(buf, f, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
         solve_to_x_spectrum<double>(c, nullptr, buf, sx, sy, gl, 1.0, 1.0);
         x_backward<double>(c, buf, gl, sx, sy, mean, fen::AxisCopies{}, part, kNoAllocParts, shift);
+        fen::launch_solve_end(c, buf, n, gl, mean ? shift : nullptr);
         FEN_HIP_CHECK(hipMemcpyAsync(f, buf, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        double s = 0.0;
-        if (mean) FEN_HIP_CHECK(hipMemcpyAsync(&s, shift, sizeof(double), hipMemcpyDeviceToHost, c->stream));
         sync(c);
-        poisson_host_fixups(c, f, n, gl, mean, s);
     });
     return FEN_OK;
 }

@@ -402,6 +402,7 @@ size_t thomas_chunk_c1_count(fen_ctx *c);
 void launch_thomas_chunk_c1(fen_ctx *c);
 void launch_thomas_chunks(fen_ctx *c);
 template <class R> void launch_apply_shift(fen_ctx *c, R *f, size_t n);
+void launch_solve_end(fen_ctx *c, double *f, size_t n, int gl, const double *shift);   // FP64 contexts
 void launch_advection_only(fen_ctx *c, double *rx, double *ry, double *rz);   // FP64 contexts
 
 // One FP64 time step (the step fen_ns_step runs, without the CFL update).

@@ -490,6 +490,39 @@ template <class R> __global__ void apply_shift_kernel(R *f, long n, const double
     if (q < n) f[q] = (R)((double)f[q] - shift[0]);
 }
 
+// What the reference's solvers do to the whole array after the x backward
+// transform (fen_poisson_solve): ghosts zeroed or divided, the mean subtracted
+// from every element or from the interior.  One thread per element; on the
+// host, one pass with a division per element each, this took 6.5 ms of a
+// 128 x 128 x 100 solve's 8.6.
+struct SolveEndArgs {
+    double *f;
+    long n, gx, gxy;
+    int nx, ny, nz, gl;
+    int zero_ghosts;      // ppn, npn, nnn with ghosts
+    double ghost_div;     // nn: ghosts divided by this (0: not)
+    int shift_ghosts;     // the mean is subtracted from ghosts too
+    const double *shift;  // the mean, or null
+};
+__global__ __launch_bounds__(kBlock) void solve_end_kernel(SolveEndArgs a)
+{
+    const long q = (long)blockIdx.x * kBlock + threadIdx.x;
+    if (q >= a.n) return;
+    bool inside = true;
+    if (a.gl) {
+        const int k = (int)(q / a.gxy), r = (int)(q - k * a.gxy), j = r / (int)a.gx, i = r - j * (int)a.gx;
+        inside = i >= 1 && i <= a.nx && j >= 1 && j <= a.ny && k >= 1 && k <= a.nz;
+    }
+    if (inside && !a.shift) return;
+    double v = a.f[q];
+    if (!inside) {
+        if (a.zero_ghosts) v = 0.0;
+        if (a.ghost_div != 0.0) v = v / a.ghost_div;
+    }
+    if (a.shift && (inside || a.shift_ghosts)) v = v - a.shift[0];
+    a.f[q] = v;
+}
+
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
@@ -785,6 +818,30 @@ template <class R> void launch_apply_shift(fen_ctx *c, R *f, size_t n)
     hipLaunchKernelGGL(apply_shift_kernel<R>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, f, (long)n,
                        (const double *)c->d_shift);
     prof_end(c, K_REDUCE, 2.0 * sizeof(R) * n);
+}
+
+// The whole-array semantics of the reference's solvers that the transforms
+// leave out: they write the interior only, so with ghosts (gl = 1) ppn/npn/nnn
+// leave them 0 (phi%f = 0 first, src/poisson.f90:1151, 1297, 1436) and nn
+// divides them by 2nx with the rest (:594); the mean is subtracted over the
+// whole array (pp :503, ppn :1171) or the interior (pn :408).  shift: the
+// mean on the device, or null.
+void launch_solve_end(fen_ctx *c, double *f, size_t n, int gl, const double *shift)
+{
+    SolveEndArgs a{};
+    const int sv = c->solver;
+    a.f = f;
+    a.n = (long)n;
+    a.gx = c->nx + 2;
+    a.gxy = (long)(c->nx + 2) * (c->ny + 2);
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.gl = gl;
+    a.zero_ghosts = gl && (sv == FEN_SOLVER_PPN || sv == FEN_SOLVER_NPN || sv == FEN_SOLVER_NNN);
+    a.ghost_div = gl && sv == FEN_SOLVER_NN ? (double)(float)(2 * c->nx) : 0.0;
+    a.shift_ghosts = sv != FEN_SOLVER_PN;
+    a.shift = shift;
+    if (!shift && !a.zero_ghosts && a.ghost_div == 0.0) return;
+    hipLaunchKernelGGL(solve_end_kernel, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream, a);
+    prof_end(c, K_REDUCE, 16.0 * n);
 }
 
 #define FEN_INSTANTIATE(R)                                                                                     \

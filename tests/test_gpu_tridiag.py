@@ -51,3 +51,23 @@ def test_columns_along_y(solver, ny):
     print("tridiag y", solver, ny, flush=True)
     err = _solve(2, (16, ny, 1), (solver == "nn", 1, 0), 0, ny)
     assert err <= 8 * (ny + 8) * EPS[0], err
+
+
+@pytest.mark.parametrize("solver", ["ppn", "ppp"])
+def test_ghosts_of_an_fp32_solve(solver):
+    """With ghosts: ppn leaves them minus the mean it subtracts, ppp as they
+    came; the interior is the ghostless solve's."""
+    n = (16, 8, 32)
+    bc = [BC_PERIODIC] * 4 + ([BC_WALL] * 2 if solver == "ppn" else [BC_PERIODIC] * 2)
+    rng = np.random.default_rng(3)
+    f = np.asfortranarray(rng.standard_normal(tuple(m + 2 for m in n)))
+    inner = np.asfortranarray(f[1:-1, 1:-1, 1:-1])
+    with Solver(3, n, (2.0, 1.0, 4.0), bc=bc, precision=FP32_REFINE) as g:
+        a, b = g.solve_poisson(f, 1), g.solve_poisson(inner, 0)
+    assert np.array_equal(a[1:-1, 1:-1, 1:-1], b)
+    ghost = np.ones(a.shape, bool)
+    ghost[1:-1, 1:-1, 1:-1] = False
+    if solver == "ppp":
+        assert np.array_equal(a[ghost], f[ghost].astype(np.float32).astype(np.float64))
+    else:
+        assert np.unique(a[ghost]).size == 1
