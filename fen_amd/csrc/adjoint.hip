@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "fen_internal.hpp"
+#include "host_copy.hpp"
 
 namespace fen {
 
@@ -366,7 +367,7 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
     double *ub[3] = {t->work, t->work + n, t->work + 2 * n}, *pb = t->work + 3 * n;
     double *dvo[3] = {t->work + 4 * n, t->work + 5 * n, t->work + 6 * n};
     for (int d = 0; d < 3; d++)
-        FEN_HIP_CHECK(hipMemcpyAsync(ub[d], seed[d], n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        copy_to_device(c->stream, ub[d], seed[d], n, sizeof(double));
     FEN_HIP_CHECK(hipMemsetAsync(pb, 0, 4 * n * sizeof(double), c->stream));   // pb and dvo
     const double dt_o_saved = c->dt_o;
     c->dt_o = t->dt_o;
@@ -380,8 +381,8 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
         for (int s = len - 1; s >= 0; s--) adjoint_step(c, t, t->seg[s], ub, pb, dvo);
     }
     for (int d = 0; d < 3; d++)
-        FEN_HIP_CHECK(hipMemcpyAsync(grad[d], ub[d], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (grad_p) FEN_HIP_CHECK(hipMemcpyAsync(grad_p, pb, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        copy_to_host(c->stream, grad[d], ub[d], n, sizeof(double));
+    if (grad_p) copy_to_host(c->stream, grad_p, pb, n, sizeof(double));
     load_state(c, t->final_state);   // leave the context at the end of the recorded run
     c->dt_o = dt_o_saved;
     c->checks_valid = false;

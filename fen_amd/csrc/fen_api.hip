@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "fen_internal.hpp"
+#include "host_copy.hpp"
 
 using fen::Box;
 using fen::GhostDesc;
@@ -218,33 +219,9 @@ template <class F> void with_type(const fen_ctx *c, F f)
     else f(float{});
 }
 
-// Host FP64 <-> device R copies (FP32: converted through a host buffer, so
-// every value is rounded to nearest once).
-void copy_in(fen_ctx *c, void *dst, const double *src, size_t n)
-{
-    if (c->precision == FEN_FP64) {
-        FEN_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
-        return;
-    }
-    std::vector<float> h(n);
-    for (size_t q = 0; q < n; q++) h[q] = (float)src[q];
-    FEN_HIP_CHECK(hipMemcpyAsync(dst, h.data(), n * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
-}
-
-void copy_out(fen_ctx *c, double *dst, const void *src, size_t n)
-{
-    if (c->precision == FEN_FP64) {
-        FEN_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
-        return;
-    }
-    std::vector<float> h(n);
-    FEN_HIP_CHECK(hipMemcpyAsync(h.data(), src, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
-    for (size_t q = 0; q < n; q++) dst[q] = (double)h[q];
-}
+// Host FP64 <-> device R copies.
+void copy_in(fen_ctx *c, void *dst, const double *src, size_t n) { fen::copy_to_device(c->stream, dst, src, n, elem(c)); }
+void copy_out(fen_ctx *c, double *dst, const void *src, size_t n) { fen::copy_to_host(c->stream, dst, src, n, elem(c)); }
 
 template <typename T> T *dev_alloc(size_t n)
 {
@@ -850,6 +827,7 @@ int fen_create(fen_ctx **out, int dim, int nx, int ny, int nz, double lx, double
         delete c;
         return FEN_ERR_HIP;
     }
+    fen::host_copy_user(+1);
     *out = c;
     return FEN_OK;
 }
@@ -860,6 +838,7 @@ int fen_destroy(fen_ctx *c)
     (void)hipStreamSynchronize(c->stream);
     free_all(c);
     delete c;
+    fen::host_copy_user(-1);
     return FEN_OK;
 }
 
@@ -1293,13 +1272,10 @@ int fen_add_advection(fen_ctx *c, double *rx, double *ry, double *rz)
         double *r[3] = {as<double>(c->d_us[0]), as<double>(c->d_us[1]), as<double>(c->d_us[2])};
         double *h[3] = {rx, ry, rz};
         const int nd = c->dim == 3 ? 3 : 2;
-        for (int d = 0; d < nd; d++)
-            FEN_HIP_CHECK(hipMemcpyAsync(r[d], h[d], c->n_int * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        for (int d = 0; d < nd; d++) copy_in(c, r[d], h[d], c->n_int);
         fen::launch_advection_only(c, r[0], r[1], r[2]);
         fen::prof_end(c, fen::K_MOMENTUM, 0.0);
-        for (int d = 0; d < nd; d++)
-            FEN_HIP_CHECK(hipMemcpyAsync(h[d], r[d], c->n_int * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        sync(c);
+        for (int d = 0; d < nd; d++) copy_out(c, h[d], r[d], c->n_int);
     });
     return FEN_OK;
 }
