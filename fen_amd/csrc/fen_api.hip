@@ -304,7 +304,7 @@ void free_all(fen_ctx *c)
     f(c->d_wallbuf);
     if (c->mf) {
         MFState &m = *c->mf;
-        for (double *q : {m.vof, m.vof1, m.vof2, m.h, m.dd, m.curv, m.nrx, m.nry, m.lx, m.ly, m.rho, m.mu, m.p_hat,
+        for (double *q : {m.vof, m.vof1, m.dd, m.curv, m.nrx, m.nry, m.lx, m.ly, m.rho, m.mu, m.p_hat,
                           m.p_o})
             f(q);
         delete c->mf;
@@ -483,9 +483,8 @@ void advance_mf(fen_ctx *c, double dt)
     using namespace fen;
     c->last_dt = dt;
     c->step_count++;
-    mf_advect_vof(c, dt);          // :82
-    // :85 and p_hat (:88-92), with ghosts; the constant-CFL form extrapolates with dt_o
-    mf_update_fields(c, true, c->constant_cfl ? dt : 0.0);
+    // :82, :85 and p_hat (:88-92); the constant-CFL form extrapolates with dt_o
+    mf_advect_vof(c, dt, true, c->constant_cfl ? dt : 0.0);
     mf_momentum(c, dt);            // predicted_velocity_field with MF (:140-213)
     solve_phi<double>(c, dt, c->d_us);
     // update_pressure with MF: p_o = p before p = p + phi (:553-559)
@@ -908,7 +907,7 @@ int fen_set_multiphase(fen_ctx *c, double rho0, double rho1, double mu0, double 
         m->rhomin = std::fmin(rho0, rho1);   // src/solver.f90:91-92
         m->irhomin = 1.0 / m->rhomin;
         c->mf = m;
-        for (double **q : {&m->vof, &m->vof1, &m->vof2, &m->h, &m->dd, &m->curv, &m->nrx, &m->nry, &m->lx, &m->ly,
+        for (double **q : {&m->vof, &m->vof1, &m->dd, &m->curv, &m->nrx, &m->nry, &m->lx, &m->ly,
                            &m->rho, &m->mu, &m->p_hat, &m->p_o})
             *q = dev_alloc<double>(c->n_ghost);
         c->config_version++;
@@ -922,7 +921,7 @@ int fen_update_material_properties(fen_ctx *c)
     if (!c->mf) return fail(c, FEN_ERR_STATE, "not in two-phase mode");
     FEN_TRY(c, {
         flush_pending(c);
-        fen::mf_update_fields(c, false);
+        fen::mf_update_fields(c);
         sync(c);
     });
     return FEN_OK;

@@ -220,7 +220,7 @@ struct MFState {
     double dt_surf = 0;          // set by set_timestep when sigma > 0 (src/navier_stokes.f90:657)
     bool have_dt_surf = false;
     int x_first = 1;
-    double *vof = nullptr, *vof1 = nullptr, *vof2 = nullptr, *h = nullptr, *dd = nullptr, *curv = nullptr;
+    double *vof = nullptr, *vof1 = nullptr, *dd = nullptr, *curv = nullptr;
     double *nrx = nullptr, *nry = nullptr, *lx = nullptr, *ly = nullptr;
     double *rho = nullptr, *mu = nullptr, *p_hat = nullptr, *p_o = nullptr;
 };
@@ -369,9 +369,10 @@ void reduce_checks(fen_ctx *c);
 // fills the ghosts of u, v and p, and `p_old` (two-phase) receives p before it.
 template <class R> void launch_project(fen_ctx *c, double dt, bool store = true, R *p_old = nullptr);
 bool fused_z_walls(const fen_ctx *c);
-void mf_advect_vof(fen_ctx *c, double dt);
-// p_hat = 2 p - p_o, or with `dt` > 0 (constant CFL) p_o + (dt + dt_o)(p - p_o)/dt_o.
-void mf_update_fields(fen_ctx *c, bool with_phat, double dt = 0.0);
+// fields: rho, mu and p_hat too; p_hat = 2 p - p_o, or with dt_hat > 0 (constant
+// CFL) p_o + (dt_hat + dt_o)(p - p_o)/dt_o.
+void mf_advect_vof(fen_ctx *c, double dt, bool fields = false, double dt_hat = 0.0);
+void mf_update_fields(fen_ctx *c);
 void mf_momentum(fen_ctx *c, double dt);
 void mf_ghost_field(fen_ctx *c, double *f);
 // npn and nnn (FP64) whose state fields keep the standard wall rules: the fused

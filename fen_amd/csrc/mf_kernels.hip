@@ -43,16 +43,40 @@ __device__ __forceinline__ Surf cell_surface(double nx, double ny, double lx, do
     return q;
 }
 
+// The MF fields' ghosts are copies (periodic images, or the neighbour at a
+// Neumann wall; src/volume_of_fluid.f90:54-219, src/multiphase.f90:44-120).
+// Rows (columns) that hold the value of interior row J, ghosts included.
+struct MFCopies {
+    int x, y;   // COPY_PERIODIC or COPY_MIRROR
+};
+
+// Stores n fields' values of cell (i, j) and the ghosts that copy them.
+template <int NF>
+__device__ __forceinline__ void put_copies(const Box &b, const MFCopies &m, int i, int j, double *const (&f)[NF],
+                                           const double (&v)[NF])
+{
+    int id[3], jd[3];
+    const int ni = copy_rows(i, b.nx, m.x, id), nj = copy_rows(j, b.ny, m.y, jd);
+    for (int y = 0; y < nj; y++)
+        for (int x = 0; x < ni; x++) {
+            const long g = b.g(id[x], jd[y], 1);
+#pragma unroll
+            for (int q = 0; q < NF; q++) f[q][g] = v[q];
+        }
+}
+
 struct VofArgs {
+    MFCopies copies;
     Box b;
     double delta, id, id2, beta, dt;
     const double *vof;
-    double *h, *dd, *curv, *nrx, *nry, *lx, *ly;
+    double *dd, *curv, *nrx, *nry, *lx, *ly;
 };
 
 // compute_norm (src/volume_of_fluid.f90:299-383) and the cell loop of
 // get_h_from_vof (:223-295) in one pass: the normalisation needs only the
-// cell's own normal and curvature terms.
+// cell's own normal and curvature terms.  (h itself, the smoothed indicator, is
+// formed by the reference and read by nothing on this path.)
 __global__ __launch_bounds__(kBX *kBY) void vof_reconstruct_kernel(VofArgs a)
 {
     const int i = blockIdx.x * kBX + threadIdx.x % kBX + 1, j = blockIdx.y * kBY + threadIdx.x / kBX + 1;
@@ -82,16 +106,11 @@ __global__ __launch_bounds__(kBX *kBY) void vof_reconstruct_kernel(VofArgs a)
     const double ny = myc / sqrt(mxc * mxc + myc * myc + kSmall);
     const double lx = 0.5 * a.delta * (nxs[3] + nxs[2] - nxs[1] - nxs[0]);   // quadratic reconstruction
     const double ly = 0.5 * a.delta * (nys[1] + nys[2] - nys[0] - nys[3]);
-    a.nrx[g] = nx;
-    a.nry[g] = ny;
-    a.lx[g] = lx;
-    a.ly[g] = ly;
-    a.curv[g] = -(lx + ly) * a.id2;
-
     const double f = V(0, 0);
+    double *const out[6] = {a.nrx, a.nry, a.lx, a.ly, a.curv, a.dd};
+    double val[6] = {nx, ny, lx, ly, -(lx + ly) * a.id2, 0.0};
     if (f <= kCut || f >= (1.0 - kCut)) {
-        a.h[g] = f;
-        a.dd[g] = 0.0;
+        put_copies(a.b, a.copies, i, j, out, val);
         return;
     }
     const Surf q = cell_surface(nx, ny, lx, ly);
@@ -108,31 +127,21 @@ __global__ __launch_bounds__(kBX *kBY) void vof_reconstruct_kernel(VofArgs a)
     const double cc = 1.0 - A * Q;
     const double x1 = (-bb + sqrt(bb * bb - 4.0 * aa * cc)) / (2.0 * aa);   // solve_quadratic (:402-416)
     const double x2 = (-bb - sqrt(bb * bb - 4.0 * aa * cc)) / (2.0 * aa);
-    const double d = log(fmax(x1, x2)) / (2.0 * beta);
-    a.dd[g] = d;
-    a.h[g] = 0.5 * (1.0 + tanh(beta * (surf_p(q, 0.5, 0.5) + d)));
-}
-
-// An_Int and Num_Int (src/volume_of_fluid.f90:636-661)
-__device__ __forceinline__ double an_int(const Surf &q, double beta, double a, double b, double xa, double xb,
-                                         double ya, double yb, double cf, double d0)
-{
-    return 0.5 * (b - a + 1.0 / (cf * beta) * log(cosh(beta * (surf_p(q, xb, yb) + d0)) /
-                                                   cosh(beta * (surf_p(q, xa, ya) + d0))));
-}
-
-__device__ __forceinline__ double num_int(double a, double b, double qrm, double qrp)
-{
-    return 0.5 * (qrm + qrp) * (b - a);
+    val[5] = log(fmax(x1, x2)) / (2.0 * beta);
+    put_copies(a.b, a.copies, i, j, out, val);
 }
 
 struct SweepArgs {
+    MFCopies copies;
     Box b;
     double delta, beta, dt;
-    const double *vof, *dd, *nrx, *nry, *lx, *ly;   // the current reconstruction
-    const double *vel;                              // u (dir 1) or v (dir 2)
-    const double *in;
-    double *out;
+    const double *vof, *dd, *nrx, *nry, *lx, *ly;   // the current reconstruction; vof is swept
+    const double *u, *v;
+    double *out;                                    // first sweep: vof after it; second: the new vof
+    // the second sweep's, if `rho` is set: material properties and p_hat of the new vof
+    double rho0, rho1, mu0, mu1, dt_hat, dt_o;
+    const double *p, *p_o;
+    double *rho, *mu, *p_hat;
 };
 
 // compute_flux (src/volume_of_fluid.f90:548-632): flux through the high face
@@ -155,57 +164,102 @@ template <int DIR> __device__ double face_flux(const SweepArgs &a, int i, int j,
     const double f = a.vof[g];
     if (f <= kCut || f >= (1.0 - kCut)) return (double)sgn * delta * f * (xb - xa) * (yb - ya);
     const Surf q = cell_surface(a.nrx[g], a.nry[g], a.lx[g], a.ly[g]);
-    const double d0 = a.dd[g], rp = gauss_rp(), rm = gauss_rm();
-    if (q.cx == 0.0)
-        return (double)sgn * delta *
-               num_int(ya, yb, an_int(q, beta, xa, xb, xa, xb, rm * (ya + yb), rm * (yb + ya), q.a10, d0),
-                       an_int(q, beta, xa, xb, xa, xb, rp * (ya + yb), rp * (yb + ya), q.a10, d0));
-    return (double)sgn * delta *
-           num_int(xa, xb, an_int(q, beta, ya, yb, rm * (xa + xb), rm * (xa + xb), ya, yb, q.a01, d0),
-                   an_int(q, beta, ya, yb, rp * (xa + xb), rp * (xa + xb), ya, yb, q.a01, d0));
+    const double d0 = a.dd[g];
+    // Num_Int of An_Int at the two Gauss points (src/volume_of_fluid.f90:636-661):
+    // analytic along x (cx = 0) or along y, two points along the other.  One
+    // loop for both directions and points: inlined eight times over, the cosh
+    // made 30 KB of code, fetched cold by every launch.
+    const bool along_x = q.cx == 0.0;
+    const double lo = along_x ? xa : ya, hi = along_x ? xb : yb;         // analytic direction
+    const double ql = along_x ? ya : xa, qh = along_x ? yb : xb;         // the other
+    const double cf = along_x ? q.a10 : q.a01;
+    double sum = 0.0;
+#pragma unroll 1
+    for (int n = 0; n < 2; n++) {
+        const double t = (n == 0 ? gauss_rm() : gauss_rp()) * (ql + qh);
+        double c[2];
+#pragma unroll 1
+        for (int m = 0; m < 2; m++) {
+            const double x = m == 0 ? hi : lo;
+            c[m] = cosh(beta * (surf_p(q, along_x ? x : t, along_x ? t : x) + d0));
+        }
+        sum = sum + 0.5 * (hi - lo + 1.0 / (cf * beta) * log(c[0] / c[1]));
+    }
+    return (double)sgn * delta * (0.5 * sum * (qh - ql));
 }
 
-// One directional sweep of advect_vof (src/volume_of_fluid.f90:437-461).
-template <int DIR> __global__ __launch_bounds__(kBX *kBY) void vof_sweep_kernel(SweepArgs a)
+// rho and mu of a cell (src/multiphase.f90:133-134), and p_hat: 2 p - p_o at
+// fixed dt (src/navier_stokes.f90:91), p_o + (dt + dt_o)(p - p_o)/dt_o with
+// constant CFL (:89; `dt` > 0).
+__device__ __forceinline__ double mix(double f, double a0, double a1) { return a1 * f + a0 * (1.0 - f); }
+__device__ __forceinline__ double p_hat_of(double p, double p_o, double dt, double dt_o)
 {
-    const int i = blockIdx.x * kBX + threadIdx.x % kBX + 1, j = blockIdx.y * kBY + threadIdx.x / kBX + 1;
-    if (i > a.b.nx || j > a.b.ny) return;
-    const long g = a.b.g(i, j, 1), sh = DIR == 1 ? 1 : a.b.gx;
-    const double fp = face_flux<DIR>(a, i, j, a.vel[g]);
-    const double fm = DIR == 1 ? face_flux<1>(a, i - 1, j, a.vel[g - sh]) : face_flux<2>(a, i, j - 1, a.vel[g - sh]);
-    a.out[g] = (a.in[g] - (fp - fm) / a.delta) / (1.0 - a.dt * (a.vel[g] - a.vel[g - sh]) / a.delta);
+    return dt > 0.0 ? p_o + (dt + dt_o) * (p - p_o) / dt_o : 2.0 * p - p_o;
 }
 
-// vof^{n+1} = vof2 - dt (vof_x du + vof_y dv) with the sweep-order weights (:463-470, :509-516).
-__global__ __launch_bounds__(kBX *kBY) void vof_finish_kernel(Box b, double delta, double dt, int x_first,
-                                                                  const double *vof1, const double *vof2,
-                                                                  const double *u, const double *v, double *vof)
+// One directional sweep of advect_vof (src/volume_of_fluid.f90:437-461).  The
+// second one also finishes the advection, vof^{n+1} = vof2 - dt (vof_x du +
+// vof_y dv) with the sweep order's weights (:463-470, :509-516; `vof` is vof1
+// there), and forms rho, mu and p_hat of the new vof.  Every output leaves with
+// its ghosts.  (The finish, the properties, a copy of vof1 and six ghost fills
+// were launches of 4 us each, as long as the sweep of a 128 x 512 grid's cells
+// themselves.)
+//
+// One thread per face of the workgroup's 16 x 16 cells along DIR (17 rows of
+// faces), each formed once and read by the cell beyond it from LDS: a face of a
+// mixed cell is some 800 dependent instructions (eight cosh, four log), and a
+// thread that formed both of its cell's, all inlined, took 11 us a sweep, now 7.4
+// (9 with the finish and the properties).
+constexpr int kFaces = (kBX + 1) * kBY;
+template <int DIR, int SECOND> __global__ __launch_bounds__(kFaces) void vof_sweep_kernel(SweepArgs a)
+{
+    static_assert(kBX == kBY, "square workgroups");
+    __shared__ double flux[kFaces];
+    // face row r (0: the low faces of the first cells) of line l; r is the slow index
+    const int l = threadIdx.x % kBX, r = threadIdx.x / kBX;
+    const int i0 = blockIdx.x * kBX, j0 = blockIdx.y * kBY;
+    const int i = i0 + (DIR == 1 ? r : l + 1), j = j0 + (DIR == 1 ? l + 1 : r);   // the cell whose high face it is
+    const double *vel = DIR == 1 ? a.u : a.v;
+    if (i <= a.b.nx && j <= a.b.ny) flux[threadIdx.x] = face_flux<DIR>(a, i, j, vel[a.b.g(i, j, 1)]);
+    __syncthreads();
+    if (r == 0 || i > a.b.nx || j > a.b.ny) return;
+    const long g = a.b.g(i, j, 1), sh = DIR == 1 ? 1 : a.b.gx;
+    const double fp = flux[threadIdx.x], fm = flux[threadIdx.x - kBX];
+    const double vof1 = a.vof[g];
+    const double swept = (vof1 - (fp - fm) / a.delta) / (1.0 - a.dt * (vel[g] - vel[g - sh]) / a.delta);
+    if constexpr (!SECOND) {
+        double *const out[1] = {a.out};
+        const double val[1] = {swept};
+        put_copies(a.b, a.copies, i, j, out, val);
+    } else {
+        const double du = a.u[g] - a.u[g - 1], dv = a.v[g] - a.v[g - a.b.gx];
+        // the direction swept first weighs with vof1
+        const double vx = DIR == 2 ? vof1 : swept, vy = DIR == 2 ? swept : vof1;
+        const double f = swept - a.dt * (vx * du / a.delta + vy * dv / a.delta);
+        if (a.rho) {
+            double *const out[4] = {a.out, a.rho, a.mu, a.p_hat};
+            const double val[4] = {f, mix(f, a.rho0, a.rho1), mix(f, a.mu0, a.mu1),
+                                   p_hat_of(a.p[g], a.p_o[g], a.dt_hat, a.dt_o)};
+            put_copies(a.b, a.copies, i, j, out, val);
+        } else {
+            double *const out[1] = {a.out};
+            const double val[1] = {f};
+            put_copies(a.b, a.copies, i, j, out, val);
+        }
+    }
+}
+
+// rho and mu of the resident vof, with ghosts.
+__global__ __launch_bounds__(kBX *kBY) void mf_fields_kernel(Box b, MFCopies copies, const double *vof, double rho0,
+                                                             double rho1, double mu0, double mu1, double *rho,
+                                                             double *mu)
 {
     const int i = blockIdx.x * kBX + threadIdx.x % kBX + 1, j = blockIdx.y * kBY + threadIdx.x / kBX + 1;
     if (i > b.nx || j > b.ny) return;
-    const long g = b.g(i, j, 1);
-    const double du = u[g] - u[g - 1], dv = v[g] - v[g - b.gx];
-    if (x_first) vof[g] = vof2[g] - dt * (vof1[g] * du / delta + vof2[g] * dv / delta);
-    else vof[g] = vof2[g] - dt * (vof2[g] * du / delta + vof1[g] * dv / delta);
-}
-
-// rho, mu from the vof over the whole array (src/multiphase.f90:133-134), and
-// p_hat in the same pass: 2 p - p_o at fixed dt (src/navier_stokes.f90:91),
-// p_o + (dt + dt_o)(p - p_o)/dt_o with constant CFL (:89; `dt` > 0).
-__global__ __launch_bounds__(256) void mf_fields_kernel(long n, const double *vof, double rho0, double rho1,
-                                                        double mu0, double mu1, double *rho, double *mu,
-                                                        const double *p, const double *p_o, double *p_hat,
-                                                        double dt, double dt_o)
-{
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q >= n) return;
-    const double f = vof[q];
-    rho[q] = rho1 * f + rho0 * (1.0 - f);
-    mu[q] = mu1 * f + mu0 * (1.0 - f);
-    if (p_hat) {
-        if (dt > 0.0) p_hat[q] = p_o[q] + (dt + dt_o) * (p[q] - p_o[q]) / dt_o;
-        else p_hat[q] = 2.0 * p[q] - p_o[q];
-    }
+    const double f = vof[b.g(i, j, 1)];
+    double *const out[2] = {rho, mu};
+    const double val[2] = {mix(f, rho0, rho1), mix(f, mu0, mu1)};
+    put_copies(b, copies, i, j, out, val);
 }
 
 struct MFMomArgs {
@@ -300,96 +354,89 @@ template <int SRC> __global__ __launch_bounds__(kBX *kBY) void mf_momentum_kerne
 
 dim3 cell_grid(const Box &b) { return dim3((unsigned)((b.nx + kBX - 1) / kBX), (unsigned)((b.ny + kBY - 1) / kBY)); }
 
-// Ghost fill of MF fields: Periodic -> images, Wall -> Neumann (the vof
-// family and rho, mu, p_hat, p_o; src/volume_of_fluid.f90:54-219,
-// src/multiphase.f90:44-120).
-void mf_ghost(fen_ctx *c, double *const *f, int n)
+MFCopies mf_copies(const fen_ctx *c)
 {
-    for (int s = 0; s < n; s += 8) {
-        GhostDesc<double> d[8];
-        const int m = n - s < 8 ? n - s : 8;
-        for (int q = 0; q < m; q++) {
-            d[q] = GhostDesc<double>{};
-            d[q].f = f[s + q];
-            for (int face = 0; face < 6; face++) {
-                d[q].type[face] = (c->dim == 3 || face < 4) ? (c->bc_phys[face] == FEN_BC_PERIODIC ? 0 : 2) : 0;
-                d[q].plane[face] = nullptr;
-            }
-            d[q].loc = 'c';
-            d[q].groups = 3;
-        }
-        launch_ghost_desc<double>(c, d, m);
-    }
+    return MFCopies{c->periodic[0] ? COPY_PERIODIC : COPY_MIRROR, c->periodic[1] ? COPY_PERIODIC : COPY_MIRROR};
 }
 
-void vof_reconstruct(fen_ctx *c)
+void vof_reconstruct(fen_ctx *c, const double *vof)
 {
     MFState &m = *c->mf;
     VofArgs a{};
+    a.copies = mf_copies(c);
     a.b = c->box;
     a.delta = c->delta;
     a.id = 1.0 / c->delta;
     a.id2 = 1.0 / (c->delta * c->delta);
     a.beta = m.beta;
-    a.vof = m.vof;
-    a.h = m.h; a.dd = m.dd; a.curv = m.curv; a.nrx = m.nrx; a.nry = m.nry; a.lx = m.lx; a.ly = m.ly;
+    a.vof = vof;
+    a.dd = m.dd; a.curv = m.curv; a.nrx = m.nrx; a.nry = m.nry; a.lx = m.lx; a.ly = m.ly;
     hipLaunchKernelGGL(vof_reconstruct_kernel, cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, a);
-    double *f[7] = {m.curv, m.nrx, m.nry, m.lx, m.ly, m.h, m.dd};
-    mf_ghost(c, f, 7);
 }
 
-template <int DIR> void vof_sweep(fen_ctx *c, const double *in, double *out, double dt)
+SweepArgs sweep_args(fen_ctx *c, const double *vof, double *out, double dt)
 {
     MFState &m = *c->mf;
     SweepArgs a{};
+    a.copies = mf_copies(c);
     a.b = c->box;
     a.delta = c->delta;
     a.beta = m.beta;
     a.dt = dt;
-    a.vof = m.vof; a.dd = m.dd; a.nrx = m.nrx; a.nry = m.nry; a.lx = m.lx; a.ly = m.ly;
-    a.vel = as<double>(DIR == 1 ? c->d_u[0] : c->d_u[1]);
-    a.in = in;
+    a.vof = vof; a.dd = m.dd; a.nrx = m.nrx; a.nry = m.nry; a.lx = m.lx; a.ly = m.ly;
+    a.u = as<double>(c->d_u[0]);
+    a.v = as<double>(c->d_u[1]);
     a.out = out;
-    hipLaunchKernelGGL((vof_sweep_kernel<DIR>), cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, a);
+    return a;
+}
+
+template <int DIR, int SECOND> void vof_sweep(fen_ctx *c, const SweepArgs &a)
+{
+    hipLaunchKernelGGL((vof_sweep_kernel<DIR, SECOND>), cell_grid(c->box), dim3(kFaces), 0, c->stream, a);
 }
 
 }  // namespace
 
-void mf_ghost_field(fen_ctx *c, double *f) { mf_ghost(c, &f, 1); }
-
-// advect_vof (src/volume_of_fluid.f90:420-544) with the resident velocity.
-void mf_advect_vof(fen_ctx *c, double dt)
+void mf_ghost_field(fen_ctx *c, double *f)
 {
-    MFState &m = *c->mf;
-    const size_t bytes = c->n_ghost * sizeof(double);
-    vof_reconstruct(c);
-    if (m.x_first) vof_sweep<1>(c, m.vof, m.vof1, dt);
-    else vof_sweep<2>(c, m.vof, m.vof1, dt);
-    // vof = vof1 over the whole array (vof1's ghosts stay zero), then its ghosts
-    FEN_HIP_CHECK(hipMemcpyAsync(m.vof, m.vof1, bytes, hipMemcpyDeviceToDevice, c->stream));
-    double *vf[1] = {m.vof};
-    mf_ghost(c, vf, 1);
-    vof_reconstruct(c);
-    if (m.x_first) vof_sweep<2>(c, m.vof1, m.vof2, dt);
-    else vof_sweep<1>(c, m.vof1, m.vof2, dt);
-    hipLaunchKernelGGL(vof_finish_kernel, cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, c->box, c->delta, dt,
-                       m.x_first, (const double *)m.vof1, (const double *)m.vof2, (const double *)as<double>(c->d_u[0]),
-                       (const double *)as<double>(c->d_u[1]), m.vof);
-    m.x_first = !m.x_first;
-    mf_ghost(c, vf, 1);
+    GhostDesc<double> d{};
+    d.f = f;
+    for (int face = 0; face < 4; face++) d.type[face] = c->bc_phys[face] == FEN_BC_PERIODIC ? 0 : 2;
+    d.loc = 'c';
+    d.groups = 3;
+    launch_ghost_desc<double>(c, &d, 1);
 }
 
-// update_material_properties (and p_hat when `with_phat`).
-void mf_update_fields(fen_ctx *c, bool with_phat, double dt)
+// advect_vof (src/volume_of_fluid.f90:420-544) with the resident velocity;
+// `fields`: also the material properties and p_hat (mf_update_fields).
+void mf_advect_vof(fen_ctx *c, double dt, bool fields, double dt_hat)
 {
     MFState &m = *c->mf;
-    const long n = (long)c->n_ghost;
-    hipLaunchKernelGGL(mf_fields_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, n,
-                       (const double *)m.vof, m.rho0, m.rho1, m.mu0, m.mu1, m.rho, m.mu,
-                       (const double *)as<double>(c->d_p), (const double *)m.p_o, with_phat ? m.p_hat : nullptr,
-                       dt, c->dt_o);
-    double *f[3] = {m.rho, m.mu, m.p_hat};
-    mf_ghost(c, f, with_phat ? 3 : 2);
+    vof_reconstruct(c, m.vof);
+    SweepArgs a = sweep_args(c, m.vof, m.vof1, dt);
+    if (m.x_first) vof_sweep<1, 0>(c, a);
+    else vof_sweep<2, 0>(c, a);
+    vof_reconstruct(c, m.vof1);
+    a = sweep_args(c, m.vof1, m.vof, dt);
+    if (fields) {
+        a.rho0 = m.rho0; a.rho1 = m.rho1; a.mu0 = m.mu0; a.mu1 = m.mu1;
+        a.dt_hat = dt_hat;
+        a.dt_o = c->dt_o;
+        a.p = as<double>(c->d_p);
+        a.p_o = m.p_o;
+        a.rho = m.rho; a.mu = m.mu; a.p_hat = m.p_hat;
+    }
+    if (m.x_first) vof_sweep<2, 1>(c, a);
+    else vof_sweep<1, 1>(c, a);
+    m.x_first = !m.x_first;
+}
+
+// update_material_properties.
+void mf_update_fields(fen_ctx *c)
+{
+    MFState &m = *c->mf;
+    hipLaunchKernelGGL(mf_fields_kernel, cell_grid(c->box), dim3(kBX * kBY), 0, c->stream, c->box, mf_copies(c),
+                       (const double *)m.vof, m.rho0, m.rho1, m.mu0, m.mu1, m.rho, m.mu);
 }
 
 void mf_momentum(fen_ctx *c, double dt)
