@@ -45,19 +45,6 @@ struct AdjDims {
 __device__ __forceinline__ int up(int i, int n) { return i + 1 == n ? 0 : i + 1; }
 __device__ __forceinline__ int dn(int i, int n) { return i == 0 ? n - 1 : i - 1; }
 
-// r = pb + (dt/rho) D ub
-__global__ __launch_bounds__(kAX * kAY) void adj_rhs_kernel(AdjDims d, const double *ub, const double *vb,
-                                                           const double *wb, const double *pb, double *r,
-                                                           double id, double dt_rho)
-{
-    const int i = blockIdx.x * kAX + threadIdx.x % kAX, j = blockIdx.y * kAY + threadIdx.x / kAX, k = blockIdx.z;
-    if (i >= d.nx || j >= d.ny) return;
-    const long q = d.q(i, j, k);
-    const double div = ((ub[q] - ub[d.q(dn(i, d.nx), j, k)]) * id + (vb[q] - vb[d.q(i, dn(j, d.ny), k)]) * id) +
-                       (wb[q] - wb[d.q(i, j, dn(k, d.nz))]) * id;
-    r[q] = pb[q] + dt_rho * div;
-}
-
 struct AdjProjArgs {
     const double *ub, *vb, *wb;   // ub'
     const double *psi;            // rb = S (pb' + (dt/rho) D ub')
@@ -283,10 +270,11 @@ void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, dou
     const double rho = c->density, dt = t->dt;
     const double id = 1.0 / c->delta;
     const double A = 1.0 + 0.5 * dt / t->dt_o, B = -(0.5 * dt / t->dt_o);
-    // r = pb' + (dt/rho) D ub', then r = S r: the adjoint of the solve's right-hand side
-    hipLaunchKernelGGL(adj_rhs_kernel, grid, blk, 0, c->stream, d, ub[0], ub[1], ub[2], pb, r, id, dt / rho);
+    // r = S (pb' + (dt/rho) D ub'): the adjoint of the solve's right-hand side,
+    // formed by the x transform's loads (a pass of its own, written and read
+    // back, took 17 + 10 us at 128^3 against 20)
     const long sx = c->nx, sy = (long)c->nx * c->ny;
-    launch_div_r2c_impl<double>(c, nullptr, r, sx, sy, 0, 1.0, 1.0, 1.0);
+    launch_adj_r2c(c, ub, pb, dt / rho);
     launch_y_fft<double>(c, -1, 1.0);
     launch_z_solve<double>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
     launch_y_fft<double>(c, +1, 1.0);
@@ -327,6 +315,24 @@ void adjoint_free(fen_ctx *c)
     c->tape = nullptr;
 }
 
+// A tape for nseg checkpoints and segments of `every` states that holds the
+// blocks of the context's last one (allocating and freeing them, 50 to 270 MB
+// each at 128^3, took a fifth of a gradient); blocks beyond these counts are
+// given back.
+static AdjointTape *reuse_tape(fen_ctx *c, int nseg, int every)
+{
+    if (!c->tape) c->tape = new AdjointTape();
+    AdjointTape *t = c->tape;
+    auto keep = [](std::vector<double *> &v, size_t n) {
+        for (; v.size() > n; v.pop_back()) (void)hipFree(v.back());
+    };
+    keep(t->ckpt, (size_t)nseg);
+    keep(t->seg, (size_t)every);
+    return t;
+}
+
+bool adjoint_recorded(const fen_ctx *c) { return c->tape && c->tape->nsteps > 0; }
+
 const char *adjoint_unsupported(const fen_ctx *c)
 {
     if (c->precision != FEN_FP64) return "the adjoint is provided for FP64 contexts";
@@ -338,23 +344,25 @@ const char *adjoint_unsupported(const fen_ctx *c)
 
 void adjoint_record(fen_ctx *c, int step0, int nsteps, int every, double dt)
 {
-    adjoint_free(c);
-    AdjointTape *t = new AdjointTape();
-    c->tape = t;
-    t->nsteps = nsteps;
+    const int nseg = (nsteps + every - 1) / every;
+    AdjointTape *t = reuse_tape(c, nseg, every);
+    t->nsteps = 0;   // nothing recorded if this fails
+    auto more = [&](std::vector<double *> &v, size_t n, size_t len) {
+        while (v.size() < n) v.push_back(dalloc(len));
+    };
+    more(t->ckpt, (size_t)nseg, ckpt_len(c));
+    if (!t->final_state) t->final_state = dalloc(ckpt_len(c));
     t->every = every;
     t->step0 = step0;
     t->dt = dt;
     t->dt_o = c->dt_o;
-    const int nseg = (nsteps + every - 1) / every;
-    for (int s = 0; s < nseg; s++) t->ckpt.push_back(dalloc(ckpt_len(c)));
-    t->final_state = dalloc(ckpt_len(c));
     for (int s = 0; s < nsteps; s += every) {
         save_state(c, t->ckpt[s / every]);
         run_fp64(c, std::min(every, nsteps - s), dt);
     }
     save_state(c, t->final_state);
     FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
+    t->nsteps = nsteps;
 }
 
 void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double *grad_p)
@@ -362,8 +370,7 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
     AdjointTape *t = c->tape;
     const size_t n = c->n_int;
     if (!t->work) t->work = dalloc(14 * n);
-    if (t->seg.empty())
-        for (int s = 0; s < t->every; s++) t->seg.push_back(dalloc(3 * c->n_ghost));
+    while ((int)t->seg.size() < std::min(t->every, t->nsteps)) t->seg.push_back(dalloc(3 * c->n_ghost));
     double *ub[3] = {t->work, t->work + n, t->work + 2 * n}, *pb = t->work + 3 * n;
     double *dvo[3] = {t->work + 4 * n, t->work + 5 * n, t->work + 6 * n};
     for (int d = 0; d < 3; d++)

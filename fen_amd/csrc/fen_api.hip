@@ -1406,7 +1406,7 @@ int fen_adjoint_backward(fen_ctx *c, const double *seed_u, const double *seed_v,
                          double *grad_u, double *grad_v, double *grad_w, double *grad_p)
 {
     if (!c || !seed_u || !seed_v || !seed_w || !grad_u || !grad_v || !grad_w) return FEN_ERR_ARG;
-    if (!c->tape) return fail(c, FEN_ERR_STATE, "no recorded run: call fen_adjoint_record first");
+    if (!fen::adjoint_recorded(c)) return fail(c, FEN_ERR_STATE, "no recorded run: call fen_adjoint_record first");
     const double *seed[3] = {seed_u, seed_v, seed_w};
     double *grad[3] = {grad_u, grad_v, grad_w};
     FEN_TRY(c, {

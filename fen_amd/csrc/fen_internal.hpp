@@ -341,6 +341,8 @@ template <class R> void launch_momentum(fen_ctx *c, double dt, double A, double 
 template <class R>
 void launch_div_r2c_impl(fen_ctx *c, const R *const *vel, const R *direct_src, long sx, long sy, int gl, double rho,
                          double dt, double post);
+// x r2c of p + scale div(vel) (interior arrays, triply periodic, FP64).
+void launch_adj_r2c(fen_ctx *c, const double *const *vel, const double *p, double scale);
 template <class R> void launch_y_fft(fen_ctx *c, int sign, double post_scale);
 template <class R> void launch_y_solve_2d(fen_ctx *c, double inv_n);
 template <class R> void launch_z_solve(fen_ctx *c, double inv_n);
@@ -428,6 +430,7 @@ const char *adjoint_unsupported(const fen_ctx *c);   // nullptr when the context
 void adjoint_record(fen_ctx *c, int step0, int nsteps, int every, double dt);
 void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double *grad_p);
 void adjoint_free(fen_ctx *c);
+bool adjoint_recorded(const fen_ctx *c);
 
 // Profiling helpers.
 void prof_begin(fen_ctx *c, int k);

@@ -34,8 +34,13 @@ template <class R> struct DivR2CArgs {
     long sx, sy;
     int gl;
     int ny_shift;   // log2(ny)
+    const R *p;     // DIRECT == 2: the other term, and the divergence's factor
+    double scale;
 };
 
+// DIRECT: 0 div(u*) rho / dt of the ghosted velocity, 1 `u` itself, 2 (FP64)
+// p + scale div(u, v, w) of interior arrays, periodic in every direction (the
+// discrete adjoint's right-hand side).
 template <class R, int D3, int N, int DIRECT, int NT = kBlock>
 __global__ __launch_bounds__(NT) void div_r2c_kernel(DivR2CArgs<R> a)
 {
@@ -60,7 +65,16 @@ __global__ __launch_bounds__(NT) void div_r2c_kernel(DivR2CArgs<R> a)
         for (int q = 0; q < 8; q++) {
             const int i = t + q * (N / 8) + 1;
             double val;
-            if constexpr (DIRECT) {
+            if constexpr (DIRECT == 2) {
+                const long row = (long)N * ((j - 1) + (long)a.b.ny * (k - 1));
+                const long rowj = (long)N * ((j == 1 ? a.b.ny - 1 : j - 2) + (long)a.b.ny * (k - 1));
+                const long rowk = (long)N * ((j - 1) + (long)a.b.ny * (k == 1 ? a.b.nz - 1 : k - 2));
+                const int x = i - 1, xm = i == 1 ? N - 1 : i - 2;
+                const double d = (((double)a.u[row + x] - (double)a.u[row + xm]) * a.id +
+                                  ((double)a.v[row + x] - (double)a.v[rowj + x]) * a.id) +
+                                 ((double)a.w[row + x] - (double)a.w[rowk + x]) * a.id;
+                val = (double)a.p[row + x] + a.scale * d;
+            } else if constexpr (DIRECT) {
                 val = a.u[(i - 1 + a.gl) + a.sx * (j - 1 + a.gl) + a.sy * (k - 1 + a.gl)];
             } else {
                 const long g = a.b.g(i, j, k);
@@ -624,6 +638,29 @@ void launch_div_r2c_impl(fen_ctx *c, const R *const *vel, const R *direct_src, l
     FEN_DISPATCH_N(c->nx, L_DIV)
 #undef L_DIV
     prof_end(c, K_DIV_R2C, bytes);
+}
+
+void launch_adj_r2c(fen_ctx *c, const double *const *vel, const double *p, double scale)
+{
+    DivR2CArgs<double> a{};
+    a.u = vel[0]; a.v = vel[1]; a.w = vel[2];
+    a.p = p;
+    a.scale = scale;
+    a.spec = as<double2>(c->d_spec);
+    a.tw = as<double2>(c->d_twx);
+    a.b = c->box;
+    a.id = 1.0 / c->delta;
+    a.post = 1.0;
+    a.nrows = (long)c->ny * c->nz;
+    a.kxs = a.nrows;
+    a.ny_shift = ilog2(c->ny);
+    const int nt = x_pass_threads(c), tj = 2 * (nt / (c->nx / 8));
+    const dim3 grid((unsigned)((a.nrows + tj - 1) / tj));
+    prof_begin(c, K_DIV_R2C);
+#define L_ADJ(NN) launch_div_r2c_n<double, 1, NN, 2>(c, grid, nt, a);
+    FEN_DISPATCH_N(c->nx, L_ADJ)
+#undef L_ADJ
+    prof_end(c, K_DIV_R2C, 4.0 * sizeof(double) * c->n_int + spec_bytes<double>(c));
 }
 
 template <class R> void launch_y_fft(fen_ctx *c, int sign, double post)
