@@ -274,10 +274,15 @@ void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, dou
     // formed by the x transform's loads (a pass of its own, written and read
     // back, took 17 + 10 us at 128^3 against 20)
     const long sx = c->nx, sy = (long)c->nx * c->ny;
-    launch_adj_r2c(c, ub, pb, dt / rho);
-    launch_y_fft<double>(c, -1, 1.0);
+    const bool plane = plane_pass(c);
+    if (plane) {
+        launch_plane_adj(c, ub, pb, dt / rho);
+    } else {
+        launch_adj_r2c(c, ub, pb, dt / rho);
+        launch_y_fft<double>(c, -1, 1.0);
+    }
     launch_z_solve<double>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
-    launch_y_fft<double>(c, +1, 1.0);
+    if (!plane) launch_y_fft<double>(c, +1, 1.0);
     launch_c2r<double>(c, r, 0, sx, sy, false, AxisCopies{});
     AdjProjArgs pa{};
     pa.ub = ub[0]; pa.vb = ub[1]; pa.wb = ub[2];

@@ -333,7 +333,8 @@ bool x_cosine(const fen_ctx *c)
 // The Poisson solve up to the x backward transform: the x transform of
 // div(u*) rho/dt (vel) or of `direct` (strides sx, sy, ghost level gl), the
 // scalings of the reference solver, and the solve in the other directions.
-// Leaves phi's x spectrum in the spectrum buffer.
+// Leaves phi's x spectrum in the spectrum buffer (plane_pass grids: the x, y
+// spectrum, which their x backward pass takes).
 template <class R>
 void solve_to_x_spectrum(fen_ctx *c, const R *const *vel, const R *direct, long sx, long sy, int gl, double rho,
                          double dt)
@@ -342,17 +343,21 @@ void solve_to_x_spectrum(fen_ctx *c, const R *const *vel, const R *direct, long 
     const double nx = (double)c->nx, ny = (double)c->ny;
     switch (c->solver) {
     case FEN_SOLVER_PPP:
-        launch_div_r2c_impl<R>(c, vel, direct, sx, sy, gl, rho, dt, 1.0);
-        launch_y_fft<R>(c, -1, 1.0);
-        launch_z_solve<R>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
-        launch_y_fft<R>(c, +1, 1.0);
+    case FEN_SOLVER_PPN: {
+        const bool ppn = c->solver == FEN_SOLVER_PPN;
+        const double px = ppn ? 1.0 / nx : 1.0, py = ppn ? 1.0 / ny : 1.0;
+        const bool plane = plane_pass(c);   // x and y in one pass each way
+        if (plane) {
+            launch_plane_fwd<R>(c, vel, direct, sx, sy, gl, rho, dt, px, py);
+        } else {
+            launch_div_r2c_impl<R>(c, vel, direct, sx, sy, gl, rho, dt, px);
+            launch_y_fft<R>(c, -1, py);
+        }
+        if (ppn) launch_thomas<R>(c);
+        else launch_z_solve<R>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
+        if (!plane) launch_y_fft<R>(c, +1, 1.0);
         return;
-    case FEN_SOLVER_PPN:
-        launch_div_r2c_impl<R>(c, vel, direct, sx, sy, gl, rho, dt, 1.0 / nx);
-        launch_y_fft<R>(c, -1, 1.0 / ny);
-        launch_thomas<R>(c);
-        launch_y_fft<R>(c, +1, 1.0);
-        return;
+    }
     case FEN_SOLVER_PP:
         launch_div_r2c_impl<R>(c, vel, direct, sx, sy, gl, rho, dt, 1.0);
         launch_y_solve_2d<R>(c, 1.0 / (double)(float)((long)c->nx * c->ny));

@@ -155,6 +155,11 @@ __device__ __forceinline__ void put_ghosted(const GhostDesc<R> &d, const Box &b,
 // Neumann faces, or not at all.
 enum { COPY_NONE = 0, COPY_PERIODIC = 1, COPY_MIRROR = 2 };
 
+struct AxisCopies {
+    int x = COPY_NONE, y = COPY_NONE, z = COPY_NONE;
+    __host__ __device__ bool any() const { return x || y || z; }
+};
+
 // The ghosted indices that hold row index J (interior 1..n) of such an axis:
 // J itself, and the ghost rows 0 and n + 1 that copy it.  Returns how many.
 __device__ __forceinline__ int copy_rows(int J, int n, int mode, int (&d)[3])
@@ -343,6 +348,17 @@ void launch_div_r2c_impl(fen_ctx *c, const R *const *vel, const R *direct_src, l
                          double dt, double post);
 // x r2c of p + scale div(vel) (interior arrays, triply periodic, FP64).
 void launch_adj_r2c(fen_ctx *c, const double *const *vel, const double *p, double scale);
+// x and y transforms of whole z planes in LDS (plane_kernels.hip): the grids
+// that take them, the forward passes (launch_div_r2c_impl / launch_adj_r2c and
+// the y transform), and the backward one (part: block sums of the mean, one per
+// plane, or null).
+bool plane_pass(const fen_ctx *c);
+template <class R>
+void launch_plane_fwd(fen_ctx *c, const R *const *vel, const R *direct, long sx, long sy, int gl, double rho, double dt,
+                      double postx, double posty);
+void launch_plane_adj(fen_ctx *c, const double *const *vel, const double *p, double scale);
+template <class R>
+void launch_plane_bwd(fen_ctx *c, R *phi, int gl, long sx, long sy, AxisCopies copies, double *part);
 template <class R> void launch_y_fft(fen_ctx *c, int sign, double post_scale);
 template <class R> void launch_y_solve_2d(fen_ctx *c, double inv_n);
 template <class R> void launch_z_solve(fen_ctx *c, double inv_n);
@@ -354,10 +370,6 @@ long c2r_blocks(const fen_ctx *c);
 // defer: leave the block sums unreduced (shift_parts) when there are at most
 // kDeferParts of them, for a 2-D projection that adds them itself.
 constexpr int kDeferParts = 256;
-struct AxisCopies {
-    int x = COPY_NONE, y = COPY_NONE, z = COPY_NONE;
-    __host__ __device__ bool any() const { return x || y || z; }
-};
 template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long sy, bool want_sum, AxisCopies copies,
                                    double *part = nullptr, size_t n_part = 0, double *shift = nullptr,
                                    bool defer = false);

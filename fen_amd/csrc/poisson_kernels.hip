@@ -792,6 +792,7 @@ template <class R, int N> static void launch_c2r_n(const fen_ctx *c, long nblk, 
 
 long c2r_blocks(const fen_ctx *c)
 {
+    if (plane_pass(c)) return c->nz;
     const int tj = 2 * (x_pass_threads(c) / (c->nx / 8));
     return ((long)c->ny * c->nz + tj - 1) / tj;
 }
@@ -831,11 +832,15 @@ template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long
     a.copies = copies;
     const long nblk = c2r_blocks(c);
     if (want_sum && (size_t)nblk > n_part) throw std::runtime_error("partial-sum buffer too small");
-    prof_begin(c, K_C2R);
+    if (plane_pass(c)) {
+        launch_plane_bwd<R>(c, phi, gl_out, sx, sy, copies, want_sum ? part : nullptr);
+    } else {
+        prof_begin(c, K_C2R);
 #define L_C(NN) launch_c2r_n<R, NN>(c, nblk, a);
-    FEN_DISPATCH_N(c->nx, L_C)
+        FEN_DISPATCH_N(c->nx, L_C)
 #undef L_C
-    prof_end(c, K_C2R, spec_bytes<R>(c) + sizeof(R) * c->n_int);
+        prof_end(c, K_C2R, spec_bytes<R>(c) + sizeof(R) * c->n_int);
+    }
     if (want_sum) {
         if (defer && nblk <= kDeferParts) c->shift_parts = nblk;
         else launch_mean_shift(c, part, nblk, shift);
