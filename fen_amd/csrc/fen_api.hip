@@ -298,7 +298,7 @@ void free_all(fen_ctx *c)
     for (int d = 0; d < 3; d++) { f(c->d_u[d]); f(c->d_us[d]); f(c->d_dvo[d]); f(c->d_S[d]); }
     f(c->d_p); f(c->d_p2); f(c->d_phi); f(c->d_spec); f(c->d_c1); f(c->d_dd);
     f(c->d_mwx); f(c->d_mwy); f(c->d_mwz); f(c->d_ta); f(c->d_tb); f(c->d_tc);
-    f(c->d_twx); f(c->d_twy); f(c->d_twz); f(c->d_spec2); f(c->d_mkx); f(c->d_mky); f(c->d_part); f(c->d_chk); f(c->d_scal);
+    f(c->d_twx); f(c->d_twy); f(c->d_twz); f(c->d_spec2); f(c->d_mkx); f(c->d_mky); f(c->d_part); f(c->d_chk); f(c->d_shift);
     for (int s = 0; s < 5; s++) for (int p = 0; p < 6; p++) f(c->d_plane[s][p]);
     f(c->d_plane_tab);
     f(c->d_wallbuf);
@@ -562,7 +562,7 @@ void flush_pending(fen_ctx *c)
 }
 
 // The checks of a pending step (max div and max |u|+|v|+|w| of its projected
-// velocity) into d_scal, without forming the state.
+// velocity) into d_chk, without forming the state.
 void pending_checks(fen_ctx *c)
 {
     if (!c->pending || c->pending_checked) return;
@@ -822,8 +822,7 @@ int fen_create(fen_ctx **out, int dim, int nx, int ny, int nz, double lx, double
         c->d_part = dev_alloc<double>(c->n_part);
         c->n_chk = std::max<size_t>(3 * 1024, 3 * (size_t)fen::stencil_blocks(c->box));
         c->d_chk = dev_alloc<double>(c->n_chk);
-        c->d_scal = dev_alloc<double>(8);
-        c->d_shift = c->d_scal + 3;
+        c->d_shift = dev_alloc<double>(1);
         FEN_HIP_CHECK(hipHostMalloc((void **)&c->h_scal, 8 * sizeof(double)));
         FEN_HIP_CHECK(hipDeviceSynchronize());
     } catch (const std::exception &) {
@@ -980,9 +979,7 @@ int fen_get_scalars(fen_ctx *c, double *maxdiv, double *maxcfl, double *dt_o, do
             if (maxcfl) *maxcfl = 0.0;
         } else if (maxdiv || maxcfl) {
             pending_checks(c);
-            fen::reduce_checks(c);
-            FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal, c->d_scal, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            sync(c);
+            fen::read_checks(c);
             if (maxdiv) *maxdiv = c->h_scal[0];
             if (maxcfl) *maxcfl = c->last_dt * c->h_scal[1] / c->delta;    // src/navier_stokes.f90:617
             if (c->h_scal[2] != 0.0) return fail(c, FEN_ERR_NONFINITE, "non-finite velocity or divergence");
@@ -1139,9 +1136,7 @@ int fen_ns_step(fen_ctx *c, int step, double *dt, double *maxdiv, double *maxcfl
                     fen::launch_checks<R>(c, vn);
                 });
             }
-            fen::reduce_checks(c);
-            FEN_HIP_CHECK(hipMemcpyAsync(c->h_scal, c->d_scal, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            sync(c);
+            fen::read_checks(c);
             c->dt_o = *dt;
             const double mv = c->h_scal[1];
             c->dt_conv = mv > 0.0 ? c->cfl * c->delta / mv : 1.0;

@@ -286,12 +286,12 @@ struct fen_ctx {
     // reductions
     double *d_part = nullptr;    // per-block sums of the mean
     double *d_chk = nullptr;     // per-block maxima of the checks
-    long chk_blocks = 0;         // > 0: that many entries of d_chk not yet reduced to d_scal (reduce_checks)
+    long chk_blocks = 0;         // > 0: that many entries of d_chk not yet read (read_checks)
     size_t n_chk = 0;
     double *d_noalloc = nullptr; // device address of the allocation-free entry point's scratch (this device)
     size_t n_part = 0;
-    double *d_scal = nullptr;    // [0] maxdiv [1] max|u|+|v|+|w| [2] nonfinite flag [3] mean shift
-    double *h_scal = nullptr;    // pinned mirror
+    // pinned: [0] maxdiv [1] max|u|+|v|+|w| [2] nonfinite flag (read_checks) [3] copy of the mean shift
+    double *h_scal = nullptr;
     double last_dt = 0.0;        // dt of the last step (for maxCFL)
     bool checks_valid = false;
 
@@ -303,7 +303,7 @@ struct fen_ctx {
     // second pressure array d_p2 swap roles with d_us and d_p after every
     // fused step, so a pending state always sits in the same places.
     bool pending = false;
-    bool pending_checked = false;   // d_scal holds the checks of the pending step
+    bool pending_checked = false;   // d_chk or h_scal holds the checks of the pending step
     double pend_dt = 0.0;           // dt of the pending step
 
     hipStream_t stream = nullptr;
@@ -375,11 +375,11 @@ template <class R> void launch_c2r(fen_ctx *c, R *phi, int gl_out, long sx, long
                                    bool defer = false);
 // The pending mean of phi from its block sums, if a 2-D step left it unreduced.
 void reduce_shift(fen_ctx *c);
-// The last checks' maxima into d_scal, if they are still per block.
-void reduce_checks(fen_ctx *c);
+// The last checks' maxima into h_scal (waits), if they are not there already.
+void read_checks(fen_ctx *c);
 // store == false: the checks of the projection only (max div, max |u|+|v|+|w|
 // of the projected velocity), nothing written but the reduction (3-D).
-// The checks stay in d_chk until reduce_checks.  In 2-D the projection also
+// The checks stay in d_chk until read_checks.  In 2-D the projection also
 // fills the ghosts of u, v and p, and `p_old` (two-phase) receives p before it.
 template <class R> void launch_project(fen_ctx *c, double dt, bool store = true, R *p_old = nullptr);
 bool fused_z_walls(const fen_ctx *c);

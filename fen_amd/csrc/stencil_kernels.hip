@@ -418,14 +418,15 @@ __global__ __launch_bounds__(kThreads) void project_kernel_2d(ProjArgs<R> a, Pro
     block_max3<kThreads>(md, mv, bad, a.part, (long)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
-// One workgroup reduces the per-workgroup partials.  Each thread issues the
-// loads of B entries before comparing any, so the pass costs about one
-// memory latency per B entries instead of one per entry.
+// One workgroup reduces the per-workgroup partials and leaves the maxima in
+// out, pinned host memory: a reader waits for this kernel instead of queueing
+// a copy behind it.  Each thread issues the loads of B entries before comparing
+// any, so the pass costs about one memory latency per B entries instead of one
+// per entry.
 constexpr int kFinalThreads = 1024;
 __global__ __launch_bounds__(kFinalThreads) void checks_final_kernel(const double *part, long n, double *out)
 {
     constexpr int NT = kFinalThreads, B = 4;
-    __shared__ double sd[NT], sv[NT], sf[NT];
     double md = -HUGE_VAL, mv = 0.0, bad = 0.0;
     for (long q0 = threadIdx.x; q0 < n; q0 += (long)NT * B) {
         double x[B][3];
@@ -445,17 +446,7 @@ __global__ __launch_bounds__(kFinalThreads) void checks_final_kernel(const doubl
             if (x[m][2] > bad) bad = x[m][2];
         }
     }
-    sd[threadIdx.x] = md; sv[threadIdx.x] = mv; sf[threadIdx.x] = bad;
-    __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            if (sd[threadIdx.x + s] > sd[threadIdx.x]) sd[threadIdx.x] = sd[threadIdx.x + s];
-            if (sv[threadIdx.x + s] > sv[threadIdx.x]) sv[threadIdx.x] = sv[threadIdx.x + s];
-            if (sf[threadIdx.x + s] > sf[threadIdx.x]) sf[threadIdx.x] = sf[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) { out[0] = sd[0]; out[1] = sv[0]; out[2] = sf[0]; }
+    block_max3<NT>(md, mv, bad, out, 0);
 }
 
 // Step n's projection and pressure update fused with step n+1's momentum in
@@ -603,13 +594,15 @@ void launch_step_2d(fen_ctx *c, double dt_p, double dt_m, double A, double B, vo
     prof_end(c, K_PROJ_MOM, (c->has_source ? 13.0 : 11.0) * sizeof(R) * c->n_int);
 }
 
-void reduce_checks(fen_ctx *c)
+void read_checks(fen_ctx *c)
 {
     if (c->chk_blocks <= 0) return;
     prof_begin(c, K_REDUCE);
     hipLaunchKernelGGL(checks_final_kernel, dim3(1), dim3(kFinalThreads), 0, c->stream, (const double *)c->d_chk,
-                       c->chk_blocks, c->d_scal);
+                       c->chk_blocks, c->h_scal);
     prof_end(c, K_REDUCE, 24.0 * c->chk_blocks);
+    FEN_HIP_CHECK(hipGetLastError());
+    FEN_HIP_CHECK(hipStreamSynchronize(c->stream));
     c->chk_blocks = 0;
 }
 
