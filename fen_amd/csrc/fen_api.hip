@@ -457,7 +457,26 @@ template <class R> void finish_step(fen_ctx *c, double dt, R *p_old = nullptr)
     c->checks_valid = true;
 }
 
-// K1 of a step: momentum into u*, v*, w* and their ghosts.
+// The ghosts of u*, v*, w* on the faces each is normal to (and the face values
+// a Dirichlet condition replaces), where the momentum did not write them as
+// images.  The divergence and the projection read no others (every face of all
+// three took 11.0 us at 128 x 256 x 101 npn, these 7.9).
+template <class R> void fill_normal_ghosts(fen_ctx *c)
+{
+    using namespace fen;
+    const int rest = remaining_groups(c, c->img_vel);
+    if (!rest) return;
+    GhostDesc<R> g[3];
+    int n = 0;
+    for (int d = 0; d < c->dim; d++) {
+        if (!(rest & (1 << d))) continue;
+        g[n] = make_desc<R>(c, FEN_U + d, c->d_us[d]);
+        g[n++].groups = 1 << d;
+    }
+    launch_ghost_desc<R>(c, g, n);
+}
+
+// K1 of a step: momentum into u*, v*, w* and the ghosts that the step reads.
 template <class R> void predict(fen_ctx *c, double dt)
 {
     using namespace fen;
@@ -466,12 +485,7 @@ template <class R> void predict(fen_ctx *c, double dt)
     c->last_dt = dt;
     c->step_count++;
     launch_momentum<R>(c, dt, A, B);
-    if (const int rest = remaining_groups(c, c->img_vel)) {
-        GhostDesc<R> g[3] = {make_desc<R>(c, FEN_U, c->d_us[0]), make_desc<R>(c, FEN_V, c->d_us[1]),
-                             make_desc<R>(c, FEN_W, c->d_us[2])};
-        for (auto &d : g) d.groups = rest;
-        launch_ghost_desc<R>(c, g, c->dim == 3 ? 3 : 2);
-    }
+    fill_normal_ghosts<R>(c);
 }
 
 // One time step; see the kernel sequence at the top of this file.
@@ -535,13 +549,7 @@ template <class R> void step_pending(fen_ctx *c, double dt, void *const *save = 
         for (int d = 0; d < 3; d++) std::swap(c->d_u[d], c->d_us[d]);
         std::swap(c->d_p, c->d_p2);
         c->config_version++;   // a captured step graph holds the old array roles
-        // ghosts of u*, v*, w* the momentum did not write as images (walls)
-        if (const int fill = remaining_groups(c, c->img_vel)) {
-            GhostDesc<R> g[3] = {make_desc<R>(c, FEN_U, c->d_us[0]), make_desc<R>(c, FEN_V, c->d_us[1]),
-                                 make_desc<R>(c, FEN_W, c->d_us[2])};
-            for (auto &d : g) d.groups = fill;
-            launch_ghost_desc<R>(c, g, 3);
-        }
+        fill_normal_ghosts<R>(c);
     }
     solve_phi<R>(c, dt, c->d_us);
     c->pending = true;

@@ -193,7 +193,7 @@ void launch_project_momentum(fen_ctx *c, double dt_p, double dt_m, double A, dou
     if (general) {
         // the state at the wall positions, read by the march below
         const long nw = pm_wall_layout(c->box).per_field;
-        hipLaunchKernelGGL(wall_state_kernel<R>, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, c->stream, a);
+        hipLaunchKernelGGL(wall_state_kernel<R>, dim3((unsigned)((nw + 255) / 256), 4), dim3(256), 0, c->stream, a);
     }
     if (save) {
         if (!std::is_same<R, double>::value) throw std::runtime_error("state saving is FP64");

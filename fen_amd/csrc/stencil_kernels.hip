@@ -39,90 +39,32 @@ template <class R> struct GhostLaunch {
     int ngx[kGhostFields], ngy[kGhostFields], ngz[kGhostFields];   // planes per group and field (0: skipped)
 };
 
-template <class R> __device__ __forceinline__ R ghost_s1(const GhostDesc<R> &d, const Box &b, int i, int j, int k)
+// The rules as one chain: the interior cell they start from (x, y and z apart),
+// then what each axis makes of its value.  Straight-line code: as nested calls,
+// inlined at each of their uses for each field, the kernel spent most of its
+// time fetching instructions (u*, v*, w* at 128 x 128 x 160: 7.4 us; as one
+// chain and on their normal faces only, 5.3).
+template <class R> __device__ __forceinline__ R ghost_value(const GhostDesc<R> &d, const Box &b, int i, int j, int k)
 {
     const R two = R(2.0);
-    const long pj = j + (long)(b.ny + 2) * k;
-    if (i == 0) {
-        const int t = d.type[0];
-        if (t == 0) return d.f[b.g(b.nx, j, k)];
-        if (t == 1) {
-            const R bc = d.plane[0][pj];
-            return d.loc == 'x' ? bc : two * bc - d.f[b.g(1, j, k)];
-        }
-        if (t == 2) return d.f[b.g(1, j, k)];
-        return d.f[b.g(i, j, k)];
-    }
-    if (i == b.nx + 1) {
-        const int t = d.type[1];
-        if (t == 0) return d.f[b.g(1, j, k)];
-        if (t == 1) {
-            const R bc = d.plane[1][pj];
-            return d.loc == 'x' ? bc : two * bc - d.f[b.g(b.nx, j, k)];
-        }
-        if (t == 2) return d.f[b.g(b.nx, j, k)];
-        return d.f[b.g(i, j, k)];
-    }
-    if (i == b.nx && d.type[1] == 1 && d.loc == 'x') return d.plane[1][pj];
-    return d.f[b.g(i, j, k)];
-}
-
-template <class R> __device__ __forceinline__ R ghost_s2(const GhostDesc<R> &d, const Box &b, int i, int j, int k)
-{
-    const R two = R(2.0);
-    const long pi = i + (long)(b.nx + 2) * k;
-    if (j == 0) {
-        const int t = d.type[2];
-        if (t == 0) return ghost_s1(d, b, i, b.ny, k);
-        if (t == 1) {
-            const R bc = d.plane[2][pi];
-            return d.loc == 'y' ? bc : two * bc - ghost_s1(d, b, i, 1, k);
-        }
-        if (t == 2) return ghost_s1(d, b, i, 1, k);
-        return ghost_s1(d, b, i, j, k);
-    }
-    if (j == b.ny + 1) {
-        const int t = d.type[3];
-        if (t == 0) return ghost_s1(d, b, i, 1, k);
-        if (t == 1) {
-            const R bc = d.plane[3][pi];
-            return d.loc == 'y' ? bc : two * bc - ghost_s1(d, b, i, b.ny, k);
-        }
-        if (t == 2) return ghost_s1(d, b, i, b.ny, k);
-        return ghost_s1(d, b, i, j, k);
-    }
-    if (j == b.ny && d.type[3] == 1 && d.loc == 'y') return d.plane[3][pi];
-    return ghost_s1(d, b, i, j, k);
-}
-
-template <class R> __device__ __forceinline__ R ghost_s3(const GhostDesc<R> &d, const Box &b, int i, int j, int k)
-{
-    const R two = R(2.0);
-    if (b.dim == 3) {
-        const long pij = i + (long)(b.nx + 2) * j;
-        if (k == 0) {
-            const int t = d.type[4];
-            if (t == 0) return ghost_s2(d, b, i, j, b.nz);
-            if (t == 1) {
-                const R bc = d.plane[4][pij];
-                return d.loc == 'z' ? bc : two * bc - ghost_s2(d, b, i, j, 1);
-            }
-            if (t == 2) return ghost_s2(d, b, i, j, 1);
-            return ghost_s2(d, b, i, j, k);
-        }
-        if (k == b.nz + 1) {
-            const int t = d.type[5];
-            if (t == 0) return ghost_s2(d, b, i, j, 1);
-            if (t == 1) {
-                const R bc = d.plane[5][pij];
-                return d.loc == 'z' ? bc : two * bc - ghost_s2(d, b, i, j, b.nz);
-            }
-            if (t == 2) return ghost_s2(d, b, i, j, b.nz);
-            return ghost_s2(d, b, i, j, k);
-        }
-        if (k == b.nz && d.type[5] == 1 && d.loc == 'z') return d.plane[5][pij];
-    }
-    return ghost_s2(d, b, i, j, k);
+    auto from = [](int g, int n, int lo, int hi) {
+        return g == 0 ? (lo == 0 ? n : 1) : (g == n + 1 ? (hi == 0 ? 1 : n) : g);
+    };
+    const bool z = b.dim == 3;
+    const int ix = from(i, b.nx, d.type[0], d.type[1]), jy = from(j, b.ny, d.type[2], d.type[3]);
+    const int kz = z ? from(k, b.nz, d.type[4], d.type[5]) : k;
+    R v = d.f[b.g(ix, jy, kz)];
+    auto rule = [&](int g, int n, int face, char loc, long at) {
+        const bool normal = d.loc == loc;
+        const int t = g == 0 ? d.type[face] : (g == n + 1 || (g == n && normal) ? d.type[face + 1] : 0);
+        if (t != 1) return;
+        const R bc = g == 0 ? d.plane[face][at] : d.plane[face + 1][at];
+        v = normal ? bc : two * bc - v;
+    };
+    rule(i, b.nx, 0, 'x', jy + (long)(b.ny + 2) * kz);
+    rule(j, b.ny, 2, 'y', i + (long)(b.nx + 2) * kz);
+    if (z) rule(k, b.nz, 4, 'z', i + (long)(b.nx + 2) * j);
+    return v;
 }
 
 // Group plane index p -> coordinate: 0 -> 0, 1 -> n+1, 2 -> n (normal overwrite).
@@ -163,7 +105,7 @@ template <class R, int Q> __device__ __forceinline__ void ghost_field(const Ghos
     } else {
         return;
     }
-    d.f[b.g(i, j, k)] = ghost_s3(d, b, i, j, k);
+    d.f[b.g(i, j, k)] = ghost_value(d, b, i, j, k);
 }
 
 template <class R> __global__ __launch_bounds__(256) void ghost_kernel(GhostLaunch<R> a)

@@ -905,46 +905,53 @@ __global__ __launch_bounds__(TX *TY / NJ, OCC) void project_momentum_kernel(PMAr
 }
 
 // The general-wall form's face buffer: u, v, w, p of step n at every wall
-// position (pm_wall_layout), one thread per position.  Each is the
-// projection of the interior cell the ghost fill reads (commit()'s
+// position (pm_wall_layout), one thread per position and field (blockIdx.y).
+// Each is the projection of the interior cell the ghost fill reads (commit()'s
 // arithmetic, so interior positions such as the overwritten face n match
 // the march's own values bit for bit), then the ghost fill's rule chain.
+// Latency bounds it, and the fetch of its code: one field per thread is a
+// third of the code of four (128 x 128 x 160 nnn: 11.7 -> 9.6 us; 128 x 256 x
+// 101 npn, where the x faces' rows, a line per value, weigh more: 11.5 -> 11.8).
 template <class R>
 __global__ __launch_bounds__(256) void wall_state_kernel(PMArgs<R> a)
 {
     const Box &b = a.m.b;
     const PMWallLayout L = pm_wall_layout(b);
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= L.per_field) return;
+    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+    const int f = blockIdx.y;
+    if ((long)idx >= L.per_field) return;
     auto coord = [](int pos, int n) { return pos == 0 ? 0 : (pos == 1 ? n + 1 : n); };
     int gi, gj, kk;
-    if (idx < L.ys) {
+    if ((long)idx < L.ys) {
         if (!(a.wall & 1)) return;
-        const long pos = idx % 3, rem = idx / 3;
-        gi = coord((int)pos, b.nx); gj = (int)(rem % (b.ny + 2)); kk = (int)(rem / (b.ny + 2));
-    } else if (idx < L.zs) {
+        const unsigned rem = idx / 3u, h = (unsigned)b.ny + 2u;
+        kk = (int)(rem / h);
+        gj = (int)(rem % h);
+        gi = coord((int)(idx % 3u), b.nx);
+    } else if ((long)idx < L.zs) {
         if (!(a.wall & 2)) return;
-        const long pos = (idx - L.ys) / L.yp, rem = (idx - L.ys) % L.yp;
-        gj = coord((int)pos, b.ny); gi = (int)(rem % (b.nx + 2)); kk = (int)(rem / (b.nx + 2));
+        const unsigned at = idx - (unsigned)L.ys, pos = at / (unsigned)L.yp, rem = at % (unsigned)L.yp;
+        const unsigned h = (unsigned)b.nx + 2u;
+        kk = (int)(rem / h);
+        gi = (int)(rem % h);
+        gj = coord((int)pos, b.ny);
     } else {
         if (!(a.wall & 4)) return;
-        const long pos = (idx - L.zs) / L.zp, rem = (idx - L.zs) % L.zp;
-        kk = coord((int)pos, b.nz); gi = (int)(rem % (b.nx + 2)); gj = (int)(rem / (b.nx + 2));
+        const unsigned at = idx - (unsigned)L.zs, pos = at / (unsigned)L.zp, rem = at % (unsigned)L.zp;
+        const unsigned h = (unsigned)b.nx + 2u;
+        gj = (int)(rem / h);
+        gi = (int)(rem % h);
+        kk = coord((int)pos, b.nz);
     }
     const int ix = pm_src(gi, b.nx, a.wall & 1), jy = pm_src(gj, b.ny, a.wall & 2), kz = pm_src(kk, b.nz, a.wall & 4);
     const long o = ix + (long)b.gx * jy + (long)b.gxy * kz;
     auto dr = [&](double x) { return over_rho(x, a.prhof, a.pirhof, a.prpow2); };
-    const double f0 = (double)a.phi[o], fx = (double)a.phi[o + 1], fy = (double)a.phi[o + b.gx],
-                 fz = (double)a.phi[o + b.gxy];
-    R st[4];
-    st[0] = (R)((double)a.us[o] - dr((fx - f0) * a.pid * a.pdt));
-    st[1] = (R)((double)a.vs[o] - dr((fy - f0) * a.pid * a.pdt));
-    st[2] = (R)((double)a.ws[o] - dr((fz - f0) * a.pid * a.pdt));
-    st[3] = (R)((double)a.p_in[o] + f0);
-#pragma unroll
-    for (int f = 0; f < 4; f++)
-        a.wbuf[f * L.per_field + idx] = pm_ghost_chain(a.gtype[f], a.gplane + 6 * f, b, a.wall, gi, gj, kk, jy, kz, st[f]);
+    const R *src = f == 0 ? a.us : (f == 1 ? a.vs : (f == 2 ? a.ws : a.p_in));
+    const long up = f == 0 ? 1 : (f == 1 ? b.gx : (f == 2 ? b.gxy : 0));
+    const int gt = f == 0 ? a.gtype[0] : (f == 1 ? a.gtype[1] : (f == 2 ? a.gtype[2] : a.gtype[3]));
+    const double v0 = (double)src[o], f0 = (double)a.phi[o], fu = (double)a.phi[o + up];
+    const R st = f == 3 ? (R)(v0 + f0) : (R)(v0 - dr((fu - f0) * a.pid * a.pdt));
+    a.wbuf[f * L.per_field + idx] = pm_ghost_chain(gt, a.gplane + 6 * f, b, a.wall, gi, gj, kk, jy, kz, st);
 }
-
 
 }  // namespace fen
