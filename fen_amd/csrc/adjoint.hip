@@ -24,6 +24,7 @@
 // the recorded states are ghosted with their periodic images in place.
 #include <algorithm>
 #include <stdexcept>
+#include <utility>
 #include <vector>
 
 #include "fen_internal.hpp"
@@ -33,8 +34,6 @@ namespace fen {
 
 namespace {
 
-constexpr int kAX = 64, kAY = 4;
-
 struct AdjDims {
     int nx, ny, nz;
     long gx, gxy;
@@ -42,121 +41,126 @@ struct AdjDims {
     __device__ long g(int i, int j, int k) const { return (i + 1) + gx * (j + 1) + gxy * (k + 1); }
 };
 
-__device__ __forceinline__ int up(int i, int n) { return i + 1 == n ? 0 : i + 1; }
-__device__ __forceinline__ int dn(int i, int n) { return i == 0 ? n - 1 : i - 1; }
-
-struct AdjProjArgs {
-    const double *ub, *vb, *wb;   // ub'
+struct AdjStepArgs {
+    const double *u, *v, *w;      // recorded state (ghosted)
+    const double *ub[3], *dvo[3]; // ub', dvob'
     const double *psi;            // rb = S (pb' + (dt/rho) D ub')
     double *pb;                   // in pb', out pb
-    double *dvo[3];               // in dvob', out dvob
-    double *us[3];                // out ub*
-    double *dvb[3];               // out dvb
-    double id, s, dt_rho, dtA, dtB;   // s = rho/dt
+    double *ub_out[3], *dvo_out[3];
+    double id, id2, mu_rho, s, dt_rho, dtA, dtB;   // s = rho/dt
+    int nbx, nby, kb;             // tiles along x, y; planes per march
 };
 
-// ub* = ub' - (rho/dt) G rb, pb += (dt/rho) D ub*, dvb = dtA ub* + dvob', dvob = dtB ub*
-__global__ __launch_bounds__(kAX * kAY) void adj_project_kernel(AdjDims d, AdjProjArgs a)
-{
-    const int i = blockIdx.x * kAX + threadIdx.x % kAX, j = blockIdx.y * kAY + threadIdx.x / kAX, k = blockIdx.z;
-    if (i >= d.nx || j >= d.ny) return;
-    const int ip = up(i, d.nx), im = dn(i, d.nx), jp = up(j, d.ny), jm = dn(j, d.ny);
-    const int kp = up(k, d.nz), km = dn(k, d.nz);
-    const long q = d.q(i, j, k);
-    const double p0 = a.psi[q];
-    const double sx = a.ub[q] - a.s * ((a.psi[d.q(ip, j, k)] - p0) * a.id);
-    const double sy = a.vb[q] - a.s * ((a.psi[d.q(i, jp, k)] - p0) * a.id);
-    const double sz = a.wb[q] - a.s * ((a.psi[d.q(i, j, kp)] - p0) * a.id);
-    const long qxm = d.q(im, j, k), qym = d.q(i, jm, k), qzm = d.q(i, j, km);
-    const double sxm = a.ub[qxm] - a.s * ((p0 - a.psi[qxm]) * a.id);
-    const double sym = a.vb[qym] - a.s * ((p0 - a.psi[qym]) * a.id);
-    const double szm = a.wb[qzm] - a.s * ((p0 - a.psi[qzm]) * a.id);
-    const double div = ((sx - sxm) * a.id + (sy - sym) * a.id) + (sz - szm) * a.id;
-    a.pb[q] = a.pb[q] + a.dt_rho * div;
-    const double st[3] = {sx, sy, sz};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        a.us[c][q] = st[c];
-        a.dvb[c][q] = a.dtA * st[c] + a.dvo[c][q];
-        a.dvo[c][q] = a.dtB * st[c];
-    }
-}
-
-struct AdjMomArgs {
-    const double *u, *v, *w;      // recorded state (ghosted)
-    const double *us[3];          // ub*
-    const double *dvb[3];         // dvb (a, b, e below)
-    double *ub[3];                // out ub
-    double id, id2, mu_rho;
-};
-
-// ub = ub* + J_adv^T dvb + (mu/rho) lap(dvb), gathered per face, as a
-// k-march: a 64x4 tile of cells walks kMK planes of z with planes k-1, k,
-// k+1 of u, v, w (ghosted, images in place) and of the three dvb arrays
-// (periodic wrap) in an LDS ring, so each value is read from memory once per
-// tile instead of once per use (up to 13 uses per cell; a one-thread-per-cell
-// form reading every operand from memory took 87 us against 60 us at 128^3).
-// Plane k+2 is loaded into registers while plane k is computed.
-constexpr int kMX = 64, kMY = 4, kMK = 16;
+// One transposed step after its solve:
+//   ub* = ub' - (rho/dt) G rb, pb += (dt/rho) D ub*, dvb = dtA ub* + dvob',
+//   dvob = dtB ub*, ub = ub* + J_adv^T dvb + (mu/rho) lap(dvb), gathered per face,
+// as a k-march: a 64x4 tile of cells walks kb planes of z with planes k-1, k,
+// k+1 of u, v, w (ghosted, images in place) and of dvb in an LDS ring, and x,
+// y of ub* at planes k, k+1 (their divergence; z is carried).  Plane k+2 is
+// loaded into registers while plane k is computed.  A thread's first tile
+// element is its own cell, so what the cell needs of ub* stays in registers;
+// the second, for the first 140 threads, is one of the halo's.
+// HBM bounds it, 18 words per cell at 3.8 TB/s (the tiles' halos come on top,
+// from the L2 that neighbouring workgroups share): 80 us at 128^3, 88 with
+// tiles dealt round the XCDs; with ub* and dvb formed by a kernel of their own,
+// 12 words more, 60 + 61.
+constexpr int kMX = 64, kMY = 4;
 constexpr int kMLX = kMX + 2, kMN = kMLX * (kMY + 2);      // haloed tile
-constexpr int kMPER = (kMN + kMX * kMY - 1) / (kMX * kMY);   // tile elements per thread
+constexpr int kMHalo = 2 * kMLX + 2 * kMY;
 
-__global__ __launch_bounds__(kMX * kMY) void adj_momentum_march_kernel(AdjDims d, AdjMomArgs a)
+__global__ __launch_bounds__(kMX * kMY) void adj_step_kernel(AdjDims d, AdjStepArgs a)
 {
     __shared__ double lds[6 * 3 * kMN];   // [field u v w A B E][slot][tile]
-    const int i0 = blockIdx.x * kMX, j0 = blockIdx.y * kMY, k0 = blockIdx.z * kMK;
-    const int kend = min(k0 + kMK, d.nz);
+    __shared__ double star[2 * 2 * kMN];  // [ub*, vb*][slot][tile]
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int i0 = bid % a.nbx * kMX, j0 = bid / a.nbx % a.nby * kMY, k0 = bid / (a.nbx * a.nby) * a.kb;
+    const int kend = min(k0 + a.kb, d.nz);
     const int tx = threadIdx.x % kMX, ty = threadIdx.x / kMX;
     const int i = i0 + tx, j = j0 + ty;
     const bool active = i < d.nx && j < d.ny;
     const int nx = d.nx, ny = d.ny, nz = d.nz;
-    // tile element e at (i0 - 1 + e % kMLX, j0 - 1 + e / kMLX); past the grid
-    // clamped to the last ghost (values no active cell reads)
-    long og[kMPER], oq[kMPER];   // ghosted and interior (wrapped) plane offsets
-#pragma unroll
-    for (int m = 0; m < kMPER; m++) {
-        const int e = min((int)threadIdx.x + m * kMX * kMY, kMN - 1);
-        const int ii = min(i0 - 1 + e % kMLX, nx), jj = min(j0 - 1 + e / kMLX, ny);
-        og[m] = (ii + 1) + d.gx * (jj + 1);
-        oq[m] = (ii < 0 ? nx - 1 : (ii == nx ? 0 : ii)) + (long)nx * (jj < 0 ? ny - 1 : (jj == ny ? 0 : jj));
+    const int c = (ty + 1) * kMLX + tx + 1;
+    // the tile elements: position in the tile, offsets in a ghosted and in an
+    // interior (wrapped) plane, and of the interior neighbours above along x, y.
+    // Past the grid clamped to the last ghost (values no active cell reads)
+    const int h = (int)threadIdx.x;
+    const bool halo = h < kMHalo;
+    int hi = 0, hj = 0;
+    if (h < 2 * kMLX) {
+        hi = h % kMLX;
+        hj = h < kMLX ? 0 : kMY + 1;
+    } else if (halo) {
+        hi = h < 2 * kMLX + kMY ? 0 : kMX + 1;
+        hj = (h - 2 * kMLX) % kMY + 1;
     }
-    const double *Af = a.dvb[0], *Bf = a.dvb[1], *Ef = a.dvb[2];
-    double raw[6][kMPER];
-    auto fetch = [&](int kk) {   // plane kk in [-1, nz]
-        const long kg = d.gxy * (kk + 1), kq = (long)nx * ny * (kk < 0 ? nz - 1 : (kk == nz ? 0 : kk));
+    const int pos[2] = {c, hi + kMLX * hj};
+    int og[2], oq[2], ox[2], oy[2];
 #pragma unroll
-        for (int m = 0; m < kMPER; m++) {
-            raw[0][m] = a.u[og[m] + kg];
-            raw[1][m] = a.v[og[m] + kg];
-            raw[2][m] = a.w[og[m] + kg];
-            raw[3][m] = Af[oq[m] + kq];
-            raw[4][m] = Bf[oq[m] + kq];
-            raw[5][m] = Ef[oq[m] + kq];
+    for (int m = 0; m < 2; m++) {
+        const int ii = min(i0 - 1 + pos[m] % kMLX, nx), jj = min(j0 - 1 + pos[m] / kMLX, ny);
+        const int iq = ii < 0 ? nx - 1 : (ii == nx ? 0 : ii), jq = jj < 0 ? ny - 1 : (jj == ny ? 0 : jj);
+        og[m] = (ii + 1) + (int)d.gx * (jj + 1);
+        oq[m] = iq + nx * jq;
+        ox[m] = (iq + 1 == nx ? 0 : iq + 1) + nx * jq;
+        oy[m] = iq + nx * (jq + 1 == ny ? 0 : jq + 1);
+    }
+    const long plane = (long)nx * ny;
+    double raw[2][13];
+    auto fetch = [&](int kk) {   // plane kk in [-1, nz]
+        const int kw = kk < 0 ? nz - 1 : (kk == nz ? 0 : kk);
+        const long kg = d.gxy * (kk + 1), kq = plane * kw, kz = plane * (kw + 1 == nz ? 0 : kw + 1);
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            if (m == 1 && !halo) continue;
+            raw[m][0] = a.u[kg + og[m]];
+            raw[m][1] = a.v[kg + og[m]];
+            raw[m][2] = a.w[kg + og[m]];
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                raw[m][3 + f] = a.ub[f][kq + oq[m]];
+                raw[m][6 + f] = a.dvo[f][kq + oq[m]];
+            }
+            raw[m][9] = a.psi[kq + oq[m]];
+            raw[m][10] = a.psi[kq + ox[m]];
+            raw[m][11] = a.psi[kq + oy[m]];
+            raw[m][12] = a.psi[kz + oq[m]];
         }
     };
-    auto commit = [&](int slot) {
+    // the fetched plane into ring slot `slot` and star slot `ss`; own: ub* of the thread's cell
+    auto commit = [&](int slot, int ss, double (&own)[3]) {
 #pragma unroll
-        for (int m = 0; m < kMPER; m++) {
-            const int e = (int)threadIdx.x + m * kMX * kMY;
-            if (e < kMN) {
+        for (int m = 0; m < 2; m++) {
+            if (m == 1 && !halo) continue;
+            const int e = pos[m];
 #pragma unroll
-                for (int f = 0; f < 6; f++) lds[(f * 3 + slot) * kMN + e] = raw[f][m];
+            for (int f = 0; f < 3; f++) {
+                const double st = raw[m][3 + f] - a.s * ((raw[m][10 + f] - raw[m][9]) * a.id);
+                lds[(f * 3 + slot) * kMN + e] = raw[m][f];
+                lds[((3 + f) * 3 + slot) * kMN + e] = a.dtA * st + raw[m][6 + f];
+                if (f < 2) star[(f * 2 + ss) * kMN + e] = st;
+                if (m == 0) own[f] = st;
             }
         }
     };
+    double below[3], here[3], above[3];   // ub* of the thread's cell at k - 1, k, k + 1
     fetch(k0 - 1);
-    commit(0);
+    commit(0, 0, below);   // (star slot 0 is written again for k0, each element by the same thread)
     fetch(k0);
-    commit(1);
+    commit(1, 0, here);
     fetch(k0 + 1);
-    int sm = 0, sc = 1, sn = 2;
-    const int c = (ty + 1) * kMLX + tx + 1;
+    int sm = 0, sc = 1, sn = 2, ss = 0;
     const double id = a.id;
     for (int k = k0; k < kend; k++) {
-        commit(sn);   // plane k + 1
+        commit(sn, ss ^ 1, above);   // plane k + 1
         __syncthreads();
         if (k + 2 <= nz && k + 2 <= kend) fetch(k + 2);
         if (active) {
+            const long q = d.q(i, j, k);
+            const double sxm = star[ss * kMN + c - 1], sym = star[(2 + ss) * kMN + c - kMLX];
+            const double div = ((here[0] - sxm) * id + (here[1] - sym) * id) + (here[2] - below[2]) * id;
+            a.pb[q] = a.pb[q] + a.dt_rho * div;
+#pragma unroll
+            for (int f = 0; f < 3; f++) a.dvo_out[f][q] = a.dtB * here[f];
             auto at = [&](int f, int di, int dj, int dk) {
                 const int sl = dk < 0 ? sm : (dk > 0 ? sn : sc);
                 return lds[(f * 3 + sl) * kMN + c + dj * kMLX + di];
@@ -185,7 +189,6 @@ __global__ __launch_bounds__(kMX * kMY) void adj_momentum_march_kernel(AdjDims d
                 return ((at(f, 1, 0, 0) - 2.0 * c0 + at(f, -1, 0, 0)) + (at(f, 0, 1, 0) - 2.0 * c0 + at(f, 0, -1, 0)) +
                         (at(f, 0, 0, 1) - 2.0 * c0 + at(f, 0, 0, -1))) * a.id2;
             };
-            const long q = d.q(i, j, k);
             const double u0 = U(0, 0, 0), v0 = V(0, 0, 0), w0 = W(0, 0, 0);
             double gu = Qxx(0, 0, 0) * 0.5 * (u0 + U(1, 0, 0)) + Qxx(-1, 0, 0) * 0.5 * (U(-1, 0, 0) + u0);
             gu += Rxy(0, 0, 0) * 0.25 * (V(1, 0, 0) + v0) + Rxy(0, -1, 0) * 0.25 * (V(1, -1, 0) + V(0, -1, 0));
@@ -196,13 +199,19 @@ __global__ __launch_bounds__(kMX * kMY) void adj_momentum_march_kernel(AdjDims d
             double gw = Qzz(0, 0, 0) * 0.5 * (w0 + W(0, 0, 1)) + Qzz(0, 0, -1) * 0.5 * (W(0, 0, -1) + w0);
             gw += Rxz(0, 0, 0) * 0.25 * (U(0, 0, 1) + u0) + Rxz(-1, 0, 0) * 0.25 * (U(-1, 0, 1) + U(-1, 0, 0));
             gw += Ryz(0, 0, 0) * 0.25 * (V(0, 0, 1) + v0) + Ryz(0, -1, 0) * 0.25 * (V(0, -1, 1) + V(0, -1, 0));
-            a.ub[0][q] = a.us[0][q] + gu + a.mu_rho * lap(3);
-            a.ub[1][q] = a.us[1][q] + gv + a.mu_rho * lap(4);
-            a.ub[2][q] = a.us[2][q] + gw + a.mu_rho * lap(5);
+            a.ub_out[0][q] = here[0] + gu + a.mu_rho * lap(3);
+            a.ub_out[1][q] = here[1] + gv + a.mu_rho * lap(4);
+            a.ub_out[2][q] = here[2] + gw + a.mu_rho * lap(5);
         }
         __syncthreads();   // every read of slot sm precedes the next commit into it
         const int t = sm;
         sm = sc; sc = sn; sn = t;
+        ss ^= 1;
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            below[f] = here[f];
+            here[f] = above[f];
+        }
     }
 }
 
@@ -216,7 +225,7 @@ struct AdjointTape {
     std::vector<double *> ckpt;    // [u v w p](ghosted) [dvo x3](interior), one block per checkpoint
     double *final_state = nullptr;
     std::vector<double *> seg;     // every x [u v w](ghosted)
-    double *work = nullptr;        // 14 interior arrays of adjoint state and temporaries
+    double *work = nullptr;        // 14 interior arrays: adjoint state [ub x3][pb][dvob x3], next [ub x3][dvob x3], rb
 };
 
 namespace {
@@ -254,19 +263,23 @@ double *dalloc(size_t n)
 
 AdjDims dims(const fen_ctx *c) { return AdjDims{c->nx, c->ny, c->nz, c->box.gx, c->box.gxy}; }
 
-dim3 cell_grid(const fen_ctx *c)
+// Planes per march: 16 (18 are formed for them) where that gives two
+// workgroups per CU, as many as its LDS holds; shorter ones on smaller grids,
+// down to 4.
+int march_planes(const fen_ctx *c, long tiles)
 {
-    return dim3((unsigned)((c->nx + kAX - 1) / kAX), (unsigned)((c->ny + kAY - 1) / kAY), (unsigned)c->nz);
+    int kb = 16;
+    while (kb > 4 && tiles * ((c->nz + kb - 1) / kb) < 2L * c->num_cu) kb /= 2;
+    return kb;
 }
 
-// One adjoint step at the recorded state `st` ([u v w] ghosted).
-void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, double *pb, double **dvo)
+// One adjoint step at the recorded state `st` ([u v w] ghosted); ub and dvo
+// become the arrays of ub_out and dvo_out, and those the old ones.
+void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, double *pb, double **dvo, double **ub_out,
+                  double **dvo_out)
 {
-    const size_t n = c->n_int;
-    double *w = t->work + 7 * n;   // temporaries after the 7 adjoint-state arrays
-    double *us[3] = {w, w + n, w + 2 * n}, *dvb[3] = {w + 3 * n, w + 4 * n, w + 5 * n}, *r = w + 6 * n;
+    double *r = t->work + 13 * c->n_int;
     const AdjDims d = dims(c);
-    const dim3 grid = cell_grid(c), blk(kAX * kAY);
     const double rho = c->density, dt = t->dt;
     const double id = 1.0 / c->delta;
     const double A = 1.0 + 0.5 * dt / t->dt_o, B = -(0.5 * dt / t->dt_o);
@@ -284,26 +297,30 @@ void adjoint_step(fen_ctx *c, AdjointTape *t, const double *st, double **ub, dou
     launch_z_solve<double>(c, 1.0 / (double)(float)((long)c->nx * c->ny * c->nz));
     if (!plane) launch_y_fft<double>(c, +1, 1.0);
     launch_c2r<double>(c, r, 0, sx, sy, false, AxisCopies{});
-    AdjProjArgs pa{};
-    pa.ub = ub[0]; pa.vb = ub[1]; pa.wb = ub[2];
-    pa.psi = r;
-    pa.pb = pb;
-    for (int k = 0; k < 3; k++) { pa.dvo[k] = dvo[k]; pa.us[k] = us[k]; pa.dvb[k] = dvb[k]; }
-    pa.id = id;
-    pa.s = rho / dt;
-    pa.dt_rho = dt / rho;
-    pa.dtA = dt * A;
-    pa.dtB = dt * B;
-    hipLaunchKernelGGL(adj_project_kernel, grid, blk, 0, c->stream, d, pa);
-    AdjMomArgs ma{};
-    ma.u = st; ma.v = st + c->n_ghost; ma.w = st + 2 * c->n_ghost;
-    for (int k = 0; k < 3; k++) { ma.us[k] = us[k]; ma.dvb[k] = dvb[k]; ma.ub[k] = ub[k]; }
-    ma.id = id;
-    ma.id2 = 1.0 / (c->delta * c->delta);
-    ma.mu_rho = c->viscosity / rho;
-    const dim3 mgrid((unsigned)((c->nx + kMX - 1) / kMX), (unsigned)((c->ny + kMY - 1) / kMY),
-                     (unsigned)((c->nz + kMK - 1) / kMK));
-    hipLaunchKernelGGL(adj_momentum_march_kernel, mgrid, dim3(kMX * kMY), 0, c->stream, d, ma);
+    AdjStepArgs a{};
+    a.u = st; a.v = st + c->n_ghost; a.w = st + 2 * c->n_ghost;
+    for (int k = 0; k < 3; k++) {
+        a.ub[k] = ub[k]; a.dvo[k] = dvo[k];
+        a.ub_out[k] = ub_out[k]; a.dvo_out[k] = dvo_out[k];
+    }
+    a.psi = r;
+    a.pb = pb;
+    a.id = id;
+    a.id2 = 1.0 / (c->delta * c->delta);
+    a.mu_rho = c->viscosity / rho;
+    a.s = rho / dt;
+    a.dt_rho = dt / rho;
+    a.dtA = dt * A;
+    a.dtB = dt * B;
+    a.nbx = (c->nx + kMX - 1) / kMX;
+    a.nby = (c->ny + kMY - 1) / kMY;
+    const long tiles = (long)a.nbx * a.nby;
+    a.kb = march_planes(c, tiles);
+    hipLaunchKernelGGL(adj_step_kernel, dim3((unsigned)(tiles * ((c->nz + a.kb - 1) / a.kb))), dim3(kMX * kMY), 0, c->stream, d, a);
+    for (int k = 0; k < 3; k++) {
+        std::swap(ub[k], ub_out[k]);
+        std::swap(dvo[k], dvo_out[k]);
+    }
 }
 
 }  // namespace
@@ -378,6 +395,8 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
     while ((int)t->seg.size() < std::min(t->every, t->nsteps)) t->seg.push_back(dalloc(3 * c->n_ghost));
     double *ub[3] = {t->work, t->work + n, t->work + 2 * n}, *pb = t->work + 3 * n;
     double *dvo[3] = {t->work + 4 * n, t->work + 5 * n, t->work + 6 * n};
+    double *ub2[3] = {t->work + 7 * n, t->work + 8 * n, t->work + 9 * n};
+    double *dvo2[3] = {t->work + 10 * n, t->work + 11 * n, t->work + 12 * n};
     for (int d = 0; d < 3; d++)
         copy_to_device(c->stream, ub[d], seed[d], n, sizeof(double));
     FEN_HIP_CHECK(hipMemsetAsync(pb, 0, 4 * n * sizeof(double), c->stream));   // pb and dvo
@@ -390,7 +409,7 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
         // the segment's states, each formed straight into its slot (the
         // state after the segment's last step is not needed)
         states_fp64(c, t->dt, len, t->seg.data());
-        for (int s = len - 1; s >= 0; s--) adjoint_step(c, t, t->seg[s], ub, pb, dvo);
+        for (int s = len - 1; s >= 0; s--) adjoint_step(c, t, t->seg[s], ub, pb, dvo, ub2, dvo2);
     }
     for (int d = 0; d < 3; d++)
         copy_to_host(c->stream, grad[d], ub[d], n, sizeof(double));

@@ -72,6 +72,9 @@ def test_plane_steps(n, wall_z):
             assert np.abs(a - b).max() <= 512 * EPS[0] * np.abs(b).max(), f
 
 
-def test_plane_adjoint(monkeypatch):
-    """The transposed projection's right-hand side, formed as the planes load."""
-    adjoint_matches_oracle((64, 32, 128), monkeypatch)
+@pytest.mark.parametrize("n", [(64, 32, 128), (128, 64, 256)])
+def test_plane_adjoint(n, monkeypatch):
+    """The transposed projection's right-hand side, formed as the planes load;
+    the transposed step's march in its shortest and longest cuts."""
+    print("plane adjoint", n, flush=True)
+    adjoint_matches_oracle(n, monkeypatch)
