@@ -82,6 +82,7 @@ __device__ __forceinline__ void dct2_out(const DctArgs &a, const double2 *buf, c
             return;
         }
     }
+#pragma unroll 4
     for (int e = threadIdx.x; e < TJ * N; e += NT) {
         const int row = k_fast ? e / N : e % TJ, k = k_fast ? e % N : e / TJ;
         const long r = row0 + row;
@@ -165,12 +166,15 @@ __global__ __launch_bounds__(kNB) void dct2_rows_kernel(DctArgs a)
 //   SRC 2: pair (2rT+2j, +1); the odd x_{2rT+2j+1} goes to thread T-1-j.
 //   SRC 0: ghosted pair (q, q+1), q = 2rT + 2j, holds elements q-1 (odd)
 //   and q (even) (ghosted x index = element + 1); the odd one goes to thread
-//   T-j, and thread 0 takes its own from chunk r+1 (lane 0 loads a fifth
-//   pair, q = N, for x_{N-1}).  Needs 16-byte aligned fields and even gx.
+//   T-j, and thread 0 takes its own from chunk r+1 (x_{N-1} for the last).
+//   Needs 16-byte aligned fields and even gx.  D3 (three components) is a
+//   template argument, no load stands behind a branch and none is scheduled
+//   among a row's arithmetic, so a row waits for memory once (256 x 200 nn:
+//   9.9 -> 7.5 us, 128 x 128 x 160 nnn: 26.7 -> 24.2).
 // MKL: the (cos, sin) table of the last step in LDS (it costs the x pass an
 // LDS-bound workgroup per CU, so only the y pass and one-wave workgroups take
 // it).
-template <int N, int SRC, int MKL, int NT = kNB>
+template <int N, int SRC, int D3, int MKL, int NT = kNB>
 __global__ __launch_bounds__(NT) void dct2_pairs_kernel(DctArgs a)
 {
     constexpr int T = nb_tpl<N>(), L = nb_lines<N, NT>(), TJ = 2 * L, LL = lds_line<N>();
@@ -204,27 +208,45 @@ __global__ __launch_bounds__(NT) void dct2_pairs_kernel(DctArgs a)
         } else {
             const int ri = (int)r, jy = ri % a.b.ny + 1, kz = ri / a.b.ny + 1;
             const long g0 = a.b.g(0, jy, kz);
-            // elements q - 1 and q from the ghosted pair (q, q + 1)
-            auto pair = [&](long gq, double &d_odd, double &d_even) {
-                const double um = a.u[gq - 1];
-                const double2 uu = ld2(a.u + gq), vv = ld2(a.v + gq), vs = ld2(a.v + gq - a.b.gx);
-                double d0 = (uu.x - um) * a.id + (vv.x - vs.x) * a.id;
-                double d1 = (uu.y - uu.x) * a.id + (vv.y - vs.y) * a.id;
-                if (a.d3) {
-                    const double2 ww = ld2(a.w + gq), ws = ld2(a.w + gq - a.b.gxy);
-                    d0 = d0 + (ww.x - ws.x) * a.id;
-                    d1 = d1 + (ww.y - ws.y) * a.id;
-                }
-                d_odd = ok ? d0 * a.rho / a.dt : 0.0;
-                d_even = ok ? d1 * a.rho / a.dt : 0.0;
+            // div(u*) rho/dt at x element e from its cell's loads
+            auto div = [&](double u0, double um, double v0, double vm, double w0, double wm) {
+                double dv = (u0 - um) * a.id + (v0 - vm) * a.id;
+                if constexpr (D3) dv = dv + (w0 - wm) * a.id;
+                return ok ? dv * a.rho / a.dt : 0.0;
             };
+            // the row's loads, in flight together; x_{N-1} is for thread 0, but
+            // every thread loads it (a branch would wait for the loads before it)
+            double um[5], un[1], vn[2], wn[2] = {};
+            double2 uu[4], vv[4], vs[4], ww[4] = {}, ws[4] = {};
 #pragma unroll
-            for (int c = 0; c < 4; c++) pair(g0 + 2 * c * T + 2 * j, od[h][c], ev[h][c]);
-            od[h][4] = 0.0;
-            if (j == 0) {
-                double unused;
-                pair(g0 + N, od[h][4], unused);
+            for (int c = 0; c < 4; c++) {
+                const long gq = g0 + 2 * c * T + 2 * j;
+                um[c] = a.u[gq - 1];
+                uu[c] = ld2(a.u + gq);
+                vv[c] = ld2(a.v + gq);
+                vs[c] = ld2(a.v + gq - a.b.gx);
+                if constexpr (D3) {
+                    ww[c] = ld2(a.w + gq);
+                    ws[c] = ld2(a.w + gq - a.b.gxy);
+                }
             }
+            const long gn = g0 + N;
+            un[0] = a.u[gn];
+            um[4] = a.u[gn - 1];
+            vn[0] = a.v[gn];
+            vn[1] = a.v[gn - a.b.gx];
+            if constexpr (D3) {
+                wn[0] = a.w[gn];
+                wn[1] = a.w[gn - a.b.gxy];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // elements q - 1 and q from the ghosted pair (q, q + 1)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                od[h][c] = div(uu[c].x, um[c], vv[c].x, vs[c].x, ww[c].x, ws[c].x);
+                ev[h][c] = div(uu[c].y, uu[c].x, vv[c].y, vs[c].y, ww[c].y, ws[c].y);
+            }
+            od[h][4] = div(un[0], um[4], vn[0], vn[1], wn[0], wn[1]);
         }
     }
     double2 v[8];
@@ -266,6 +288,8 @@ struct Dct3Args {
     AxisCopies copies;   // x pass with gl == 1: ghosts to write (x: COPY_MIRROR)
     double post;
 };
+
+typedef double Pair8 __attribute__((ext_vector_type(2), aligned(8)));   // a ghosted row starts at 8 bytes
 
 template <int N, int DST, int NT = kNB>
 __global__ __launch_bounds__(NT) void dct3_rows_kernel(Dct3Args a)
@@ -334,7 +358,33 @@ __global__ __launch_bounds__(NT) void dct3_rows_kernel(Dct3Args a)
     }
     fft_regs<N, 1>(v, line, t, tw);
     // y_{2m} = u_m, y_{2m+1} = u_{N-1-m}: position p holds y_i,
-    // i = 2p (p < N/2), 2(N-1-p)+1 (p >= N/2)
+    // i = 2p (p < N/2), 2(N-1-p)+1 (p >= N/2).  Where a line's threads are in
+    // one wave, the odd neighbour of position t + q N/8 comes from thread
+    // N/8 - 1 - t's register 7 - q and both go out in one 16-byte store (apart,
+    // every store left half of its lines; 128 x 128 x 160 nnn, y pass: 15.6 ->
+    // 13.6 us).
+    constexpr int T8 = N / 8;
+    double2 odd[4];
+    if constexpr (T8 <= 64) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            odd[q] = double2{__shfl(v[7 - q].x, T8 - 1 - t, T8), __shfl(v[7 - q].y, T8 - 1 - t, T8)};
+    }
+    auto put = [&](double *orow, int h) {
+        if constexpr (T8 <= 64) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<Pair8 *>(orow + 2 * (t + q * T8)) =
+                    Pair8{(h ? v[q].y : v[q].x) * a.post, (h ? odd[q].y : odd[q].x) * a.post};
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const int p = t + q * T8;
+                const int i = p < N / 2 ? 2 * p : 2 * (N - 1 - p) + 1;
+                orow[i] = (h ? v[q].y : v[q].x) * a.post;
+            }
+        }
+    };
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const long r = row0 + 2 * l + h;
@@ -351,12 +401,7 @@ __global__ __launch_bounds__(NT) void dct3_rows_kernel(Dct3Args a)
             for (int dk = 0; dk < nk; dk++)
                 for (int dj = 0; dj < nj; dj++) {
                     double *orow = a.out + a.gl + a.sx * jd[dj] + a.sy * kd[dk];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        const int p = t + q * (N / 8);
-                        const int i = p < N / 2 ? 2 * p : 2 * (N - 1 - p) + 1;
-                        orow[i] = (h ? v[q].y : v[q].x) * a.post;
-                    }
+                    put(orow, h);
                     // Neumann x ghosts: phi(0) = phi(1) is y_0 (position 0),
                     // phi(N+1) = phi(N) is y_{N-1} (position N/2): thread 0's q = 0, 4
                     if (a.copies.x && t == 0) {
@@ -366,12 +411,7 @@ __global__ __launch_bounds__(NT) void dct3_rows_kernel(Dct3Args a)
                 }
         } else {
             double *orow = a.out + r * N;
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const int p = t + q * (N / 8);
-                const int i = p < N / 2 ? 2 * p : 2 * (N - 1 - p) + 1;
-                orow[i] = (h ? v[q].y : v[q].x) * a.post;
-            }
+            put(orow, h);
         }
     }
 }
@@ -646,14 +686,14 @@ static bool one_wave(const fen_ctx *c, long nrows, int N)
     return N <= 512 && (long)row_blocks(nrows, N) < c->num_cu / 2;
 }
 
-template <int N, int SRC, int MKL> static void launch_dct2_pairs(const fen_ctx *c, const DctArgs &a)
+template <int N, int SRC, int D3, int MKL> static void launch_dct2_pairs(const fen_ctx *c, const DctArgs &a)
 {
     if constexpr (N <= 512) {
         if (one_wave(c, a.nrows, N))
-            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, 1, 64>), dim3(row_blocks(a.nrows, N, 64)), dim3(64), 0,
+            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, D3, 1, 64>), dim3(row_blocks(a.nrows, N, 64)), dim3(64), 0,
                                c->stream, a);
         else
-            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, MKL>), dim3(row_blocks(a.nrows, N)), dim3(kNB), 0, c->stream,
+            hipLaunchKernelGGL((dct2_pairs_kernel<N, SRC, D3, MKL>), dim3(row_blocks(a.nrows, N)), dim3(kNB), 0, c->stream,
                                a);
     } else {
         throw std::logic_error("dct2_pairs_kernel takes N <= 512");
@@ -700,7 +740,8 @@ void launch_dct2_x(fen_ctx *c, const double *const *vel, const double *direct, l
     const bool pairs = vel && c->nx <= 512 && c->box.gx % 2 == 0 && aligned16(a.u) && aligned16(a.v) &&
                        (!a.d3 || aligned16(a.w));
 #define L_D2(NN)                                                                              \
-    if (pairs) launch_dct2_pairs<NN, 0, 0>(c, a);                                             \
+    if (pairs && a.d3) launch_dct2_pairs<NN, 0, 1, 0>(c, a);                                  \
+    else if (pairs) launch_dct2_pairs<NN, 0, 0, 0>(c, a);                                     \
     else if (vel) hipLaunchKernelGGL((dct2_rows_kernel<NN, 0>), dim3(grid), dim3(kNB), 0, c->stream, a); \
     else hipLaunchKernelGGL((dct2_rows_kernel<NN, 1>), dim3(grid), dim3(kNB), 0, c->stream, a);
     FEN_NB_DISPATCH(c->nx, L_D2)
@@ -756,7 +797,7 @@ void launch_dct_y(fen_ctx *c, int inverse, double post)
         a.orr = c->ny;
         // the register-loading form for N <= 512, with the DCT's (cos, sin) table in LDS
 #define L_DY(NN)                                                                              \
-    if (c->ny <= 512) launch_dct2_pairs<NN, 2, 1>(c, a);                                      \
+    if (c->ny <= 512) launch_dct2_pairs<NN, 2, 0, 1>(c, a);                                   \
     else hipLaunchKernelGGL((dct2_rows_kernel<NN, 2>), dim3(grid), dim3(kNB), 0, c->stream, a);
         FEN_NB_DISPATCH(c->ny, L_DY)
 #undef L_DY
