@@ -38,7 +38,6 @@ struct AdjDims {
     int nx, ny, nz;
     long gx, gxy;
     __device__ long q(int i, int j, int k) const { return i + (long)nx * (j + (long)ny * k); }   // 0-based
-    __device__ long g(int i, int j, int k) const { return (i + 1) + gx * (j + 1) + gxy * (k + 1); }
 };
 
 struct AdjStepArgs {

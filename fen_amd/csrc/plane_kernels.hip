@@ -19,6 +19,7 @@
 
 #include "fen_internal.hpp"
 #include "fft_device.hpp"
+#include "rhs_device.hpp"
 
 namespace fen {
 
@@ -26,8 +27,7 @@ namespace {
 
 template <class R> struct PlaneArgs {
     using C = typename Cplx<R>::type;
-    // forward.  MODE 0: ghosted u, v, w; 1: u is the right-hand side (strides
-    // sx, sy, ghost level gl); 2: interior u, v, w and p (launch_adj_r2c's)
+    // forward (rhs_load's)
     const R *u, *v, *w, *p;
     C *spec;
     const C *twx, *twy;
@@ -64,28 +64,13 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void plane_fwd_kernel(Pl
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const int j = 2 * l + h + 1;
+        R f[8][7];   // the row's loads, all issued before the first is used
+#pragma unroll
+        for (int q = 0; q < 8; q++) rhs_load<R, MODE, 1>(a, f[q], t + q * TX + 1, j, k);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            const int i = t + q * TX + 1;
-            double val;
-            if constexpr (MODE == 2) {
-                const long row = (long)NX * ((j - 1) + (long)NY * (k - 1));
-                const long rowj = (long)NX * ((j == 1 ? NY - 1 : j - 2) + (long)NY * (k - 1));
-                const long rowk = (long)NX * ((j - 1) + (long)NY * (k == 1 ? a.nz - 1 : k - 2));
-                const int x = i - 1, xm = i == 1 ? NX - 1 : i - 2;
-                const double d = (((double)a.u[row + x] - (double)a.u[row + xm]) * a.id +
-                                  ((double)a.v[row + x] - (double)a.v[rowj + x]) * a.id) +
-                                 ((double)a.w[row + x] - (double)a.w[rowk + x]) * a.id;
-                val = (double)a.p[row + x] + a.scale * d;
-            } else if constexpr (MODE == 1) {
-                val = a.u[(i - 1 + a.gl) + a.sx * (j - 1 + a.gl) + a.sy * (k - 1 + a.gl)];
-            } else {
-                const long g = a.b.g(i, j, k);
-                const double d = (((double)a.u[g] - (double)a.u[g - 1]) * a.id +
-                                  ((double)a.v[g] - (double)a.v[g - a.b.gx]) * a.id) +
-                                 ((double)a.w[g] - (double)a.w[g - a.b.gxy]) * a.id;
-                val = d * a.rho / a.dt;
-            }
+            const double val = rhs_value<R, MODE, 1>(a, f[q]);
             if (h == 0) v[q].x = (R)val;
             else v[q].y = (R)val;
         }

@@ -11,6 +11,7 @@
 
 #include "fen_internal.hpp"
 #include "fft_device.hpp"
+#include "rhs_device.hpp"
 
 namespace fen {
 
@@ -38,11 +39,12 @@ template <class R> struct DivR2CArgs {
     double scale;
 };
 
-// DIRECT: 0 div(u*) rho / dt of the ghosted velocity, 1 `u` itself, 2 (FP64)
-// p + scale div(u, v, w) of interior arrays, periodic in every direction (the
-// discrete adjoint's right-hand side).
+// DIRECT: the right-hand side, rhs_load's MODE.
+// 512-thread workgroups keep to 128 registers, so that a CU holds two (512 x 256
+// x 192: 179 us; 210 at 130 registers); smaller ones are faster with what a
+// row's loads take (256^3: 112 us against 117, 128^3: 16.1 against 17.3).
 template <class R, int D3, int N, int DIRECT, int NT = kBlock>
-__global__ __launch_bounds__(NT) void div_r2c_kernel(DivR2CArgs<R> a)
+__global__ __launch_bounds__(NT, NT > 256 ? 4 : 1) void div_r2c_kernel(DivR2CArgs<R> a)
 {
     using C = typename Cplx<R>::type;
     constexpr int T = threads_per_line<N>(), L = NT / T, TJ = 2 * L, LL = lds_line<N>();
@@ -61,28 +63,13 @@ __global__ __launch_bounds__(NT) void div_r2c_kernel(DivR2CArgs<R> a)
         const bool ok = r < a.nrows;
         const long rr = ok ? r : row0;   // a valid row: the loads are kept, their values dropped
         const int j = (int)(rr & (a.b.ny - 1)) + 1, k = (int)(rr >> a.ny_shift) + 1;
+        R f[8][7];   // the row's loads, all issued before the first is used
+#pragma unroll
+        for (int q = 0; q < 8; q++) rhs_load<R, DIRECT, D3>(a, f[q], t + q * (N / 8) + 1, j, k);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            const int i = t + q * (N / 8) + 1;
-            double val;
-            if constexpr (DIRECT == 2) {
-                const long row = (long)N * ((j - 1) + (long)a.b.ny * (k - 1));
-                const long rowj = (long)N * ((j == 1 ? a.b.ny - 1 : j - 2) + (long)a.b.ny * (k - 1));
-                const long rowk = (long)N * ((j - 1) + (long)a.b.ny * (k == 1 ? a.b.nz - 1 : k - 2));
-                const int x = i - 1, xm = i == 1 ? N - 1 : i - 2;
-                const double d = (((double)a.u[row + x] - (double)a.u[row + xm]) * a.id +
-                                  ((double)a.v[row + x] - (double)a.v[rowj + x]) * a.id) +
-                                 ((double)a.w[row + x] - (double)a.w[rowk + x]) * a.id;
-                val = (double)a.p[row + x] + a.scale * d;
-            } else if constexpr (DIRECT) {
-                val = a.u[(i - 1 + a.gl) + a.sx * (j - 1 + a.gl) + a.sy * (k - 1 + a.gl)];
-            } else {
-                const long g = a.b.g(i, j, k);
-                double d = ((double)a.u[g] - (double)a.u[g - 1]) * a.id +
-                           ((double)a.v[g] - (double)a.v[g - a.b.gx]) * a.id;
-                if constexpr (D3) d = d + ((double)a.w[g] - (double)a.w[g - a.b.gxy]) * a.id;
-                val = d * a.rho / a.dt;
-            }
+            const double val = rhs_value<R, DIRECT, D3>(a, f[q]);
             if (h == 0) v[q].x = ok ? (R)val : R(0);
             else v[q].y = ok ? (R)val : R(0);
         }
