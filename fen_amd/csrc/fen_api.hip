@@ -6,12 +6,13 @@
 //   K2 div(u*)*rho/dt + x r2c or DCT-II
 //   K3..K5 y / z passes: FFT, eigenvalue divide or Thomas per solver
 //   K6 x c2r or DCT-III -> phi (+ mean, pp/ppn/pn)   ghost(phi)
+//   (small ppp and ppn planes: K2 with the y pass, and K6 with the one back, as one)
 //   K7 projection + p update           ghost(u, p)
 //   K8 checks
-// On the grids the fused kernels support (deferrable) a step ends after K6 with
-// K7-K8 pending; the next step
-// runs them fused with its K1 (step_pending), and anything that reads or
-// changes the state first completes them (flush_pending).
+// The ghost launches are for what the producers do not write themselves.  On
+// the grids the fused kernels support (deferrable) a step ends after K6 with
+// K7-K8 pending; the next step runs them fused with its K1 (step_pending), and
+// anything that reads or changes the state first completes them (flush_pending).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>

@@ -241,7 +241,10 @@ bool plane_pass(const fen_ctx *c)
     // planes 209 -> 191); with sixteen (128 x 128) one workgroup fills a CU, and
     // 128 planes leave the others idle (128^3: 93 -> 97; 256 planes 201 -> 194).
     if (c->dim != 3 || (c->solver != FEN_SOLVER_PPP && c->solver != FEN_SOLVER_PPN)) return false;
+    // One block sum per plane: at most the 32768 that the allocation-free
+    // solve's fixed scratch holds, so that it takes every grid it would without.
     const long m = (long)c->nx * c->ny;
+    if (c->nz > 32768) return false;
     return c->nx >= 16 && c->nx <= 128 && c->ny >= 16 && c->ny <= 128 && m >= 1024 && (m <= 4096 || (m <= 8192 && c->nz >= 128));
 }
 

@@ -24,14 +24,14 @@ import sys
 
 # demangled kernel name -> the library's profiler name (fen_profile_name)
 _PATTERNS = [
-    (r"project_momentum_kernel", "project_momentum"),
+    (r"project_momentum_kernel|step_kernel_2d", "project_momentum"),
     (r"wall_state_kernel", "wall_state"),
     (r"(?<!adj_)momentum_march_kernel|momentum_kernel_2d", "momentum"),
     (r"project_march_kernel|project_kernel_2d", "project"),
-    (r"div_r2c_kernel", "div_r2c"),
-    (r"y_kernel<(?:double|float), \d+, -1, 0>", "y_fwd"),
-    (r"y_kernel<(?:double|float), \d+, 1, 0>", "y_inv"),
-    (r"y_kernel<(?:double|float), \d+, -?1, 1>", "y_solve"),
+    (r"div_r2c_kernel|plane_fwd_kernel", "div_r2c"),
+    (r"y_kernel<(?:double|float), \d+, -1, 0(?:, \d+)?>", "y_fwd"),
+    (r"y_kernel<(?:double|float), \d+, 1, 0(?:, \d+)?>", "y_inv"),
+    (r"y_kernel<(?:double|float), \d+, -?1, 1(?:, \d+)?>", "y_solve"),
     (r"z_solve_kernel|z_solve_pair_kernel", "z_solve"),
     (r"thomas_c1_kernel|thomas_starts_kernel", "thomas_c1"),
     (r"thomas_kernel|thomas_general_kernel|thomas_column_kernel|thomas_chunk_kernel", "thomas"),
@@ -41,15 +41,17 @@ _PATTERNS = [
     (r"mf_fields_kernel", "mf_fields"),
     (r"mf_momentum_kernel", "mf_momentum"),
     (r"adj_momentum_(march_)?kernel", "adj_momentum"),
+    (r"adj_step_kernel", "adj_step"),
     (r"adj_project_kernel", "adj_project"),
     (r"adj_rhs_kernel", "adj_rhs"),
     (r"dct2_(rows|pairs)_kernel", "dct2"),
     (r"dct3_rows_kernel", "dct3"),
     (r"rfft_rows_kernel|irfft_rows_kernel", "rfft_y"),
-    (r"c2r_kernel", "c2r"),
+    (r"c2r_kernel|plane_bwd_kernel", "c2r"),
     (r"ghost_kernel", "ghost"),
     (r"checks_final_kernel|checks_kernel", "checks"),
     (r"mean_shift_kernel|apply_shift_kernel", "shift"),
+    (r"solve_end_kernel", "solve_end"),
     (r"copyBuffer", "hip_copy"),
 ]
 

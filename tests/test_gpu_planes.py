@@ -45,6 +45,15 @@ def test_plane_solves(n, wall_z, precision):
     assert np.abs(a - b).max() <= bar * EPS[precision] * np.abs(b).max()
 
 
+def test_long_grid_without_allocation():
+    """More planes than the allocation-free solve's scratch holds sums: the separate passes."""
+    n = (32, 32, 32770)
+    print("plane", n, flush=True)
+    f = np.asfortranarray(np.random.default_rng(1).standard_normal(n))
+    with Solver(3, n, tuple(m / 8.0 for m in n), bc=_bc(1)) as g:
+        assert np.array_equal(g.solve_poisson_noalloc(f, 0), g.solve_poisson(f, 0))
+
+
 @pytest.mark.parametrize("wall_z", [0, 1])
 @pytest.mark.parametrize("n", [(16, 64, 8), (32, 32, 8), (64, 16, 8), (128, 32, 8), (128, 64, 128)])
 def test_plane_steps(n, wall_z):
