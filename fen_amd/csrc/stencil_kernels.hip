@@ -216,6 +216,13 @@ static void grid_blocks(const Box &b, int ty, int kb, int *nbx, int *nby, int *n
     }
 }
 
+// Workgroups of project_checks_kernel, each marching kb planes of 64 x 8 cells.
+constexpr int kCheckPlanes = 8;
+static long checks_blocks(const Box &b, int kb)
+{
+    return (long)((b.nx + 63) / 64) * ((b.ny + 7) / 8) * (b.dim == 3 ? (b.nz + kb - 1) / kb : 1);
+}
+
 // Workgroups of the kernels that write one partial each (the projection),
 // either element type: the partial buffer's size.
 long stencil_blocks(const Box &b)
@@ -228,7 +235,7 @@ long stencil_blocks(const Box &b)
         grid_blocks(b, sh[0], sh[1], &nbx, &nby, &nbz, sh[2]);
         most = std::max(most, (long)nbx * nby * nbz);
     }
-    return most;
+    return std::max(most, checks_blocks(b, kCheckPlanes));
 }
 
 template <class R> void launch_momentum(fen_ctx *c, double dt, double A, double B)
@@ -579,24 +586,31 @@ template <class R> void launch_project(fen_ctx *c, double dt, bool store, R *p_o
     int nbz;
     using SH = Shape<R>;
     grid_blocks(c->box, SH::PTY, SH::PKB, &a.nbx, &a.nby, &nbz, SH::PTXW);
-    const long nblk = (long)a.nbx * a.nby * nbz;
-    if ((size_t)(3 * nblk) > c->n_chk) throw std::runtime_error("partial buffer too small");
+    long nblk = (long)a.nbx * a.nby * nbz;
     const bool sh = c->shift_active;
     const int d3 = c->box.dim == 3;
+    int kb = kCheckPlanes;
+    if (d3 && !store) {
+        // shorter marches (each loads two planes more) where they leave CUs idle
+        while (kb > 2 && checks_blocks(c->box, kb) < 2L * c->num_cu && (size_t)(3 * checks_blocks(c->box, kb / 2)) <= c->n_chk)
+            kb /= 2;
+        a.nbx = (c->nx + 63) / 64;
+        a.nby = (c->ny + 7) / 8;
+        nblk = checks_blocks(c->box, kb);
+    }
+    if ((size_t)(3 * nblk) > c->n_chk) throw std::runtime_error("partial buffer too small");
     const int kid = store ? K_PROJECT : K_CHECKS;
     prof_begin(c, kid);
-    if (d3) {
+    if (d3 && !store) {
+        if (sh) hipLaunchKernelGGL((project_checks_kernel<R, 1>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a, kb);
+        else hipLaunchKernelGGL((project_checks_kernel<R, 0>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a, kb);
+    } else if (d3) {
         const dim3 grid((unsigned)nblk);
-#define FEN_PJ(SH_, ST_)                                                                                            \
-    hipLaunchKernelGGL((project_march_kernel<R, SH_, SH::PTY, SH::PKB, SH::PUN, SH::PPF, SH::POCC, SH::PTXW, ST_>), \
+#define FEN_PJ(SH_)                                                                                            \
+    hipLaunchKernelGGL((project_march_kernel<R, SH_, SH::PTY, SH::PKB, SH::PUN, SH::PPF, SH::POCC, SH::PTXW>), \
                        grid, dim3(SH::PTXW * SH::PTY), 0, c->stream, a)
-        if (store) {
-            if (sh) FEN_PJ(1, 1);
-            else FEN_PJ(0, 1);
-        } else {
-            if (sh) FEN_PJ(1, 0);
-            else FEN_PJ(0, 0);
-        }
+        if (sh) FEN_PJ(1);
+        else FEN_PJ(0);
 #undef FEN_PJ
     } else {
         const dim3 grid((unsigned)a.nbx, (unsigned)a.nby);

@@ -196,8 +196,7 @@ __global__ __launch_bounds__(TX * TY, OCC) void momentum_march_kernel(MomArgs<R>
 // Ring fields: phi, u*, v* (u* and v* need the cell below in i and j for the
 // checks); w* and p are prefetched one plane ahead, w* one plane below is
 // carried in a register.
-// ST == 0: the checks of the projection only; nothing is stored and p is not read.
-template <class R, int SHIFT, int TY, int KB, int UNROLL, int PF = 1, int TX = 64, int ST = 1>
+template <class R, int SHIFT, int TY, int KB, int UNROLL, int PF = 1, int TX = 64>
 struct ProjectMarch {
     static_assert((PF == 1 && (UNROLL == 1 || UNROLL == 3)) || (PF == 2 && UNROLL == 2), "launch shape");
     using S = TileShape<TY, TX>;
@@ -217,7 +216,7 @@ struct ProjectMarch {
         const long g = a.b.g(i, j, k);
         if (active && k + 1 <= kend) {
             wnext = a.ws[g + a.b.gxy];
-            if constexpr (ST) pnext = a.p[g + a.b.gxy];
+            pnext = a.p[g + a.b.gxy];
         }
         if (active) {
             auto L = [&](int f, int di, int dj, int dk) -> double {
@@ -229,8 +228,8 @@ struct ProjectMarch {
                 else return L(0, di, dj, dk);
             };
             auto img = [&](R *f, R v) { march_images(f, a.b, a.img, i, j, k, v, xedge); };
-            project_cell<1, R, decltype(F), decltype(img), ST>(a, i, j, k, F, L(1, 0, 0, 0), L(2, 0, 0, 0), wsc, pc,
-                                                              L(1, -1, 0, 0), L(2, 0, -1, 0), wsm, md, mv, bad, img);
+            project_cell<1>(a, i, j, k, F, L(1, 0, 0, 0), L(2, 0, 0, 0), wsc, pc, L(1, -1, 0, 0), L(2, 0, -1, 0), wsm, md,
+                            mv, bad, img);
         }
         wsm = wsc;
         wsc = wnext;
@@ -270,7 +269,7 @@ struct ProjectMarch {
         if (active) {
             wsm = a.ws[b.g(i, j, k0 - 1)];
             wsc = a.ws[b.g(i, j, k0)];
-            if constexpr (ST) pc = a.p[b.g(i, j, k0)];
+            pc = a.p[b.g(i, j, k0)];
         }
         if constexpr (PF == 2) {
             int sm = 0, sc = 1, sn = 2;
@@ -308,11 +307,83 @@ struct ProjectMarch {
     }
 };
 
-template <class R, int SHIFT, int TY, int KB, int UNROLL, int PF = 1, int OCC = 1, int TX = 64, int ST = 1>
+template <class R, int SHIFT, int TY, int KB, int UNROLL, int PF = 1, int OCC = 1, int TX = 64>
 __global__ __launch_bounds__(TX * TY, OCC) void project_march_kernel(ProjArgs<R> a)
 {
     __shared__ R lds[ring_size<TileShape<TY, TX>, 3>()];
-    ProjectMarch<R, SHIFT, TY, KB, UNROLL, PF, TX, ST>::run(a, lds);
+    ProjectMarch<R, SHIFT, TY, KB, UNROLL, PF, TX>::run(a, lds);
+}
+
+// The checks of a pending step: project_cell without its stores, on columns of
+// cells two rows wide that a thread walks in k, reading x and y neighbours from
+// the caches (no LDS, no barrier) and carrying what plane k needs of k - 1; the
+// loads of plane k + 2 are in flight while plane k is computed.  HBM bounds it,
+// 4 words per cell (the projection's march without its stores -> this: 256^3
+// 158 -> 145 us, 128^3 22 -> 18.4).
+template <class R, int SHIFT> __global__ __launch_bounds__(256) void project_checks_kernel(ProjArgs<R> a, int kb)
+{
+    constexpr int TX = 64, TY = 4, NJ = 2;
+    const Box &b = a.b;
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int bx = bid % a.nbx, rest = bid / a.nbx, by = rest % a.nby, bz = rest / a.nby;
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    const int i = bx * TX + tx + 1, j = (by * TY + ty) * NJ + 1, k0 = bz * kb + 1, kend = min(k0 + kb - 1, b.nz);
+    const double s = SHIFT ? a.shift[0] : 0.0;
+    int off[NJ + 2];   // rows j - 1 .. j + NJ; past the grid clamped to its last (values no active cell uses)
+#pragma unroll
+    for (int r = 0; r < NJ + 2; r++) off[r] = min(i, b.nx) + (int)b.gx * min(j - 1 + r, b.ny + 1);
+    struct Plane {
+        R f[NJ + 2], fe[NJ], fw[NJ], u[NJ], uw[NJ], v[NJ + 1], w[NJ];
+    };
+    // plane k; of the one after the march's last only phi is read
+    auto load = [&](Plane &p, int k) {
+        const long base = (long)k * b.gxy;
+        const R *f = a.phi + base, *u = a.us + base, *v = a.vs + base, *w = a.ws + base;
+#pragma unroll
+        for (int r = 0; r < NJ + 2; r++) p.f[r] = f[off[r]];
+        if (k > kend) return;
+#pragma unroll
+        for (int r = 0; r < NJ + 1; r++) p.v[r] = v[off[r]];
+#pragma unroll
+        for (int y = 0; y < NJ; y++) {
+            p.fe[y] = f[off[y + 1] + 1];
+            p.fw[y] = f[off[y + 1] - 1];
+            p.u[y] = u[off[y + 1]];
+            p.uw[y] = u[off[y + 1] - 1];
+            p.w[y] = w[off[y + 1]];
+        }
+    };
+    R fb[NJ], wb[NJ];   // phi and w* of plane k - 1
+#pragma unroll
+    for (int y = 0; y < NJ; y++) {
+        fb[y] = a.phi[off[y + 1] + (long)(k0 - 1) * b.gxy];
+        wb[y] = a.ws[off[y + 1] + (long)(k0 - 1) * b.gxy];
+    }
+    Plane c, n{}, x{};
+    load(c, k0);
+    load(n, k0 + 1);
+    double md = -HUGE_VAL, mv = 0.0, bad = 0.0;
+    for (int k = k0; k <= kend; k++) {
+        if (k < kend) load(x, k + 2);
+#pragma unroll
+        for (int y = 0; y < NJ; y++) {
+            if (i <= b.nx && j + y <= b.ny) {
+                auto F = [&](int di, int dj, int dk) {
+                    const R f = di > 0 ? c.fe[y] : di < 0 ? c.fw[y] : dk > 0 ? n.f[y + 1] : dk < 0 ? fb[y] : c.f[y + 1 + dj];
+                    if constexpr (SHIFT) return (double)f - s;
+                    else return (double)f;
+                };
+                auto none = [](R *, R) {};
+                project_cell<1, R, decltype(F), decltype(none), 0>(a, i, j + y, k, F, c.u[y], c.v[y + 1], c.w[y], 0.0,
+                                                                   c.uw[y], c.v[y], wb[y], md, mv, bad, none);
+            }
+            fb[y] = c.f[y + 1];
+            wb[y] = c.w[y];
+        }
+        c = n;
+        n = x;
+    }
+    block_max3<256>(md, mv, bad, a.part, bid);
 }
 
 // ------------------------------------------------- projection + momentum

@@ -27,6 +27,7 @@ _PATTERNS = [
     (r"project_momentum_kernel|step_kernel_2d", "project_momentum"),
     (r"wall_state_kernel", "wall_state"),
     (r"(?<!adj_)momentum_march_kernel|momentum_kernel_2d", "momentum"),
+    (r"project_checks_kernel", "project_checks"),
     (r"project_march_kernel|project_kernel_2d", "project"),
     (r"div_r2c_kernel|plane_fwd_kernel", "div_r2c"),
     (r"y_kernel<(?:double|float), \d+, -1, 0(?:, \d+)?>", "y_fwd"),
