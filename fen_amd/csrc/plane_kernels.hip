@@ -238,8 +238,9 @@ bool plane_pass(const fen_ctx *c)
     // slower than its passes (32 x 16 x 32: 25.7 -> 32 us per step); up to four
     // waves it is faster at every nz; eight waves need planes for half the CUs
     // (128 x 64, FP64: 64 planes 47.1 -> 47.7, 128 planes 70 -> 64.6, 512
-    // planes 209 -> 191); with sixteen (128 x 128) one workgroup fills a CU, and
-    // 128 planes leave the others idle (128^3: 93 -> 97; 256 planes 201 -> 194).
+    // planes 209 -> 191); with sixteen (128 x 128) one workgroup fills a CU and few
+    // planes leave the others idle (32 planes 48 -> 68; 128: the passes 67 us
+    // either way; 256: 201 -> 194).
     if (c->dim != 3 || (c->solver != FEN_SOLVER_PPP && c->solver != FEN_SOLVER_PPN)) return false;
     // One block sum per plane: at most the 32768 that the allocation-free
     // solve's fixed scratch holds, so that it takes every grid it would without.
