@@ -160,18 +160,19 @@ struct AxisCopies {
     __host__ __device__ bool any() const { return x || y || z; }
 };
 
-// The ghosted indices that hold row index J (interior 1..n) of such an axis:
-// J itself, and the ghost rows 0 and n + 1 that copy it.  Returns how many.
-__device__ __forceinline__ int copy_rows(int J, int n, int mode, int (&d)[3])
+// The ghosted indices that hold row index J (interior 1..n) of an axis whose
+// faces have these modes: J itself, and the ghost rows 0 (face lo) and n + 1
+// (face hi) that copy it.  Returns how many.
+__device__ __forceinline__ int copy_rows(int J, int n, int lo, int hi, int (&d)[3])
 {
     int m = 0;
     d[m++] = J;
-    if (mode != COPY_NONE) {
-        if (J == (mode == COPY_PERIODIC ? n : 1)) d[m++] = 0;
-        if (J == (mode == COPY_PERIODIC ? 1 : n)) d[m++] = n + 1;
-    }
+    if (lo != COPY_NONE && J == (lo == COPY_PERIODIC ? n : 1)) d[m++] = 0;
+    if (hi != COPY_NONE && J == (hi == COPY_PERIODIC ? 1 : n)) d[m++] = n + 1;
     return m;
 }
+
+__device__ __forceinline__ int copy_rows(int J, int n, int mode, int (&d)[3]) { return copy_rows(J, n, mode, mode, d); }
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X; this
 // renumbering gives every XCD one contiguous range of the grid (a k-slab),

@@ -44,10 +44,10 @@ __device__ __forceinline__ Surf cell_surface(double nx, double ny, double lx, do
 }
 
 // The MF fields' ghosts are copies (periodic images, or the neighbour at a
-// Neumann wall; src/volume_of_fluid.f90:54-219, src/multiphase.f90:44-120).
-// Rows (columns) that hold the value of interior row J, ghosts included.
+// Neumann wall; src/volume_of_fluid.f90:54-219, src/multiphase.f90:44-120), by
+// each face's own rule: an axis may have one periodic face and one wall.
 struct MFCopies {
-    int x, y;   // COPY_PERIODIC or COPY_MIRROR
+    int face[4];   // COPY_PERIODIC or COPY_MIRROR: left, right, bottom, top
 };
 
 // Stores n fields' values of cell (i, j) and the ghosts that copy them.
@@ -56,7 +56,7 @@ __device__ __forceinline__ void put_copies(const Box &b, const MFCopies &m, int 
                                            const double (&v)[NF])
 {
     int id[3], jd[3];
-    const int ni = copy_rows(i, b.nx, m.x, id), nj = copy_rows(j, b.ny, m.y, jd);
+    const int ni = copy_rows(i, b.nx, m.face[0], m.face[1], id), nj = copy_rows(j, b.ny, m.face[2], m.face[3], jd);
     for (int y = 0; y < nj; y++)
         for (int x = 0; x < ni; x++) {
             const long g = b.g(id[x], jd[y], 1);
@@ -356,7 +356,9 @@ dim3 cell_grid(const Box &b) { return dim3((unsigned)((b.nx + kBX - 1) / kBX), (
 
 MFCopies mf_copies(const fen_ctx *c)
 {
-    return MFCopies{c->periodic[0] ? COPY_PERIODIC : COPY_MIRROR, c->periodic[1] ? COPY_PERIODIC : COPY_MIRROR};
+    MFCopies m{};
+    for (int f = 0; f < 4; f++) m.face[f] = c->bc_phys[f] == FEN_BC_PERIODIC ? COPY_PERIODIC : COPY_MIRROR;
+    return m;
 }
 
 void vof_reconstruct(fen_ctx *c, const double *vof)
