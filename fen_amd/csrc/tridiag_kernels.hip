@@ -7,12 +7,14 @@
 // Thomas sweep's two recurrences,
 //   d_k = (r_k - a d_{k-1}) f_k,  f_k = 1 / (b_k - a c1_{k-1}),  c1_k = a f_k,
 //   x_k = d_k - c1_k x_{k+1},
-// are first-order and linear in the carried value, so a column is cut into
-// chunks of M rows, one thread each: every thread runs its chunk from a zero
-// carry, keeping only the end value and the product of the multipliers; the
-// chunks' (product, end) pairs go through LDS, each thread folds those before
-// (behind) its own into its carry, and runs the chunk again from it.  The
-// multipliers are at most 1 in magnitude, so the products only shrink.
+// (2-D: divided by the pivot) are first-order and linear in the carried value,
+// so a column is cut into chunks of M rows, one thread each: every thread runs
+// its chunk from a zero carry, keeping only the end value and the product of
+// the multipliers; the chunks' (product, end) pairs go through LDS, each thread
+// folds those before (behind) its own into its carry, and runs the chunk again
+// from it.  The multipliers are at most 1 in magnitude, so the products only
+// shrink.
+#include <cmath>
 #include <stdexcept>
 
 #include "fen_internal.hpp"
@@ -26,6 +28,8 @@ __host__ __device__ __forceinline__ double2 t_load(float2 v) { return double2{(d
 __host__ __device__ __forceinline__ double t_load(double v) { return v; }
 __device__ __forceinline__ double2 t_mul(double2 a, double f) { return double2{a.x * f, a.y * f}; }
 __device__ __forceinline__ double t_mul(double a, double f) { return a * f; }
+__device__ __forceinline__ double2 t_div(double2 a, double f) { return double2{a.x / f, a.y / f}; }
+__device__ __forceinline__ double t_div(double a, double f) { return a / f; }
 __device__ __forceinline__ double2 t_sub(double2 a, double2 b) { return double2{a.x - b.x, a.y - b.y}; }
 __device__ __forceinline__ double t_sub(double a, double b) { return a - b; }
 __device__ __forceinline__ double2 t_add(double2 a, double2 b) { return double2{a.x + b.x, a.y + b.y}; }
@@ -60,15 +64,19 @@ struct ChunkArgs {
 //
 // The workgroup of the singular column (mwx + mwy = 0: column 0) runs its
 // chunks one after the other instead, in the sweep's own order: whether the
-// last pivot of that column is exactly zero, and what round-off leaves when
-// it is not, is then the sweep's own.
+// last pivot of that column is exactly zero is then the sweep's own, and when
+// it is not, so is what round-off leaves (but for the last row's quotient,
+// here a product with the reciprocal as on every other row).
 //
 // D2: the 2-D solvers (pn, nn), a few hundred contiguous columns bound by the
 // latency of one sweep: c1 is read (formed once per context, by divisions, so
 // the singular column's is exactly -1 and its last pivot exactly 0, and the
-// column needs no order of its own), which leaves the divisions of a chunk
-// independent.  One wave per column with the sweep on one or two of its lanes
-// took 70 us at 512 rows and 29 at 200, now 9 and 5.4.
+// column needs no order of its own), and its rows are divided by their pivots,
+// as the 2-D sweep's: all rows of the singular column have the same pivot, and
+// the error of one rounded reciprocal would sum up over them (700 rows at a
+// spacing that is no power of two: 11 times the round-off).  One wave per
+// column with the sweep on one or two of its lanes took 70 us at 512 rows and
+// 29 at 200, now 9.2 and 5.9 (with reciprocals 8.5 and 5.6).
 template <class E, int M, int CW, int NT, int OCC, int D2>
 __global__ __launch_bounds__(NT, OCC) void thomas_chunk_kernel(ChunkArgs p)
 {
@@ -90,7 +98,7 @@ __global__ __launch_bounds__(NT, OCC) void thomas_chunk_kernel(ChunkArgs p)
         r[u] = k0 + u < n ? v : A{};
     }
     const double mx = p.mwx[o], my = D2 ? 0.0 : p.mwy[q], a0 = ch > 0 ? p.a : 0.0;
-    double f[M], g[D2 ? M : 1];   // 1/pivot; D2: the stored c1
+    double f[M], g[D2 ? M : 1];   // 1/pivot; D2: the pivot, and the stored c1
     double cp = 0.0;
     if constexpr (D2) {
         const double *c1 = p.c1 + tt * n;
@@ -100,6 +108,10 @@ __global__ __launch_bounds__(NT, OCC) void thomas_chunk_kernel(ChunkArgs p)
     } else if (ch > 0) {
         cp = p.c1[(long)(ch - 1) * p.ncol + tt];
     }
+    auto row = [](A x, double by) {
+        if constexpr (D2) return t_div(x, by);
+        else return t_mul(x, by);
+    };
     double P = 1.0;
     A e{};
 #pragma unroll
@@ -108,15 +120,22 @@ __global__ __launch_bounds__(NT, OCC) void thomas_chunk_kernel(ChunkArgs p)
         const double b = (u == 0 && k == 0) ? p.b0 : (k == n - 1 ? p.bn : p.bi);
         const double ak = u == 0 ? a0 : p.a;
         const double piv = ((b + mx) + my) - ak * cp;
-        f[u] = (k < n && piv != 0.0) ? 1.0 / piv : 0.0;   // a zero last pivot gives 0; rows past the end too
-        cp = D2 ? g[D2 ? u : 0] : p.a * f[u];
-        e = t_mul(t_sub(r[u], t_mul(e, ak)), f[u]);
-        P = -(ak * f[u]) * P;
+        // a zero last pivot gives 0; rows past the end too
+        if constexpr (D2) {
+            f[u] = (k < n && piv != 0.0) ? piv : HUGE_VAL;
+            cp = g[u];
+            P = -g[u] * P;   // a / pivot (the first row's enters no carry, and the last's)
+        } else {
+            f[u] = (k < n && piv != 0.0) ? 1.0 / piv : 0.0;
+            cp = p.a * f[u];
+            P = -(ak * f[u]) * P;
+        }
+        e = row(t_sub(r[u], t_mul(e, ak)), f[u]);
     }
     auto forward = [&](A d) {
 #pragma unroll
         for (int u = 0; u < M; u++) {
-            d = t_mul(t_sub(r[u], t_mul(d, u == 0 ? a0 : p.a)), f[u]);
+            d = row(t_sub(r[u], t_mul(d, u == 0 ? a0 : p.a)), f[u]);
             r[u] = d;
         }
         return d;
