@@ -168,8 +168,20 @@ __device__ __forceinline__ void fft_lds(C *line, int t, const C *tw)
 // the results are bitwise equal.  `line` is this thread's line in LDS
 // (padded indexing); all threads of the block must call this (barriers),
 // and on return every read of `line` is complete.  C may be a CPair of the
-// twiddles' type TW (two lines per thread).
-template <int N, int NS, int SIGN, typename C, typename TW>
+// twiddles' type TW (two lines per thread).  WAVE: the threads of the line are
+// in one wave, which calls this by itself: its LDS accesses take place in order
+// and need no barrier.
+template <int WAVE> __device__ __forceinline__ void fft_sync()
+{
+    if constexpr (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+template <int N, int NS, int SIGN, int WAVE, typename C, typename TW>
 __device__ __forceinline__ void fft_regs_stages(C (&v)[8], C *line, int t, const TW *tw)
 {
     constexpr int REM = N / NS;
@@ -185,7 +197,7 @@ __device__ __forceinline__ void fft_regs_stages(C (&v)[8], C *line, int t, const
 #pragma unroll
             for (int r = 0; r < R; r++) v[m * R + r] = line[lds_pad(j + r * (N / R))];
         }
-        __syncthreads();   // every read of this stage precedes any write below (in place)
+        fft_sync<WAVE>();   // every read of this stage precedes any write below (in place)
     }
 #pragma unroll
     for (int m = 0; m < NB; m++) {
@@ -219,16 +231,16 @@ __device__ __forceinline__ void fft_regs_stages(C (&v)[8], C *line, int t, const
 #pragma unroll
             for (int r = 0; r < R; r++) line[lds_pad(base + r * NS)] = v[m * R + r];
         }
-        __syncthreads();
-        fft_regs_stages<N, NS * R, SIGN>(v, line, t, tw);
+        fft_sync<WAVE>();
+        fft_regs_stages<N, NS * R, SIGN, WAVE>(v, line, t, tw);
     }
 }
 
-template <int N, int SIGN, typename C, typename TW>
+template <int N, int SIGN, int WAVE = 0, typename C, typename TW>
 __device__ __forceinline__ void fft_regs(C (&v)[8], C *line, int t, const TW *tw)
 {
-    fft_regs_stages<N, 1, SIGN>(v, line, t, tw);
-    if constexpr (N > 8) __syncthreads();   // the last stage's LDS reads are done
+    fft_regs_stages<N, 1, SIGN, WAVE>(v, line, t, tw);
+    if constexpr (N > 8) fft_sync<WAVE>();   // the last stage's LDS reads are done
 }
 
 // Copies the twiddle table W_N^m (m < N) into LDS.

@@ -6,10 +6,16 @@
 //
 // Forward: row pairs as complex lines through the x FFT; each kx column is
 // unpacked from the packed lines in LDS straight into the y FFT's registers.
-// Columns 0 and NX/2 are real sequences in y, so they share one complex line
-// (NX/2 columns in all, as many threads as for the rows).  Backward: the same
-// steps in reverse.  Half spectrum [kx][k][j], as the separate passes' (their
-// arithmetic, but for the shared line: rounding apart).
+// Backward: the same steps in reverse.  Half spectrum [kx][k][j] and
+// arithmetic are the separate passes'.
+//
+// There are NX/2 + 1 columns and threads for NX/2: the last one waits in an LDS
+// line of its own until the first wave has transformed its other columns.  (The
+// columns 0 and NX/2 are real sequences in y and could share one complex line,
+// but column NX/2 then takes on the round-off of column 0, which is far larger in
+// a solution: up to 1.39 times the error of a solve, at 16 x 64 x 32.  A line of
+// its own costs 32 x 128 x 32 1.6 us per step, the others at most 0.6; as NY/8
+// more threads it cost 128 x 64 x 128 14, one workgroup per CU instead of two.)
 //
 // What bounds it: the latency of one workgroup's chain, load to store; the
 // separate passes pay it twice each way, with a launch between.  Us per step,
@@ -54,7 +60,7 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void plane_fwd_kernel(Pl
 {
     using C = typename Cplx<R>::type;
     constexpr int TX = NX / 8, TY = NY / 8, LX = lds_line<NX>(), LY = lds_line<NY>();
-    __shared__ C buf[plane_lds<NX, NY>()];
+    __shared__ C buf[plane_lds<NX, NY>()], last[LY];   // last: column NX/2
     __shared__ C twx[NX], twy[NY];
     load_twiddles<NX>(twx, a.twx);   // first read after the first stage's barrier
     load_twiddles<NY>(twy, a.twy);
@@ -80,41 +86,38 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void plane_fwd_kernel(Pl
 #pragma unroll
     for (int q = 0; q < 8; q++) line[lds_pad(t + q * TX)] = v[q];
     __syncthreads();
-    // column c: rows 2l, 2l + 1 of every pair at kx = c; column 0 also NX/2
+    // column c: rows 2l, 2l + 1 of every pair at kx = c
     const int c = threadIdx.x / TY, s = threadIdx.x % TY;
     const R half = R(0.5), postx = (R)a.postx;
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const int j = s + q * TY;
+    auto unpack = [&](int kx, int j) {
         const C *ln = buf + (j >> 1) * LX;
-        const C zk = ln[lds_pad(c)], zn = ln[lds_pad(c == 0 ? NX / 2 : NX - c)];
+        const C zk = ln[lds_pad(kx)], zn = ln[lds_pad((NX - kx) & (NX - 1))];
         C x;
-        if (c == 0) x = (j & 1) ? C{zk.y, zn.y} : C{zk.x, zn.x};
-        else if (j & 1) x = C{(zk.y + zn.y) * half, (zn.x - zk.x) * half};
+        if (j & 1) x = C{(zk.y + zn.y) * half, (zn.x - zk.x) * half};
         else x = C{(zk.x + zn.x) * half, (zk.y - zn.y) * half};
-        v[q] = C{x.x * postx, x.y * postx};
-    }
-    __syncthreads();   // every read of the packed lines precedes the y stages' writes
-    C *col = buf + c * LY;
-    fft_regs<NY, -1>(v, col, s, twy);
-    if (c == 0) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) col[lds_pad(s + q * TY)] = v[q];
-    }
-    __syncthreads();
-    auto put = [&](int kx, int ky, C x) {
-        a.spec[((long)kx * a.nz + (k - 1)) * NY + ky] = C{(R)((double)x.x * a.posty), (R)((double)x.y * a.posty)};
+        return C{x.x * postx, x.y * postx};
     };
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const int ky = s + q * TY;
-        if (c == 0) {
-            const C zk = v[q], zn = col[lds_pad((NY - ky) & (NY - 1))];
-            put(0, ky, C{(zk.x + zn.x) * half, (zk.y - zn.y) * half});
-            put(NX / 2, ky, C{(zk.y + zn.y) * half, (zn.x - zk.x) * half});
-        } else {
-            put(c, ky, v[q]);
-        }
+    for (int q = 0; q < 8; q++) v[q] = unpack(c, s + q * TY);
+    if (c == 0) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) last[lds_pad(s + q * TY)] = unpack(NX / 2, s + q * TY);
+    }
+    __syncthreads();   // every read of the packed lines precedes the y stages' writes
+    auto put = [&](int kx) {
+        C *out = a.spec + ((long)kx * a.nz + (k - 1)) * NY;
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            out[s + q * TY] = C{(R)((double)v[q].x * a.posty), (R)((double)v[q].y * a.posty)};
+    };
+    fft_regs<NY, -1>(v, buf + c * LY, s, twy);
+    put(c);
+    if (c == 0) {   // the threads of column 0, all in the first wave
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = last[lds_pad(s + q * TY)];
+        fft_sync<1>();
+        fft_regs<NY, -1, 1>(v, last, s, twy);
+        put(NX / 2);
     }
 }
 
@@ -123,38 +126,40 @@ __global__ __launch_bounds__((plane_threads<NX, NY>())) void plane_bwd_kernel(Pl
 {
     using C = typename Cplx<R>::type;
     constexpr int TX = NX / 8, TY = NY / 8, LX = lds_line<NX>(), LY = lds_line<NY>(), NT = plane_threads<NX, NY>();
-    __shared__ C buf[plane_lds<NX, NY>()];
+    __shared__ C buf[plane_lds<NX, NY>()], last[LY];   // last: column NX/2
     __shared__ C twx[NX], twy[NY];
     load_twiddles<NX>(twx, a.twx);
     load_twiddles<NY>(twy, a.twy);
     const int k = blockIdx.x;
     const int c = threadIdx.x / TY, s = threadIdx.x % TY;
     const C *in = a.spec + ((long)c * a.nz + k) * NY;
-    C v[8];
+    C v[8], vl[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) v[q] = in[s + q * TY];
-    if (c == 0) {   // columns 0 and NX/2 (real in y) as one line
-        const C *in2 = a.spec + ((long)(NX / 2) * a.nz + k) * NY;
+    if (c == 0) {
+        const C *il = a.spec + ((long)(NX / 2) * a.nz + k) * NY;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const C x = in2[s + q * TY];
-            v[q] = C{v[q].x - x.y, v[q].y + x.x};
-        }
+        for (int q = 0; q < 8; q++) vl[q] = il[s + q * TY];
     }
     C *col = buf + c * LY;
     fft_regs<NY, 1>(v, col, s, twy);
 #pragma unroll
     for (int q = 0; q < 8; q++) col[lds_pad(s + q * TY)] = v[q];
+    if (c == 0) {   // the threads of column 0, all in the first wave
+        fft_regs<NY, 1, 1>(vl, last, s, twy);
+#pragma unroll
+        for (int q = 0; q < 8; q++) last[lds_pad(s + q * TY)] = vl[q];
+    }
     __syncthreads();
     const int l = threadIdx.x / TX, t = threadIdx.x % TX;
     const int r0 = lds_pad(2 * l), r1 = lds_pad(2 * l + 1);
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         const int kx = t + q * TX;
-        const int m = kx == NX / 2 ? 0 : (kx < NX / 2 ? kx : NX - kx);
-        const C x1 = buf[m * LY + r0], x2 = buf[m * LY + r1];
-        if (kx == 0) v[q] = C{x1.x, x2.x};
-        else if (kx == NX / 2) v[q] = C{x1.y, x2.y};
+        const int m = kx <= NX / 2 ? kx : NX - kx;
+        const C *cl = m == NX / 2 ? last : buf + m * LY;
+        const C x1 = cl[r0], x2 = cl[r1];
+        if (kx == 0 || kx == NX / 2) v[q] = C{x1.x, x2.x};   // Im of bins 0 and NX/2 ignored
         else if (kx < NX / 2) v[q] = C{x1.x - x2.y, x1.y + x2.x};
         else v[q] = C{x1.x + x2.y, x2.x - x1.y};
     }
