@@ -8,9 +8,8 @@
 // 5.1 ms, FP32 21.3 -> 4.5; FP32 from the host 19.6 -> 3.7.  FP64 from the host
 // stays with hipMemcpy (4.6 ms, staged 4.7), and so does FP64 into an array that
 // the runtime knows (pinned by the caller, managed): 2.4 ms, staged 4.8.  More
-// host threads (2 to 8)
-// brought 3.5 ms on an idle host and 5 to 7 beside a spinning OpenMP pool, so
-// the calling thread does it alone.
+// host threads (2 to 8) brought 3.5 ms on an idle host and 5 to 7 beside a
+// spinning OpenMP pool, so the calling thread does it alone.
 //
 // The buffers belong to the process: allocated by the first large copy, shared
 // by every context (a copy that finds them taken goes the plain way) and freed
@@ -89,6 +88,24 @@ void from_host(void *dst, const double *src, size_t n, size_t es)
     }
 }
 
+// The stream's device is current while this lives: the copy's events have to
+// belong to it, and the caller may have another one current.
+struct OnDeviceOf {
+    int before = 0;
+    bool ok = false, changed = false;
+    explicit OnDeviceOf(hipStream_t s)
+    {
+        hipDevice_t dev = 0;
+        ok = hipGetDevice(&before) == hipSuccess && hipStreamGetDevice(s, &dev) == hipSuccess;
+        if (ok && dev != before) ok = changed = hipSetDevice(dev) == hipSuccess;
+        if (!ok) (void)hipGetLastError();
+    }
+    ~OnDeviceOf()
+    {
+        if (changed) (void)hipSetDevice(before);
+    }
+};
+
 // The copy through the two buffers, one piece on the bus while the other is on
 // the host; everything it queued is done when it returns or throws.
 struct Pipe {
@@ -152,6 +169,8 @@ bool staged(hipStream_t stream, void *devp, double *host, size_t n, size_t es, b
     Staging &s = staging();
     std::unique_lock<std::mutex> lock(s.busy, std::try_to_lock);
     if (!lock.owns_lock() || !s.allocate()) return false;
+    OnDeviceOf device(stream);
+    if (!device.ok) return false;
     Pipe(stream).run(s.piece, static_cast<char *>(devp), host, n, es, out);
     return true;
 }
