@@ -396,8 +396,7 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
     double *dvo[3] = {t->work + 4 * n, t->work + 5 * n, t->work + 6 * n};
     double *ub2[3] = {t->work + 7 * n, t->work + 8 * n, t->work + 9 * n};
     double *dvo2[3] = {t->work + 10 * n, t->work + 11 * n, t->work + 12 * n};
-    for (int d = 0; d < 3; d++)
-        copy_to_device(c->stream, ub[d], seed[d], n, sizeof(double));
+    for (int d = 0; d < 3; d++) queue_to_device(c->stream, ub[d], seed[d], n);
     FEN_HIP_CHECK(hipMemsetAsync(pb, 0, 4 * n * sizeof(double), c->stream));   // pb and dvo
     const double dt_o_saved = c->dt_o;
     c->dt_o = t->dt_o;
@@ -410,9 +409,8 @@ void adjoint_backward(fen_ctx *c, const double *seed[3], double *grad[3], double
         states_fp64(c, t->dt, len, t->seg.data());
         for (int s = len - 1; s >= 0; s--) adjoint_step(c, t, t->seg[s], ub, pb, dvo, ub2, dvo2);
     }
-    for (int d = 0; d < 3; d++)
-        copy_to_host(c->stream, grad[d], ub[d], n, sizeof(double));
-    if (grad_p) copy_to_host(c->stream, grad_p, pb, n, sizeof(double));
+    for (int d = 0; d < 3; d++) queue_to_host(c->stream, grad[d], ub[d], n);
+    if (grad_p) queue_to_host(c->stream, grad_p, pb, n);
     load_state(c, t->final_state);   // leave the context at the end of the recorded run
     c->dt_o = dt_o_saved;
     c->checks_valid = false;

@@ -1280,10 +1280,11 @@ int fen_add_advection(fen_ctx *c, double *rx, double *ry, double *rz)
         double *r[3] = {as<double>(c->d_us[0]), as<double>(c->d_us[1]), as<double>(c->d_us[2])};
         double *h[3] = {rx, ry, rz};
         const int nd = c->dim == 3 ? 3 : 2;
-        for (int d = 0; d < nd; d++) copy_in(c, r[d], h[d], c->n_int);
+        for (int d = 0; d < nd; d++) fen::queue_to_device(c->stream, r[d], h[d], c->n_int);
         fen::launch_advection_only(c, r[0], r[1], r[2]);
         fen::prof_end(c, fen::K_MOMENTUM, 0.0);
-        for (int d = 0; d < nd; d++) copy_out(c, h[d], r[d], c->n_int);
+        for (int d = 0; d < nd; d++) fen::queue_to_host(c->stream, h[d], r[d], c->n_int);
+        sync(c);
     });
     return FEN_OK;
 }

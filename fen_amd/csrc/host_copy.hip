@@ -187,14 +187,25 @@ void host_copy_user(int change)
     s.release();
 }
 
+void queue_to_host(hipStream_t stream, double *dst, const double *src, size_t n)
+{
+    if (staged(stream, const_cast<double *>(src), dst, n, sizeof(double), true)) return;
+    check(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, stream));
+}
+
+void queue_to_device(hipStream_t stream, double *dst, const double *src, size_t n)
+{
+    check(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, stream));
+}
+
 void copy_to_host(hipStream_t stream, double *dst, const void *src, size_t n, size_t es)
 {
-    if (staged(stream, const_cast<void *>(src), dst, n, es, true)) return;
     if (es == sizeof(double)) {
-        check(hipMemcpyAsync(dst, src, n * es, hipMemcpyDeviceToHost, stream));
+        queue_to_host(stream, dst, static_cast<const double *>(src), n);
         check(hipStreamSynchronize(stream));
         return;
     }
+    if (staged(stream, const_cast<void *>(src), dst, n, es, true)) return;
     std::vector<float> h(n);
     check(hipMemcpyAsync(h.data(), src, n * es, hipMemcpyDeviceToHost, stream));
     check(hipStreamSynchronize(stream));
@@ -204,7 +215,7 @@ void copy_to_host(hipStream_t stream, double *dst, const void *src, size_t n, si
 void copy_to_device(hipStream_t stream, void *dst, const double *src, size_t n, size_t es)
 {
     if (es == sizeof(double)) {
-        check(hipMemcpyAsync(dst, src, n * es, hipMemcpyHostToDevice, stream));
+        queue_to_device(stream, static_cast<double *>(dst), src, n);
         check(hipStreamSynchronize(stream));
         return;
     }
