@@ -1,8 +1,8 @@
 """Steps replayed from the captured HIP graph equal eager steps to the bit.
 
 Grids whose steps end pending never reach the graph, so fusion is off in both
-arms (FEN_FUSED_RUN=0), but for the Inflow/Outflow grids, which take the graph
-as they are.  Between replays the scalars and PHI are read: a read turns the
+arms (FEN_FUSED_RUN=0), but for the 2-D Inflow/Outflow grid, whose steps do not
+(phi is fixed at its Outflow face) and which takes the graph as it is.  Between replays the scalars and PHI are read: a read turns the
 step's block sums of the mean and its unread checks into numbers, and the next
 replay has to leave both pending again."""
 import numpy as np
@@ -27,7 +27,7 @@ RUNS = [(name, 0) for name in CASES] + [(name, FP32_REFINE) for name in ("pp", "
 def test_replays_between_reads(name, precision, monkeypatch):
     print("step graph", name, precision, flush=True)
     case = CASES[name]()
-    if "inflow" in name:
+    if name == "pn inflow":
         monkeypatch.delenv("FEN_FUSED_RUN", raising=False)
     else:
         monkeypatch.setenv("FEN_FUSED_RUN", "0")
