@@ -679,11 +679,16 @@ static unsigned row_blocks(long nrows, int N, int nt = kNB)
 }
 
 // Grids whose rows would fill fewer than half the CUs with 256-thread
-// workgroups take one wave per workgroup (256 x 200 nn: x DCT-II 11.6 -> 9.9
-// us, DCT-III 6.8 -> 6.0).
+// workgroups take one wave per workgroup: 256 x 256 nn 28.7 -> 26.5 us per step,
+// 256 x 1500 50.5 -> 48.0, 32 x 128 x 20 nnn 51.7 -> 47.2.  A wave of
+// two 512-point rows writes runs of 16 bytes; where the rows of a 2-D grid are
+// many, larger workgroups are faster: 512 x 128 nn 29.1 -> 28.2, 512 x 300 32.8 ->
+// 32.2, but 512 x 384 34.0 -> 35.3, 512 x 1000 48.2 -> 53.2 (in 3-D not: 512 x 16 x
+// 30 nnn 59.4 -> 58.4).
 static bool one_wave(const fen_ctx *c, long nrows, int N)
 {
-    return N <= 512 && (long)row_blocks(nrows, N) < c->num_cu / 2;
+    const int share = N == 512 && c->box.dim == 2 ? 6 : 2;   // of the CUs
+    return N <= 512 && (long)row_blocks(nrows, N) < c->num_cu / share;
 }
 
 template <int N, int SRC, int D3, int MKL> static void launch_dct2_pairs(const fen_ctx *c, const DctArgs &a)

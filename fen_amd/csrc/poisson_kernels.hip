@@ -558,14 +558,33 @@ template <class R> using CplxT = typename Cplx<R>::type;
 // lines).  x passes at N = 512 run 512 threads: 16 rows per workgroup, so each
 // access to a kx plane of the spectrum covers 256 contiguous bytes instead of
 // 128.  Where 256-thread workgroups would leave most of the chip idle (fewer
-// than one for every other CU) one wave each takes their place: the transform's barriers
-// then cost nothing and the lines spread over four times as many CUs.
-// (32^3: div_r2c 7.5 -> 5.7 us, z 5.2 -> 4.2, y 3.5 -> 3.0; a step 35.1 ->
-// 30.9; 128^2: y solve 6.5 -> 5.5, a step 40.5 -> 38.1.)
+// than one for every other CU) one wave each takes their place: the transform's
+// barriers then cost nothing and the lines spread over four times as many CUs.
+// Us per step with larger workgroups -> one wave in the x passes: 32 x 32 x 64
+// 23.1 -> 21.2 (FP32), 16 x 16 x 512 44.0 -> 40.3, 512 x 16 x 8 35.6 -> 29.5, 2-D
+// 512 x 256 29.8 -> 25.6, 512 x 512 33.4 -> 32.3; in the y passes: 16 x 16 x 16
+// 26.1 -> 24.6, 512 x 32 x 16 40.2 -> 37.6, 2-D 512 x 256 27.2 -> 25.6.
+static bool few_blocks(const fen_ctx *c, int n, long lines, double share = 0.5)
+{
+    return n <= 512 && (double)(lines * (n / 8)) < kBlock * share * c->num_cu;
+}
 static int line_threads(const fen_ctx *c, int n, long lines, bool x_pass)
 {
-    if (n <= 512 && lines * (n / 8) < (long)kBlock * (c->num_cu / 2)) return 64;
+    if (few_blocks(c, n, lines)) return 64;
     return x_pass && n == 512 ? 512 : kBlock;
+}
+// The z pass, whose lines are strided: a wave of 512/nz lines reads runs of as
+// many values per k row.  Short runs cost more than the barriers once there is
+// enough work, so the share of the chip up to which one wave is taken falls with
+// them (FP64 below 64 bytes, FP32 below 16).  Larger workgroups -> one wave, us
+// per step: FP64, nz = 512: 16 x 8 32.0 -> 31.8, 16 x 16 39.4 -> 40.4, 64 x 8 39.2
+// -> 42.5; nz = 256: 16 x 16 31.4 -> 30.4, 16 x 32 the same, 32 x 32 37.0 -> 38.9;
+// nz = 128: 16 x 32 30.9 -> 29.8, 32 x 64 the same.  FP32, nz = 512: 16 x 16 36.8 ->
+// 35.7, 32 x 16 39.5 -> 40.5; nz = 256: 16 x 16 31.0 -> 28.6, 32 x 32 the same.
+template <class R> static bool z_one_wave(const fen_ctx *c)
+{
+    const double run = 512.0 / c->nz;
+    return few_blocks(c, c->nz, (long)c->ny * c->hx, 0.5 * std::min(1.0, run * 2.0 / sizeof(R)));
 }
 static int x_pass_threads(const fen_ctx *c) { return line_threads(c, c->nx, ((long)c->ny * c->nz + 1) / 2, true); }
 
@@ -708,8 +727,8 @@ template <class R> void launch_z_solve(fen_ctx *c, double inv_n)
     // so every k row of a workgroup is a 128-byte run instead of 64 bytes
     // (measured at 256^3: 61 -> 52 us).  FP64 keeps 256 threads: 512 would
     // need 74 KB of LDS per workgroup and leave 2 per CU (87 -> 100 us).
-    // Small grids take one wave per workgroup (line_threads).
-    const bool small = line_threads(c, c->nz, (long)c->ny * c->hx, false) == 64;
+    // Small grids take one wave per workgroup (z_one_wave).
+    const bool small = z_one_wave<R>(c);
     const int nt = small ? 64 : (sizeof(R) == sizeof(float) && c->ny % (512 / (c->nz / 8)) == 0) ? 512 : kBlock;
     const int L = nt / (c->nz / 8);
     const dim3 grid((unsigned)((c->ny + L - 1) / L), (unsigned)c->hx);
