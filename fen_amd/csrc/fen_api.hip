@@ -446,14 +446,12 @@ template <class R> void solve_phi(fen_ctx *c, double dt, void *const *us)
 template <class R> void finish_step(fen_ctx *c, double dt, R *p_old = nullptr)
 {
     using namespace fen;
-    const bool d3 = c->dim == 3;
     launch_project<R>(c, dt, true, p_old);
-    if (const int rest = remaining_groups(c, c->img_vel & c->img_p)) {
+    if (const int rest = remaining_groups(c, c->img_vel & c->img_p)) {   // 3-D
         GhostDesc<R> g[4] = {make_desc<R>(c, FEN_U, c->d_u[0]), make_desc<R>(c, FEN_V, c->d_u[1]),
-                             d3 ? make_desc<R>(c, FEN_W, c->d_u[2]) : make_desc<R>(c, FEN_P, c->d_p),
-                             make_desc<R>(c, FEN_P, c->d_p)};
+                             make_desc<R>(c, FEN_W, c->d_u[2]), make_desc<R>(c, FEN_P, c->d_p)};
         for (auto &d : g) d.groups = rest;
-        launch_ghost_desc<R>(c, g, d3 ? 4 : 3);
+        launch_ghost_desc<R>(c, g, 4);
     }
     c->checks_valid = true;
 }

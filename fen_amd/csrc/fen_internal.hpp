@@ -65,27 +65,9 @@ __host__ __device__ inline int image_axes(const int *type, int dim)
 
 // Writes v to every periodic image of interior cell (i,j,k) along the axes
 // in `ax` (bit 0 x, 1 y, 2 z): the ghost cells whose final value is a copy
-// of this cell (src/scalar.f90:254-388, periodic branches).
-template <class R>
-__device__ __forceinline__ void write_images(R *f, const Box &b, int ax, int i, int j, int k, R v)
-{
-    const int ii = (ax & 1) ? (i == 1 ? b.nx + 1 : (i == b.nx ? 0 : -1)) : -1;
-    const int jj = (ax & 2) ? (j == 1 ? b.ny + 1 : (j == b.ny ? 0 : -1)) : -1;
-    const int kk = (ax & 4) ? (k == 1 ? b.nz + 1 : (k == b.nz ? 0 : -1)) : -1;
-    if (ii < 0 && jj < 0 && kk < 0) return;
-    if (ii >= 0) f[b.g(ii, j, k)] = v;
-    if (jj >= 0) f[b.g(i, jj, k)] = v;
-    if (kk >= 0) f[b.g(i, j, kk)] = v;
-    if (ii >= 0 && jj >= 0) f[b.g(ii, jj, k)] = v;
-    if (ii >= 0 && kk >= 0) f[b.g(ii, j, kk)] = v;
-    if (jj >= 0 && kk >= 0) f[b.g(i, jj, kk)] = v;
-    if (ii >= 0 && jj >= 0 && kk >= 0) f[b.g(ii, jj, kk)] = v;
-}
-
-// write_images() for callers whose j and k are the same across a wave (a
-// k-marching tile row, an x line of the c2r): only the x test varies across
-// lanes; `xedge` says whether the wave can hold i == 1 or i == nx.  Writes
-// exactly the cells write_images() writes.
+// of this cell (src/scalar.f90:254-388, periodic branches).  For callers whose
+// j and k are the same across a wave (a k-marching tile row): only the x test
+// varies across lanes; `xedge` says whether the wave can hold i == 1 or i == nx.
 template <class R>
 __device__ __forceinline__ void march_images(R *f, const Box &b, int ax, int i, int j, int k, R v, bool xedge)
 {

@@ -78,14 +78,9 @@ void to_host(double *dst, const void *src, size_t n, size_t es)
     }
 }
 
-void from_host(void *dst, const double *src, size_t n, size_t es)
+void from_host(float *dst, const double *src, size_t n)   // (FP64 arrays come the plain way)
 {
-    if (es == sizeof(double)) {
-        std::memcpy(dst, src, n * sizeof(double));
-    } else {
-        float *f = static_cast<float *>(dst);
-        for (size_t q = 0; q < n; q++) f[q] = (float)src[q];
-    }
+    for (size_t q = 0; q < n; q++) dst[q] = (float)src[q];
 }
 
 // The stream's device is current while this lives: the copy's events have to
@@ -139,7 +134,7 @@ struct Pipe {
             if (out) {
                 check(hipMemcpyAsync(piece[b], devp + a * es, m * es, hipMemcpyDeviceToHost, stream));
             } else {
-                from_host(piece[b], host + a, m, es);
+                from_host(static_cast<float *>(piece[b]), host + a, m);
                 check(hipMemcpyAsync(devp + a * es, piece[b], m * es, hipMemcpyHostToDevice, stream));
             }
             check(hipEventRecord(ev[b], stream));
@@ -221,7 +216,7 @@ void copy_to_device(hipStream_t stream, void *dst, const double *src, size_t n, 
     }
     if (staged(stream, dst, const_cast<double *>(src), n, es, false)) return;
     std::vector<float> h(n);
-    from_host(h.data(), src, n, es);
+    from_host(h.data(), src, n);
     check(hipMemcpyAsync(dst, h.data(), n * es, hipMemcpyHostToDevice, stream));
     check(hipStreamSynchronize(stream));
 }

@@ -843,8 +843,9 @@ void launch_rfft_y(fen_ctx *c, int inverse, double post)
     prof_end(c, kid, 16.0 * c->n_int);
 }
 
-// Column layout of the pn, nn, npn and nnn sweeps (and of ppn's, whose
-// sweep kernel is thomas_kernel): element type and association form.
+// Column layout of the nn, npn and nnn sweeps (and of ppn's, whose sweep
+// kernel is thomas_kernel): element type and association form.  (pn's columns
+// are never too long for thomas_chunk_kernel.)
 static ThomasGArgs thomas_layout(fen_ctx *c, bool *complex_out, bool *assoc2d_out)
 {
     ThomasGArgs a{};
@@ -857,10 +858,6 @@ static ThomasGArgs thomas_layout(fen_ctx *c, bool *complex_out, bool *assoc2d_ou
     const int hy = c->ny / 2 + 1;
     bool complex_e = false, assoc2d = false;
     switch (c->solver) {
-    case FEN_SOLVER_PN:   // complex [kx][j], columns along j
-        a.x = c->d_spec; complex_e = true; assoc2d = true;
-        a.ncol = c->hx; a.ni = 1; a.os = c->ny; a.s = 1; a.n = c->ny;
-        break;
     case FEN_SOLVER_NN:   // real [kx][j]
         a.x = c->d_spec; assoc2d = true;
         a.ncol = c->nx; a.ni = 1; a.os = c->ny; a.s = 1; a.n = c->ny;
@@ -911,11 +908,9 @@ void launch_thomas_neumann(fen_ctx *c)
     ThomasGArgs a = thomas_layout(c, &complex_e, &assoc2d);
     const dim3 grid((unsigned)((a.ncol + kNB - 1) / kNB));
     prof_begin(c, K_THOMAS);
-    if (complex_e) {
-        // real and imaginary parts on adjacent threads
+    if (complex_e) {   // npn: real and imaginary parts on adjacent threads
         const dim3 g2((unsigned)((2 * a.ncol + kNB - 1) / kNB));
-        if (assoc2d) hipLaunchKernelGGL((thomas_general_kernel<double, 1, 1>), g2, dim3(kNB), 0, c->stream, a);
-        else hipLaunchKernelGGL((thomas_general_kernel<double, 0, 1>), g2, dim3(kNB), 0, c->stream, a);
+        hipLaunchKernelGGL((thomas_general_kernel<double, 0, 1>), g2, dim3(kNB), 0, c->stream, a);
     }
     else if (assoc2d) hipLaunchKernelGGL((thomas_general_kernel<double, 1>), grid, dim3(kNB), 0, c->stream, a);
     else hipLaunchKernelGGL((thomas_general_kernel<double, 0>), grid, dim3(kNB), 0, c->stream, a);

@@ -38,13 +38,10 @@ _PATTERNS = [
     (r"thomas_kernel|thomas_general_kernel|thomas_column_kernel|thomas_chunk_kernel", "thomas"),
     (r"vof_reconstruct_kernel", "vof_reconstruct"),
     (r"vof_sweep_kernel", "vof_sweep"),
-    (r"vof_finish_kernel", "vof_finish"),
     (r"mf_fields_kernel", "mf_fields"),
     (r"mf_momentum_kernel", "mf_momentum"),
     (r"adj_momentum_(march_)?kernel", "adj_momentum"),
     (r"adj_step_kernel", "adj_step"),
-    (r"adj_project_kernel", "adj_project"),
-    (r"adj_rhs_kernel", "adj_rhs"),
     (r"dct2_(rows|pairs)_kernel", "dct2"),
     (r"dct3_rows_kernel", "dct3"),
     (r"rfft_rows_kernel|irfft_rows_kernel", "rfft_y"),
