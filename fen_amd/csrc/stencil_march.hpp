@@ -408,7 +408,8 @@ template <class R, int SHIFT> __global__ __launch_bounds__(256) void project_che
 // value; a pending mean shift of phi is subtracted as the projection does.
 //
 // What bounds it: HBM on large grids (256^3 FP64 2.013 GB in 420 us, 4.8
-// TB/s, 0.84 of what a copy reaches); on small ones the chain of one plane
+// TB/s, what a device copy reaches and 0.84 of a large FP64 add; 430 to 440 us
+// inside a run, the figures here are of launches back to back); on small ones the chain of one plane
 // (load, form, barrier, stencil: 2.4 us alone on a CU).  Both ask for more
 // work per plane and barrier, so a thread owns two rows: the tile's halo is
 // 1.27 instead of 1.52 of its cells, the rows share their neighbours, edge
